@@ -412,6 +412,29 @@ int mlr_silu_mul(const void *gate_up, int64_t gate_up_stride, void *out, int64_t
                  int64_t rows, int64_t intermediate, int dtype, void *stream);
 
 /*
+ * A linear layer over at most 32 rows: out[r, j] = sum_i x[r, i] * weight[j, i]
+ * (+ bias[j]), FP32 accumulation, one rounding to the dtype. With `gated`,
+ * weight is [2 n, k] with the gate's rows first, and out[r, j] is
+ * silu(gate) * up of the two products, each rounded to the dtype first and
+ * combined as mlr_silu_mul does; the gated form takes no bias.
+ *   x      : [rows, k], row stride x_stride (elements); weight [n or 2 n, k]
+ *            contiguous; both 16-byte aligned with 16-byte multiples as rows
+ *   out    : [rows, n], row stride out_stride
+ *   workspace : mlr_rows_linear_workspace_size(...) bytes (0 for most sizes),
+ *            any content; FP32 sums of a long k dealt to several workgroups
+ * dtype bf16, fp16 or FP32.
+ *
+ * Replaces the o_proj of
+ * Qwen2Attention and the projections of Qwen2MLP (model/qwen2.py:
+ * 282-370, 768-792) for a decode step's few rows.
+ */
+int mlr_rows_linear(const void *x, int64_t x_stride, const void *weight, const void *bias,
+                    void *out, int64_t out_stride, int64_t rows, int64_t n, int64_t k,
+                    int gated, int dtype, void *workspace, size_t workspace_bytes,
+                    void *stream);
+size_t mlr_rows_linear_workspace_size(int64_t rows, int64_t n, int64_t k, int gated, int dtype);
+
+/*
  * Diagnostics. No counterpart in the reference: a read-only pass that
  * measures the memory floor of a decode step on its own block list.
  *

@@ -35,6 +35,7 @@
 #include <type_traits>
 
 #include "mlr_common.h"
+#include "silu.h"
 
 // Every product and sum is rounded on its own, as PyTorch's separate kernels
 // round them: no multiply-add contraction in this file.
@@ -191,7 +192,6 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const T *__restrict__ gat
                                                        int64_t gu_stride, T *__restrict__ out,
                                                        int64_t out_stride, int64_t rows,
                                                        int inter) {
-  using E = Elem<T>;
   using C = Chunk<T, N>;
   const int chunks = inter / N;
   const int64_t total = rows * chunks;
@@ -204,11 +204,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const T *__restrict__ gat
     const C a = g[c], b = u[c];
     C o;
 #pragma unroll
-    for (int e = 0; e < N; ++e) {
-      const float gf = E::to_f32(a.v[e]);
-      const T s = E::from_f32(gf / (1.0f + expf(-gf)));
-      o.v[e] = E::from_f32(E::to_f32(s) * E::to_f32(b.v[e]));
-    }
+    for (int e = 0; e < N; ++e) o.v[e] = silu_mul_elem<T>(a.v[e], b.v[e]);
     reinterpret_cast<C *>(out + row * out_stride)[c] = o;
   }
 }

@@ -12,6 +12,8 @@ FP32 on a HIP device; there is no PyTorch fallback.
 from __future__ import annotations
 
 import torch
+import torch.nn as nn
+import torch.nn.functional as F
 
 from .. import _lib
 
@@ -87,3 +89,108 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
                                   _lib.stream_handle(gate_up.device))
     _lib.check(status, "mlr_silu_mul")
     return out
+
+
+# ---------------------------------------------------------------------------
+# Linear layers over a decode step's few rows
+# ---------------------------------------------------------------------------
+_MB = 1 << 20
+# Largest weight, in bytes, that mlr_rows_linear takes by (16-bit, rows above
+# 16, gated): a few rows make the product a read of the weight, and the GEMM
+# library is as good at that once the weight fills its tiles. Measured in
+# graphs on cold weights, us, kernel / library (gated: library GEMM + silu_mul):
+# bf16, 16 rows: 896x4864 7.7 / 17.1, 3584x3584 10.4 / 12.1, 4608x3584
+# 16.5 / 12.3; gated 896x4864 8.4 / 11.3, 1536x8960 16.7 / 42.0, 3584x18944
+# 65 / 61. 32 rows: 896x4864 9.6 / 13.3, 2048x2048 9.7 / 11.3, 3584x3584
+# 15.1 / 11.9; gated 896x4864 11.2 / 14.3, 2048x5632 22.2 / 19.2. FP32, 16
+# rows: 4864x896 10.3 / 15.1, 3584x3584 18.6 / 14.1; gated 896x4864
+# 13.5 / 15.2, 2048x5632 27.5 / 25.0; at 32 rows the library wins.
+_ROWS_LIMIT = {
+    (True, False, False): 28 * _MB, (True, False, True): 64 * _MB,
+    (True, True, False): 16 * _MB, (True, True, True): 20 * _MB,
+    (False, False, False): 28 * _MB, (False, False, True): 40 * _MB,
+    (False, True, False): 0, (False, True, True): 0,
+}
+
+
+def _transformed() -> bool:
+    """Whether something is to see the call as torch operations: tracing,
+    compilation, a dispatch or function mode, a functorch transform, forward
+    differentiation or autocast."""
+    c = torch._C
+    return (torch.is_autocast_enabled() or c._get_tracing_state() is not None
+            or c._len_torch_dispatch_stack() > 0 or c._len_torch_function_stack() > 0
+            or c._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch.compiler.is_compiling())
+
+
+def _rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
+                 gated: bool) -> torch.Tensor | None:
+    """The product by mlr_rows_linear, or None for a call that it does not
+    take (the caller then runs the PyTorch operations)."""
+    dtype = x.dtype
+    if not x.is_cuda or weight.dtype != dtype or dtype not in DTYPES or weight.ndim != 2:
+        return None
+    n, k = weight.shape
+    if x.ndim < 2 or x.shape[-1] != k or k == 0:
+        return None
+    rows, size = x.numel() // k, dtype.itemsize
+    if (rows == 0 or rows > 32
+            or n * k * size > _ROWS_LIMIT[size == 2, rows > 16, gated]):
+        return None
+    if (weight.device != x.device or not weight.is_contiguous() or k * size % 16
+            or x.stride(-1) != 1 or type(x) is not torch.Tensor
+            or type(weight) not in (torch.Tensor, nn.Parameter)):
+        return None
+    if bias is not None and (bias.dtype != dtype or bias.device != x.device
+                             or bias.shape != (n,) or not bias.is_contiguous()
+                             or type(bias) not in (torch.Tensor, nn.Parameter)):
+        return None
+    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad
+                                    or (bias is not None and bias.requires_grad)):
+        return None
+    xr = x.reshape(rows, k)
+    stride = xr.stride(0) if rows > 1 else k
+    if stride < k or stride >= 1 << 22 or stride * size % 16 or xr.stride(1) != 1:
+        return None
+    xp, wp = xr.data_ptr(), weight.data_ptr()
+    if (xp | wp) & 15 or _transformed():
+        return None
+    n_out = n // 2 if gated else n
+    device = x.device
+    out = torch.empty((*x.shape[:-1], n_out), dtype=dtype, device=device)
+    lib = _lib.load()
+    code = _lib.DTYPE_CODES[dtype]
+    nbytes = lib.mlr_rows_linear_workspace_size(rows, n_out, k, gated, code)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
+    with torch.cuda.device(device):
+        status = lib.mlr_rows_linear(
+            xp, stride, wp, bias.data_ptr() if bias is not None else None, out.data_ptr(), n_out,
+            rows, n_out, k, gated, code, ws.data_ptr() if ws is not None else None, nbytes,
+            _lib.stream_handle(device))
+    _lib.check(status, "mlr_rows_linear")
+    return out
+
+
+def linear_silu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor) -> torch.Tensor:
+    """silu(x @ gate.T) * (x @ up.T) for the stacked weight [gate; up]
+    [2 * intermediate, hidden]: one launch for a few rows, else the GEMM and
+    silu_mul."""
+    out = None
+    if gate_up_weight.shape[0] % 2 == 0:
+        out = _rows_linear(x, gate_up_weight, None, True)
+    return silu_mul(F.linear(x, gate_up_weight)) if out is None else out
+
+
+def apply_linear(module: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """module(x) for a projection of the model: a plain nn.Linear without
+    hooks goes through linear(), anything else is called as it is."""
+    if (type(module) is nn.Linear and not module._forward_hooks
+            and not module._forward_pre_hooks and not module._backward_hooks
+            and not module._backward_pre_hooks and "forward" not in module.__dict__
+            and not nn.modules.module._has_any_global_hook()):
+        out = _rows_linear(x, module.weight, module.bias, False)
+        if out is not None:
+            return out
+    return module(x)

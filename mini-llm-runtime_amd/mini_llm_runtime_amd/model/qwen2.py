@@ -148,8 +148,9 @@ class Qwen2MLP(nn.Module):
         if kops.supported(hidden_states):
             # One GEMM for both projections, then one launch for
             # silu(gate) * up (mlr_silu_mul, the same roundings as below).
-            gate_up = F.linear(hidden_states, self._gate_up_weight())
-            return self.down_proj(kops.silu_mul(gate_up))
+            # A decode step's few rows: both in one (mlr_rows_linear).
+            gated = kops.linear_silu_mul(hidden_states, self._gate_up_weight())
+            return kops.apply_linear(self.down_proj, gated)
         return self.down_proj(F.silu(self.gate_proj(hidden_states)) * self.up_proj(hidden_states))
 
 

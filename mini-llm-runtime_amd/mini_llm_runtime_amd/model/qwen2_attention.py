@@ -37,6 +37,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from ..kernels import layer_ops as kops
 from ..kernels import paged_attention as kpa
 from ..kernels import pre_attention as kpre
 from ..runtime.paged_kv_cache import PagedKVCache
@@ -279,7 +280,7 @@ class Qwen2Attention(nn.Module):
         kv_cache.write_slots(slot_mapping=slot_mapping, k=key.squeeze(0),
                              v=value.squeeze(0), layer_idx=layer_idx)
         out = self._attend_fresh(query.squeeze(0), key.squeeze(0), value.squeeze(0))
-        return self.o_proj(out.reshape(1, -1, self.hidden_size))
+        return kops.apply_linear(self.o_proj, out.reshape(1, -1, self.hidden_size))
 
     def _attend_fresh(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         """Causal attention of a whole prompt over its own K/V with the chunk
@@ -328,7 +329,7 @@ class Qwen2Attention(nn.Module):
         out = kpa.paged_attention_decode(q=query[0], k_cache=k_layer, v_cache=v_layer,
                                          block_table=block_table, seq_len=context_len,
                                          block_size=kv_cache.block_size)
-        return self.o_proj(out.reshape(1, 1, self.hidden_size))
+        return kops.apply_linear(self.o_proj, out.reshape(1, 1, self.hidden_size))
 
     # ------------------------------------------------------------------
     # Batched decode (reference :538-622)
@@ -380,12 +381,12 @@ class Qwen2Attention(nn.Module):
             out = kpre.qkv_rope_decode(qkv, self.rotary_embedding.inv_freq, kv_cache,
                                        layer_idx, slot_mapping, block_tables, context_lens,
                                        self.num_attention_heads)
-            return self.o_proj(out.reshape(batch, 1, self.hidden_size))
+            return kops.apply_linear(self.o_proj, out.reshape(batch, 1, self.hidden_size))
         k_layer, v_layer = kv_cache.get_layer_cache(layer_idx)
         query = self._fused_qkv_rope_write(hidden_states[:, 0], position_ids[:, 0], kv_cache,
                                            layer_idx, slot_mapping)
         out = kpa.paged_decode_launch(query, k_layer, v_layer, block_tables, context_lens)
-        return self.o_proj(out.reshape(batch, 1, self.hidden_size))
+        return kops.apply_linear(self.o_proj, out.reshape(batch, 1, self.hidden_size))
 
     @staticmethod
     def _check_decode_metadata(kv_cache, position_ids, slot_mapping, block_tables,
@@ -456,7 +457,7 @@ class Qwen2Attention(nn.Module):
         out = kpa.paged_prefill_launch(query, k_layer, v_layer,
                                        block_tables, query_start_loc, context_lens,
                                        max_query_len)
-        return self.o_proj(out.reshape(-1, self.hidden_size))
+        return kops.apply_linear(self.o_proj, out.reshape(-1, self.hidden_size))
 
     # ------------------------------------------------------------------
     # Chunk prefill (reference :624-767)
@@ -519,4 +520,4 @@ class Qwen2Attention(nn.Module):
             q=query, k_cache=k_layer, v_cache=v_layer, block_table=table,
             prefix_len=prefix_len, context_len=context_len, block_size=bs,
             tile_size=tile_size)
-        return self.o_proj(out.reshape(1, chunk_len, self.hidden_size))
+        return kops.apply_linear(self.o_proj, out.reshape(1, chunk_len, self.hidden_size))
