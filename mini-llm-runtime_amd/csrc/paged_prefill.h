@@ -62,8 +62,8 @@ __device__ __forceinline__ SeqRange seq_range(const PrefillParams &p, int s) {
 }
 
 // True when the matrix-core kernel covers these arguments (bf16 or fp16,
-// head_dim 64 or 128, power-of-two block_size >= 16, aligned rows, positive
-// scale).
+// head_dim a multiple of 8 up to 128, power-of-two block_size >= 16, aligned
+// rows, positive scale).
 bool prefill_mfma_eligible(const PrefillParams &p, int dtype);
 int launch_prefill_mfma(const PrefillParams &p, int dtype, int64_t max_query_len,
                         hipStream_t stream);

@@ -51,6 +51,19 @@
 // not done here), and P is rounded to bf16 as the MFMA operand. fp16 runs the
 // same kernel with fp16 operands (the same two roundings, to fp16: relative
 // 2^-12), round-to-nearest-even throughout.
+//
+// Head sizes other than 64 and 128 (kPad: multiples of 8 up to 128) run in the
+// next larger kernel: copies of the 16-byte chunks past the head fall outside
+// the buffer resource, so the LDS rows are padded with zeros, Q likewise.
+// They ran on the generic kernel, whose queries, scores and probabilities
+// are FP32, so this form keeps them: q is not pre-scaled (the scores are
+// scaled and shifted by one FP32 fma each), and each probability goes to the
+// matrix cores as two 16-bit parts, the rounded value and what was rounded
+// off. That is half as many MFMAs again and 40 registers; the generic kernel
+// was bound by one FP32 multiply-add per lane and three shuffles per key.
+// fp16, 3 sequences of 60..400 queries on prefixes up to 800, 8/2 heads of 96:
+// 1,618 us per call before, 31.7 us now; error against 64 bits 6.7e-4 before,
+// 2.1e-4 now (the generic kernel rounds each score to the 16-bit type).
 #include "paged_prefill.h"
 
 #include <atomic>
@@ -161,8 +174,9 @@ __device__ __forceinline__ int workgroup_rank(int b, int nwg, int ncu, int pair_
   return b < paired ? single + b : b - paired;
 }
 
-template <typename T, int D, int BN, int KS>
-__global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
+template <typename T, int D, int BN, int KS, bool kPad>
+__global__ __launch_bounds__(256 * KS)
+    __attribute__((amdgpu_waves_per_eu(D == 64 && !kPad ? 4 : 2)))
 void prefill_mfma(PrefillParams p) {
   using C = Cfg<D, BN>;
   using M = Mma<T>;
@@ -170,6 +184,7 @@ void prefill_mfma(PrefillParams p) {
   constexpr int QS = D / 16;         // 16-dim k-steps of S^T
   constexpr int NB = D / 32;         // 32-dim blocks of O^T
   constexpr int KB = C::kBlocks;     // 32-key blocks per tile
+  const int d = kPad ? p.d : D;      // head size: with kPad any multiple of 8 up to D
   static_assert(KS == 2, "the ping-pong schedule pairs two splits");
   // Per split: two stages of K and of V, each a separate LDS object, so that
   // reads of one stage need not wait for copies into another. Byte w of
@@ -281,19 +296,25 @@ void prefill_mfma(PrefillParams p) {
   // before issuing the block-id loads and the first copies).
   uint4 qraw[QS];
 #pragma unroll
-  for (int s = 0; s < QS; ++s) qraw[s] = *reinterpret_cast<const uint4 *>(qrow + 16 * s + 8 * hh);
+  for (int s = 0; s < QS; ++s) {
+    const int e = 16 * s + 8 * hh;
+    qraw[s] = *reinterpret_cast<const uint4 *>(qrow + (kPad && e >= d ? 0 : e));
+  }
   v8 qf[QS];
 
   // Copy role: copy i of a span moves chunk positions [64i, 64i + 64) of its 16
   // rows; lane l fills position 64i + l (row rr, physical chunk pc) with
   // logical chunk pc ^ swz(rr) of source row rr.
-  const uint32_t row_bytes = static_cast<uint32_t>(p.hkv) * D * 2;  // slot stride
+  const uint32_t row_bytes = static_cast<uint32_t>(p.hkv) * d * 2;  // slot stride
   uint32_t src_off[C::kCopies];
 #pragma unroll
   for (int i = 0; i < C::kCopies; ++i) {
     const int pos = 64 * i + lane;
     const int rr = pos / C::kChunks, pc = pos % C::kChunks;
-    src_off[i] = rr * row_bytes + ((pc ^ swz<D>(rr)) << 4);
+    const int chunk = pc ^ swz<D>(rr);
+    src_off[i] = rr * row_bytes + (chunk << 4);
+    // Chunks past a padded head lie outside every resource: zeros.
+    if (kPad && 8 * chunk >= d) src_off[i] = 0x7fffffffu;
   }
   // The block table is read-only for the whole launch: read it through the
   // constant address space, so the wave-uniform lookups are scalar loads.
@@ -362,7 +383,7 @@ void prefill_mfma(PrefillParams p) {
 #pragma unroll
       for (int st = 0; st < QS; ++st) {
         const v8 a = *reinterpret_cast<const v8 *>(kst + 32 * j * C::kRowB + koff[st]);
-        s[j] = M::mfma(a, qf[st], st == 0 ? negm : s[j]);
+        s[j] = M::mfma(a, qf[st], st == 0 ? (kPad ? f32x16_t{} : negm) : s[j]);
       }
     }
     // At most two K reads ahead of the MFMAs (four VGPRs each): hoisting all
@@ -438,7 +459,7 @@ void prefill_mfma(PrefillParams p) {
   // Launches with num_blocks < 2^31 and blocks < 2^31 bytes only.
   const uint32_t nb32 = static_cast<uint32_t>(p.num_blocks);
   const uint32_t block_bytes = row_bytes << bs_log2;
-  const uint32_t kv_bytes = static_cast<uint32_t>(kvh) * (2 * D);
+  const uint32_t kv_bytes = static_cast<uint32_t>(kvh) * (2 * d);
 
   // The wave's span of tile t: the byte offset and record count of a buffer
   // resource covering the rows the workgroup needs (rows past them, and a
@@ -460,7 +481,7 @@ void prefill_mfma(PrefillParams p) {
     const bool ok = live && hi == 0u && lo < nb32;
     const uint32_t nrows = static_cast<uint32_t>(min(kv_end - pos0, kSpanRows));
     Span sp;
-    sp.nrec = ok ? (nrows - 1) * row_bytes + 2 * D : 0u;
+    sp.nrec = ok ? (nrows - 1) * row_bytes + 2 * d : 0u;
     const uint64_t byte0 = static_cast<uint64_t>(ok ? lo : 0u) * block_bytes +
                            (static_cast<uint32_t>((t * BN) & bs_mask) * row_bytes + inblk_w);
     sp.off_lo = static_cast<uint32_t>(byte0);
@@ -492,9 +513,12 @@ void prefill_mfma(PrefillParams p) {
     }
     if (bad != nullptr) bad[4 * lane + w] = static_cast<unsigned char>(sp.bad);
   };
+  constexpr int kLowBlocks = kPad ? KB : 1;
   // exp2 of a tile's S^T packed to the 16-bit type (the P@V operand), with the FP32
   // probabilities added to the row sum (four chains).
-  auto probs = [&](const f32x16_t (&sc)[KB], uint32_t (&pk)[KB][8]) __attribute__((always_inline)) {
+  // With kPad the rounded-off part of each probability is packed as well.
+  auto probs = [&](const f32x16_t (&sc)[KB], uint32_t (&pk)[KB][8],
+                   uint32_t (&pl)[kLowBlocks][8]) __attribute__((always_inline)) {
     float lsum[4];
 #pragma unroll
     for (int j = 0; j < KB; ++j)
@@ -503,6 +527,7 @@ void prefill_mfma(PrefillParams p) {
         const float p0 = __builtin_amdgcn_exp2f(sc[j][2 * x]);
         const float p1 = __builtin_amdgcn_exp2f(sc[j][2 * x + 1]);
         pk[j][x] = M::pack2(p0, p1);
+        if constexpr (kPad) pl[j][x] = M::pack2(p0 - M::lo(pk[j][x]), p1 - M::hi(pk[j][x]));
         if (j == 0 && x < 2) {
           lsum[2 * x] = p0;
           lsum[2 * x + 1] = p1;
@@ -514,7 +539,8 @@ void prefill_mfma(PrefillParams p) {
     l_run += (lsum[0] + lsum[1]) + (lsum[2] + lsum[3]);
   };
   // O^T += V^T P^T from packed P.
-  auto pv = [&](const uint32_t (&pk)[KB][8], const unsigned char *vst) __attribute__((always_inline)) {
+  auto pv = [&](const uint32_t (&pk)[KB][8], const uint32_t (&pl)[kLowBlocks][8],
+                const unsigned char *vst) __attribute__((always_inline)) {
     int voff[2][NB];
     voffs(voff);
 #pragma unroll
@@ -534,17 +560,23 @@ void prefill_mfma(PrefillParams p) {
           const uint2 ulo = __builtin_bit_cast(uint2, lo), uhi = __builtin_bit_cast(uint2, hi);
           const v8 a = __builtin_bit_cast(v8, make_uint4(ulo.x, ulo.y, uhi.x, uhi.y));
           acc[n] = M::mfma(a, pb, acc[n]);
+          if constexpr (kPad)
+            acc[n] = M::mfma(a,
+                             __builtin_bit_cast(v8, make_uint4(pl[j][4 * h16], pl[j][4 * h16 + 1],
+                                                               pl[j][4 * h16 + 2],
+                                                               pl[j][4 * h16 + 3])),
+                             acc[n]);
         }
       }
     // Two MFMAs' V^T reads (two each) ahead of the MFMAs.
-    constexpr int kMfma = 2 * KB * NB;
+    constexpr int kMfma = 2 * KB * NB, kEach = kPad ? 2 : 1;
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
     for (int g = 0; g < kMfma - 2; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, kEach, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 2 * kEach, 0);
   };
 
   // Main loop: a ping-pong schedule of the two key-range splits (waves w and
@@ -588,19 +620,20 @@ void prefill_mfma(PrefillParams p) {
   const float c2 = static_cast<float>(p.scale) * kLog2e;
 #pragma unroll
   for (int s = 0; s < QS; ++s) {
-    const uint4 raw = q_ok ? qraw[s] : make_uint4(0, 0, 0, 0);
+    const bool in = q_ok && (!kPad || 16 * s + 8 * hh < d);
+    const uint4 raw = in ? qraw[s] : make_uint4(0, 0, 0, 0);
     const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
     uint32_t o4[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      o4[e] = M::pack2(M::lo(w4[e]) * c2, M::hi(w4[e]) * c2);
+      o4[e] = kPad ? w4[e] : M::pack2(M::lo(w4[e]) * c2, M::hi(w4[e]) * c2);
     qf[s] = __builtin_bit_cast(v8, make_uint4(o4[0], o4[1], o4[2], o4[3]));
   }
   if (split == 1) __builtin_amdgcn_s_barrier();
   // S^T (M to V) and packed P (V to M) are defined in every phase, idle
   // ones included, so neither is live across the phase that does not use it.
   f32x16_t s[KB];
-  uint32_t pk[KB][8];
+  uint32_t pk[KB][8], pl[kLowBlocks][8];
   uint32_t badw = 0;
   // M_i: K stage kst holds K(i) and its out-of-range flags kbad (read here:
   // V_i overwrites them), V stage vst holds V(i-1).
@@ -610,7 +643,7 @@ void prefill_mfma(PrefillParams p) {
     // Raised wave priority for the matrix work: the other split's softmax
     // phase on this SIMD takes the issue slots the MFMAs leave.
     __builtin_amdgcn_s_setprio(3);
-    if (i >= 1 && i - 1 < nw) pv(pk, vst);
+    if (i >= 1 && i - 1 < nw) pv(pk, pl, vst);
     // P dies with the last P@V MFMA before S^T is allocated.
     __builtin_amdgcn_sched_barrier(0);
     if (i < nw) {
@@ -635,14 +668,21 @@ void prefill_mfma(PrefillParams p) {
     issue_span(dv, p.vc, vdst, nullptr);
     if (i < nw) {
       const int t = t_lo + i;
+      if constexpr (kPad) {  // unscaled q: base-2 scores relative to m here
+#pragma unroll
+        for (int j = 0; j < KB; ++j) s[j] = s[j] * c2 + negm;
+      }
       if (t >= wave_nfull || badw != 0) mask(t, badw, s);
       rescale(tile_max(s), s);
-      probs(s, pk);
+      probs(s, pk, pl);
     } else {
 #pragma unroll
       for (int j = 0; j < KB; ++j)
 #pragma unroll
-        for (int x = 0; x < 8; ++x) pk[j][x] = 0;
+        for (int x = 0; x < 8; ++x) {
+          pk[j][x] = 0;
+          if constexpr (kPad) pl[j][x] = 0;
+        }
     }
     __builtin_amdgcn_s_waitcnt(kWaitBatch);
     __builtin_amdgcn_s_barrier();
@@ -717,6 +757,7 @@ void prefill_mfma(PrefillParams p) {
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) {
         // acc[n][4g4 + e] = O[query][32n + 8g4 + 4hh + e].
+        if (kPad && 32 * n + 8 * g4 >= d) continue;
         const f32x16_t &a = acc[n];
         const uint2 v = make_uint2(
             M::bits(a[4 * g4] * inv) | (M::bits(a[4 * g4 + 1] * inv) << 16),
@@ -726,7 +767,7 @@ void prefill_mfma(PrefillParams p) {
   }
 }
 
-template <typename T, int D, int BN, int KS>
+template <typename T, int D, int BN, int KS, bool kPad>
 int launch(const PrefillParams &p, int64_t max_query_len, hipStream_t stream) {
   PrefillParams q = p;
   q.n_qtiles = static_cast<int>(ceil_div(max_query_len, kBM));
@@ -744,7 +785,7 @@ int launch(const PrefillParams &p, int64_t max_query_len, hipStream_t stream) {
     int ncu = 0, per_cu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void *>(prefill_mfma<T, D, BN, KS>), 256 * KS, 0) !=
+            &per_cu, reinterpret_cast<const void *>(prefill_mfma<T, D, BN, KS, kPad>), 256 * KS, 0) !=
             hipSuccess)
       return set_error(MLR_ERR_HIP, "mlr_paged_prefill: device query failed");
     per_cu_of[dev].store(per_cu, std::memory_order_relaxed);
@@ -752,7 +793,7 @@ int launch(const PrefillParams &p, int64_t max_query_len, hipStream_t stream) {
   }
   q.ncu = ncu_of[dev].load(std::memory_order_acquire);
   q.pair_cu = per_cu_of[dev].load(std::memory_order_relaxed) == 2 ? 1 : 0;
-  prefill_mfma<T, D, BN, KS><<<dim3(static_cast<unsigned>(blocks)), 256 * KS, 0, stream>>>(q);
+  prefill_mfma<T, D, BN, KS, kPad><<<dim3(static_cast<unsigned>(blocks)), 256 * KS, 0, stream>>>(q);
   return check_launch("mlr_paged_prefill(mfma)");
 }
 
@@ -768,22 +809,28 @@ bool prefill_mfma_eligible(const PrefillParams &p, int dtype) {
   // Positions, block ids and in-block byte offsets are 32-bit inside the
   // kernel; a 16-row span must fit a block.
   constexpr int64_t k2g = int64_t(1) << 31;
-  return (dtype == MLR_DTYPE_BF16 || dtype == MLR_DTYPE_F16) && (p.d == 64 || p.d == 128) &&
+  return (dtype == MLR_DTYPE_BF16 || dtype == MLR_DTYPE_F16) && p.d % 8 == 0 && p.d <= 128 &&
          aligned &&
          p.bs_log2 >= 4 && p.max_blocks * p.block_size < k2g && p.num_blocks < k2g &&
          p.block_size * p.hkv * p.d * 2 < k2g && p.scale > 0.0 && p.scale < 1e30;
+}
+
+template <typename T>
+int launch_dims(const PrefillParams &p, int64_t max_query_len, hipStream_t stream) {
+  if (p.d == 64) return launch<T, 64, 64, 2, false>(p, max_query_len, stream);
+  if (p.d == 128) return launch<T, 128, 64, 2, false>(p, max_query_len, stream);
+  // Other head sizes that are whole 16-byte chunks, up to 128: the next larger
+  // kernel, its LDS rows and Q padded with zeros.
+  if (p.d < 64) return launch<T, 64, 64, 2, true>(p, max_query_len, stream);
+  return launch<T, 128, 64, 2, true>(p, max_query_len, stream);
 }
 
 int launch_prefill_mfma(const PrefillParams &p, int dtype, int64_t max_query_len,
                         hipStream_t stream) {
   // The reference's tile_size only orders the FP32 accumulation; the kernel's
   // key tile is fixed per head_dim by its LDS budget.
-  if (dtype == MLR_DTYPE_F16) {
-    if (p.d == 64) return launch<f16_t, 64, 64, 2>(p, max_query_len, stream);
-    return launch<f16_t, 128, 64, 2>(p, max_query_len, stream);
-  }
-  if (p.d == 64) return launch<bf16_t, 64, 64, 2>(p, max_query_len, stream);
-  return launch<bf16_t, 128, 64, 2>(p, max_query_len, stream);
+  if (dtype == MLR_DTYPE_F16) return launch_dims<f16_t>(p, max_query_len, stream);
+  return launch_dims<bf16_t>(p, max_query_len, stream);
 }
 
 }  // namespace mlr

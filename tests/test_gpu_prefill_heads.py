@@ -1,0 +1,72 @@
+"""Packed prefill at head sizes other than 64 and 128 against attention in 64
+bits.
+
+Bound per output: q.k of 16-bit inputs in FP32 is off by at most
+(d + 2) * 2^-24 * sum |q||k| (under 2^-15 after the scale, for these inputs),
+which moves a probability by that much relative; exp2 and the sums add a few
+2^-22, and the probability operand of the matrix cores carries at least 16
+bits (two 8-bit bf16 parts): 2^-16. The weighted mean of V is then off by
+under 2^-13 max |V|, and the result is rounded once (2^-8 bf16, 2^-11 fp16).
+"""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from mini_llm_runtime_amd.kernels import paged_attention as kpa
+
+pytestmark = pytest.mark.gpu
+
+HALF_ULP = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+def _attend(q, k, v, prefix):
+    group = q.shape[1] // k.shape[1]
+    k, v = (t.repeat_interleave(group, dim=1).transpose(0, 1) for t in (k, v))
+    scores = torch.matmul(q.transpose(0, 1), k.transpose(1, 2).contiguous()) / math.sqrt(q.shape[2])
+    seen = torch.arange(k.shape[1])[None, :] <= prefix + torch.arange(q.shape[0])[:, None]
+    probs = torch.softmax(scores.masked_fill(~seen, float("-inf")), dim=-1)
+    return torch.matmul(probs, v.contiguous()).transpose(0, 1)
+
+
+@pytest.mark.parametrize("dtype", list(HALF_ULP), ids=lambda t: str(t)[6:])
+@pytest.mark.parametrize("d,hq,hkv,bs", [(8, 4, 2, 16), (16, 4, 2, 16), (24, 6, 6, 32),
+                                         (40, 5, 1, 16), (56, 4, 2, 64), (72, 4, 4, 16),
+                                         (80, 10, 2, 16), (96, 8, 2, 16), (120, 3, 1, 32)])
+def test_other_head_sizes_match_float64(device, dtype, d, hq, hkv, bs):
+    gen = torch.Generator().manual_seed(d)
+    seqs = [(0, 1), (130, 33), (0, 129), (700, 200), (15, 64)]  # (prefix, queries)
+    need = [-(-(p + n) // bs) for p, n in seqs]
+    perm = torch.randperm(sum(need) + 3, generator=gen).tolist()
+    # Rows past each context hold NaN: nothing may read them into a product.
+    kc = torch.full((sum(need) + 3, bs, hkv, d), float("nan"), dtype=dtype)
+    vc = kc.clone()
+    tables, want, qs, at = [], [], [], 0
+    for (p, n), nb in zip(seqs, need):
+        table = perm[at:at + nb]
+        at += nb
+        tables.append(table + [-1] * (max(need) - nb))
+        k, v = (torch.randn(p + n, hkv, d, generator=gen).to(dtype) for _ in range(2))
+        pos = torch.arange(p + n)
+        blocks = torch.tensor(table)[pos // bs]
+        kc[blocks, pos % bs], vc[blocks, pos % bs] = k, v
+        q = torch.randn(n, hq, d, generator=gen).to(dtype)
+        qs.append(q)
+        want.append(_attend(q.double(), k.double(), v.double(), p))
+    want = torch.cat(want)
+    lens = [n for _, n in seqs]
+    # q as rows of a wider buffer, as a view of a fused projection would be.
+    wide = torch.full((sum(lens), hq, d + 8), 7.0, dtype=dtype)
+    wide[..., :d] = torch.cat(qs)
+    args = (kc.to(device), vc.to(device), torch.tensor(tables).to(device),
+            torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)]).to(device),
+            torch.tensor([p + n for p, n in seqs]).to(device), bs)
+    got = kpa.paged_attention_prefill_varlen(wide.to(device)[..., :d], *args).double().cpu()
+    vmax = float(torch.nan_to_num(vc.float()).abs().max())
+    bound = HALF_ULP[dtype] * 1.01 * want.abs() + 2.0 ** -13 * vmax
+    assert bool(((got - want).abs() <= bound).all()), ((got - want).abs() - bound).max()
+    assert torch.equal(
+        kpa.paged_attention_prefill_varlen(torch.cat(qs).to(device), *args).double().cpu(), got)
