@@ -315,6 +315,39 @@ int mlr_paged_prefill_chunk(const void *q, int64_t q_stride_t,
                             int64_t out_stride_h, void *stream);
 
 /*
+ * The two prefill calls with a workspace. Where a call's work items (128-query
+ * tiles x query heads) leave most of the GPU idle, a long key range is split
+ * over several workgroups, whose FP32 partial results go through the
+ * workspace, and a second kernel merges them; results differ from the calls
+ * above by the order of FP32 sums. workspace: 16-byte aligned, any content,
+ * at least mlr_paged_prefill_workspace_size bytes for the split to be taken
+ * (0: no split for these sizes); with less the call runs as the one above.
+ * max_context: max_blocks_per_seq * block_size, or context_len.
+ */
+size_t mlr_paged_prefill_workspace_size(int64_t num_seqs, int64_t max_query_len,
+                                        int64_t max_context, int64_t num_q_heads,
+                                        int64_t head_dim, int dtype);
+int mlr_paged_prefill_split(const void *q, int64_t q_stride_t, int64_t q_stride_h,
+                            const void *k_cache, const void *v_cache, int64_t num_blocks,
+                            int64_t block_size, int64_t num_kv_heads, int64_t head_dim,
+                            const int64_t *block_tables, int64_t block_table_stride,
+                            int64_t max_blocks_per_seq, const int64_t *query_start_loc,
+                            const int64_t *context_lens, int64_t num_seqs,
+                            int64_t max_query_len, int64_t num_q_heads, double scale,
+                            int dtype, int64_t kv_tile, void *out, int64_t out_stride_t,
+                            int64_t out_stride_h, void *workspace, size_t workspace_bytes,
+                            void *stream);
+int mlr_paged_prefill_chunk_split(const void *q, int64_t q_stride_t, int64_t q_stride_h,
+                                  const void *k_cache, const void *v_cache, int64_t num_blocks,
+                                  int64_t block_size, int64_t num_kv_heads, int64_t head_dim,
+                                  const int64_t *block_table, int64_t block_table_len,
+                                  int64_t prefix_len, int64_t context_len,
+                                  int64_t num_q_heads, double scale, int dtype,
+                                  int64_t kv_tile, void *out, int64_t out_stride_t,
+                                  int64_t out_stride_h, void *workspace,
+                                  size_t workspace_bytes, void *stream);
+
+/*
  * Fused pre-attention step of one layer: optional projection bias, rotary
  * embedding of the q and k heads, and the KV-cache write, in one launch.
  *

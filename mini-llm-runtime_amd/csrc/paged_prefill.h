@@ -32,6 +32,10 @@ struct PrefillParams {
   int pair_cu;  // 1: the launch fits two workgroups per CU (matrix-core kernel)
   void *out;
   int64_t o_st, o_sh;
+  int max_splits;   // key-range splits of a work item, at most (matrix-core kernel)
+  int split_tiles;  // key tiles per split
+  void *ws;         // partial results of split items
+  size_t ws_bytes;
 };
 
 // Sequence metadata as the kernels see it (clamped to the block-table span).
@@ -65,6 +69,10 @@ __device__ __forceinline__ SeqRange seq_range(const PrefillParams &p, int s) {
 // head_dim a multiple of 8 up to 128, power-of-two block_size >= 16, aligned
 // rows, positive scale).
 bool prefill_mfma_eligible(const PrefillParams &p, int dtype);
+// Bytes of workspace with which launch_prefill_mfma would split the key ranges
+// of this call (0: it would not).
+size_t prefill_mfma_workspace(int64_t num_seqs, int64_t max_query_len, int64_t max_context,
+                              int64_t num_q_heads, int64_t head_dim, int dtype);
 int launch_prefill_mfma(const PrefillParams &p, int dtype, int64_t max_query_len,
                         hipStream_t stream);
 

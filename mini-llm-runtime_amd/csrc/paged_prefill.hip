@@ -194,7 +194,14 @@ int check_common(const void *q, const void *k_cache, const void *v_cache,
 
 using namespace mlr;
 
-extern "C" int mlr_paged_prefill(
+extern "C" size_t mlr_paged_prefill_workspace_size(int64_t num_seqs, int64_t max_query_len,
+                                                   int64_t max_context, int64_t num_q_heads,
+                                                   int64_t head_dim, int dtype) {
+  return prefill_mfma_workspace(num_seqs, max_query_len, max_context, num_q_heads, head_dim,
+                                dtype);
+}
+
+extern "C" int mlr_paged_prefill_split(
     const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *k_cache,
     const void *v_cache, int64_t num_blocks, int64_t block_size,
     int64_t num_kv_heads, int64_t head_dim, const int64_t *block_tables,
@@ -202,7 +209,7 @@ extern "C" int mlr_paged_prefill(
     const int64_t *query_start_loc, const int64_t *context_lens,
     int64_t num_seqs, int64_t max_query_len, int64_t num_q_heads, double scale,
     int dtype, int64_t kv_tile, void *out, int64_t out_stride_t,
-    int64_t out_stride_h, void *stream) {
+    int64_t out_stride_h, void *workspace, size_t workspace_bytes, void *stream) {
   clear_error();
   int rc = check_common(q, k_cache, v_cache, num_blocks, block_size,
                         num_kv_heads, head_dim, num_q_heads, dtype, out);
@@ -237,16 +244,33 @@ extern "C" int mlr_paged_prefill(
   p.out = out;
   p.o_st = out_stride_t;
   p.o_sh = out_stride_h;
+  p.ws = workspace;
+  p.ws_bytes = workspace_bytes;
   return run_prefill(p, dtype, max_query_len, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int mlr_paged_prefill_chunk(
+extern "C" int mlr_paged_prefill(
+    const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *k_cache,
+    const void *v_cache, int64_t num_blocks, int64_t block_size,
+    int64_t num_kv_heads, int64_t head_dim, const int64_t *block_tables,
+    int64_t block_table_stride, int64_t max_blocks_per_seq,
+    const int64_t *query_start_loc, const int64_t *context_lens,
+    int64_t num_seqs, int64_t max_query_len, int64_t num_q_heads, double scale,
+    int dtype, int64_t kv_tile, void *out, int64_t out_stride_t,
+    int64_t out_stride_h, void *stream) {
+  return mlr_paged_prefill_split(q, q_stride_t, q_stride_h, k_cache, v_cache, num_blocks,
+      block_size, num_kv_heads, head_dim, block_tables, block_table_stride, max_blocks_per_seq,
+      query_start_loc, context_lens, num_seqs, max_query_len, num_q_heads, scale, dtype, kv_tile,
+      out, out_stride_t, out_stride_h, nullptr, 0, stream);
+}
+
+extern "C" int mlr_paged_prefill_chunk_split(
     const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *k_cache,
     const void *v_cache, int64_t num_blocks, int64_t block_size,
     int64_t num_kv_heads, int64_t head_dim, const int64_t *block_table,
     int64_t block_table_len, int64_t prefix_len, int64_t context_len,
     int64_t num_q_heads, double scale, int dtype, int64_t kv_tile, void *out,
-    int64_t out_stride_t, int64_t out_stride_h, void *stream) {
+    int64_t out_stride_t, int64_t out_stride_h, void *workspace, size_t workspace_bytes, void *stream) {
   clear_error();
   int rc = check_common(q, k_cache, v_cache, num_blocks, block_size,
                         num_kv_heads, head_dim, num_q_heads, dtype, out);
@@ -283,5 +307,19 @@ extern "C" int mlr_paged_prefill_chunk(
   p.out = out;
   p.o_st = out_stride_t;
   p.o_sh = out_stride_h;
+  p.ws = workspace;
+  p.ws_bytes = workspace_bytes;
   return run_prefill(p, dtype, p.s_qlen, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int mlr_paged_prefill_chunk(
+    const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *k_cache,
+    const void *v_cache, int64_t num_blocks, int64_t block_size,
+    int64_t num_kv_heads, int64_t head_dim, const int64_t *block_table,
+    int64_t block_table_len, int64_t prefix_len, int64_t context_len,
+    int64_t num_q_heads, double scale, int dtype, int64_t kv_tile, void *out,
+    int64_t out_stride_t, int64_t out_stride_h, void *stream) {
+  return mlr_paged_prefill_chunk_split(q, q_stride_t, q_stride_h, k_cache, v_cache, num_blocks,
+      block_size, num_kv_heads, head_dim, block_table, block_table_len, prefix_len, context_len,
+      num_q_heads, scale, dtype, kv_tile, out, out_stride_t, out_stride_h, nullptr, 0, stream);
 }

@@ -52,6 +52,13 @@
 // same kernel with fp16 operands (the same two roundings, to fp16: relative
 // 2^-12), round-to-nearest-even throughout.
 //
+// A call whose work items leave CUs idle (one sequence's chunk over a long
+// context, few heads) cuts the key range of each item over several workgroups
+// (kSplit; the rule is at key_splits): each stores its FP32 (O^T, m, l) to
+// the caller's workspace and prefill_merge adds them. A 500-query bf16 chunk
+// after 16,000 keys, 28/4 heads of 128 (112 workgroups for 256 CUs): 213 us
+// in one part, 142 us in two (825 TFLOP/s).
+//
 // Head sizes other than 64 and 128 (kPad: multiples of 8 up to 128) run in the
 // next larger kernel: copies of the 16-byte chunks past the head fall outside
 // the buffer resource, so the LDS rows are padded with zeros, Q likewise.
@@ -66,6 +73,7 @@
 // 2.1e-4 now (the generic kernel rounds each score to the 16-bit type).
 #include "paged_prefill.h"
 
+#include <algorithm>
 #include <atomic>
 
 namespace mlr {
@@ -174,7 +182,49 @@ __device__ __forceinline__ int workgroup_rank(int b, int nwg, int ncu, int pair_
   return b < paired ? single + b : b - paired;
 }
 
-template <typename T, int D, int BN, int KS, bool kPad>
+// The key tiles [lo, hi) of split s of an item with `tiles` of them, and the
+// item's split count: as many as hold split_tiles each, evenly cut. Splits
+// past the count are empty.
+struct SplitRange {
+  int lo, hi, count;
+};
+__device__ __forceinline__ SplitRange split_range(const PrefillParams &p, int tiles, int s) {
+  const int count = max(1, min(p.max_splits, (tiles + p.split_tiles - 1) / p.split_tiles));
+  const int per = (tiles + count - 1) / count;
+  return SplitRange{min(tiles, s * per), s < count ? min(tiles, (s + 1) * per) : min(tiles, s * per),
+                    count};
+}
+
+// Partial results of one split of (item, head): per wave of 32 queries, `words`
+// rows of 64 lanes (O^T, m, l as the wave holds them).
+__device__ __forceinline__ float *partial_of(const PrefillParams &p, int item, int s, int h, int w,
+                                             int words) {
+  const int64_t row = (static_cast<int64_t>(item) * p.max_splits + s) * p.hq + h;
+  return static_cast<float *>(p.ws) + (row * 4 + w) * words * 64;
+}
+
+// One query's output from O^T in the layout of the 32x32 MFMA.
+template <typename T, int NB, bool kPad>
+__device__ __forceinline__ void store_row(const PrefillParams &p, const f32x16_t (&acc)[NB],
+                                          float inv, int64_t row, int h, int hh) {
+  using M = Mma<T>;
+  uint16_t *orow =
+      static_cast<uint16_t *>(p.out) + row * p.o_st + static_cast<int64_t>(h) * p.o_sh;
+#pragma unroll
+  for (int n = 0; n < NB; ++n)
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      // acc[n][4g4 + e] = O[query][32n + 8g4 + 4hh + e].
+      if (kPad && 32 * n + 8 * g4 >= p.d) continue;
+      const f32x16_t &a = acc[n];
+      const uint2 v = make_uint2(
+          M::bits(a[4 * g4] * inv) | (M::bits(a[4 * g4 + 1] * inv) << 16),
+          M::bits(a[4 * g4 + 2] * inv) | (M::bits(a[4 * g4 + 3] * inv) << 16));
+      *reinterpret_cast<uint2 *>(orow + 32 * n + 8 * g4 + 4 * hh) = v;
+    }
+}
+
+template <typename T, int D, int BN, int KS, bool kPad, bool kSplit>
 __global__ __launch_bounds__(256 * KS)
     __attribute__((amdgpu_waves_per_eu(D == 64 && !kPad ? 4 : 2)))
 void prefill_mfma(PrefillParams p) {
@@ -209,7 +259,8 @@ void prefill_mfma(PrefillParams p) {
   // rank, and CUs left with one workgroup get the heaviest; later workgroups
   // follow in rank order (list scheduling).
   const int nqt = p.n_qtiles;
-  const int nitems = p.num_seqs * nqt;
+  const int ns = kSplit ? p.max_splits : 1;  // virtual items per item
+  const int nitems = p.num_seqs * nqt * ns;
   const int wr = workgroup_rank(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x),
                                 p.ncu, p.pair_cu);
   // Heads of one item on one XCD. The dispatcher deals workgroups to the 8
@@ -235,10 +286,17 @@ void prefill_mfma(PrefillParams p) {
   if (nitems <= kRankMax) {
     __shared__ int item_len[kRankMax];
     __shared__ int ranked_item;
-    auto keys_of = [&](int i) __attribute__((always_inline)) -> int {
+    auto keys_of = [&](int v) __attribute__((always_inline)) -> int {
+      const int i = v / ns;
       const SeqRange r = seq_range(p, i / nqt);
       const int64_t lo = static_cast<int64_t>(i % nqt) * kBM;
-      return lo < r.qlen ? static_cast<int>(r.prefix + min<int64_t>(r.qlen, lo + kBM)) : 0;
+      const int keys =
+          lo < r.qlen ? static_cast<int>(r.prefix + min<int64_t>(r.qlen, lo + kBM)) : 0;
+      if constexpr (kSplit) {  // tiles of this split
+        const SplitRange sr = split_range(p, (keys + BN - 1) / BN, v % ns);
+        return sr.hi - sr.lo;
+      }
+      return keys;
     };
     for (int i = threadIdx.x; i < nitems; i += blockDim.x) item_len[i] = keys_of(i);
     __syncthreads();
@@ -256,6 +314,8 @@ void prefill_mfma(PrefillParams p) {
   } else {
     item = (rank / nqt) * nqt + (nqt - 1 - rank % nqt);
   }
+  const int vsplit = item % ns;  // which of the item's key-range splits
+  item /= ns;
   const int seq = item / nqt, qt = item % nqt;
   SeqRange rg = seq_range(p, seq);
   // Workgroup-uniform: kept in scalar registers.
@@ -275,9 +335,11 @@ void prefill_mfma(PrefillParams p) {
   // Keys the workgroup needs: up to its last query position; split k takes
   // tiles [t_lo, t_hi).
   const int kv_end = prefix + min(qlen, q0 + kBM);
-  const int ntiles = (kv_end + BN - 1) / BN;
-  const int chunk = (ntiles + KS - 1) / KS;
-  const int t_lo = split * chunk, t_hi = min(ntiles, t_lo + chunk);
+  SplitRange tiles{0, (kv_end + BN - 1) / BN, 1};
+  if constexpr (kSplit) tiles = split_range(p, tiles.hi, vsplit);
+  if (kSplit && tiles.lo >= tiles.hi) return;  // uniform
+  const int chunk = (tiles.hi - tiles.lo + KS - 1) / KS;
+  const int t_lo = tiles.lo + split * chunk, t_hi = min(tiles.hi, t_lo + chunk);
   // This wave's queries [wq, wq_end); tiles it reads; tiles it sees whole.
   const int wq = q0 + 32 * w;
   const int wq_end = min(qlen, wq + 32);
@@ -742,6 +804,18 @@ void prefill_mfma(PrefillParams p) {
     }
   }
 
+  if constexpr (kSplit) {
+    if (tiles.count > 1) {  // uniform: prefill_merge adds the splits
+      float *part = partial_of(p, item, vsplit, h, w, 16 * NB + 2) + lane;
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) part[(16 * n + i) * 64] = acc[n][i];
+      part[16 * NB * 64] = m_run;
+      part[(16 * NB + 1) * 64] = l_run;
+      return;
+    }
+  }
   const float l_tot = pair_sum(l_run);
   // The lane's query and half are recomputed from the lane id here rather
   // than kept in registers across the main loop (which spilled them).
@@ -749,52 +823,126 @@ void prefill_mfma(PrefillParams p) {
   asm volatile("" : "+v"(lane_e));
   const int qi_e = wq + (lane_e & 31), hh_e = lane_e >> 5;
   if (qi_e < qlen) {
-    const float inv = 1.f / l_tot;
-    uint16_t *orow = static_cast<uint16_t *>(p.out) + (rg.q0 + qi_e) * p.o_st +
-                     static_cast<int64_t>(h) * p.o_sh;
+    store_row<T, NB, kPad>(p, acc, 1.f / l_tot, rg.q0 + qi_e, h, hh_e);
+  }
+}
+
+// The splits of each split item, merged: one workgroup per (item, query head),
+// its four waves laid out as the producers'. Bound by reading the partials
+// (FP32, coalesced, mostly still in the caches).
+template <typename T, int D, int BN, bool kPad>
+__global__ __launch_bounds__(256) void prefill_merge(PrefillParams p) {
+  constexpr int NB = D / 32, A = 16 * NB + 2;
+  const int item = blockIdx.x / p.hq, h = blockIdx.x % p.hq;
+  const int seq = item / p.n_qtiles, q0 = (item % p.n_qtiles) * kBM;
+  const SeqRange rg = seq_range(p, seq);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int qi = q0 + 32 * w + (lane & 31);
+  if (q0 + 32 * w >= rg.qlen) return;  // whole waves
+  const int kv_end = static_cast<int>(rg.prefix + min<int64_t>(rg.qlen, q0 + kBM));
+  const int count = split_range(p, (kv_end + BN - 1) / BN, 0).count;
+  if (count <= 1) return;  // its one workgroup stored the output
+  float m = kFloor;
+  for (int s = 0; s < count; ++s)
+    m = fmaxf(m, partial_of(p, item, s, h, w, A)[16 * NB * 64 + lane]);
+  f32x16_t acc[NB];
+#pragma unroll
+  for (int n = 0; n < NB; ++n) acc[n] = f32x16_t{};
+  float l = 0.f;
+  for (int s = 0; s < count; ++s) {
+    const float *part = partial_of(p, item, s, h, w, A) + lane;
+    const float f = __builtin_amdgcn_exp2f(part[16 * NB * 64] - m);
+    l += f * part[(16 * NB + 1) * 64];
 #pragma unroll
     for (int n = 0; n < NB; ++n)
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        // acc[n][4g4 + e] = O[query][32n + 8g4 + 4hh + e].
-        if (kPad && 32 * n + 8 * g4 >= d) continue;
-        const f32x16_t &a = acc[n];
-        const uint2 v = make_uint2(
-            M::bits(a[4 * g4] * inv) | (M::bits(a[4 * g4 + 1] * inv) << 16),
-            M::bits(a[4 * g4 + 2] * inv) | (M::bits(a[4 * g4 + 3] * inv) << 16));
-        *reinterpret_cast<uint2 *>(orow + 32 * n + 8 * g4 + 4 * hh_e) = v;
-      }
+      for (int i = 0; i < 16; ++i) acc[n][i] += f * part[(16 * n + i) * 64];
   }
+  const float l_tot = pair_sum(l);
+  if (qi < rg.qlen) store_row<T, NB, kPad>(p, acc, 1.f / l_tot, rg.q0 + qi, h, lane >> 5);
+}
+
+constexpr int kKeyTile = 64;      // BN of every instantiation
+constexpr int kMaxKeySplits = 8;  // most splits of an item's key range
+constexpr int kMinSplitTiles = 8; // fewest key tiles worth a workgroup
+
+// How a launch of `items` work items x `hq` heads splits key ranges of up to
+// max_tiles tiles: into as many parts as give the GPU one workgroup per CU,
+// each of at least kMinSplitTiles tiles, and only where the longest item
+// becomes shorter by enough tiles (about 0.53 us each at head size 64, 0.8 us
+// at 128) to pay for writing, reading and merging the partials (6-8 us).
+// Measured, bf16, graphs, us per call split / unsplit: 14/2 heads of 64, a
+// chunk of 16 after 2000 keys 18.8 / 23.2, of 64 after 4000 24.0 / 39.0, of 512
+// after 16000 60 / 142 (with two workgroups per CU; one is better still), but
+// 16 tiles in two 17.3 / 17.2 and a 1024-token prompt in two 20.6 / 17.6.
+// 28/4 heads of 128: a chunk of 16 after 2000 27.2 / 36.8, of 512 after 4000
+// 57 / 69, after 16000 142 / 213; of 512 after 1000 36.3 / 33.6.
+struct KeySplits {
+  int max_splits, split_tiles;  // max_splits 1: no split
+};
+KeySplits key_splits(int64_t items, int64_t hq, int64_t max_tiles, int64_t head_dim) {
+  const int64_t want =
+      std::min<int64_t>(kMaxKeySplits, current_device_cus() / (items * hq));
+  if (want < 2 || items * want > kRankMax) return {1, 1};
+  const int64_t per = std::max<int64_t>(kMinSplitTiles, ceil_div(max_tiles, want));
+  if (max_tiles - per < (head_dim == 64 ? 20 : 16)) return {1, 1};
+  return {static_cast<int>(ceil_div(max_tiles, per)), static_cast<int>(per)};
+}
+
+size_t split_bytes(int64_t items, int64_t hq, int d, int splits) {
+  const int64_t words = 16 * (d / 32) + 2;
+  return static_cast<size_t>(items) * splits * hq * 4 * words * 64 * sizeof(float);
+}
+
+template <typename T, int D, int BN, int KS, bool kPad, bool kSplit>
+int launch_kernel(PrefillParams &q, hipStream_t stream) {
+  const int64_t items = static_cast<int64_t>(q.num_seqs) * q.n_qtiles;
+  const int64_t blocks = items * q.max_splits * q.hq;
+  if (blocks > INT32_MAX)
+    return set_error(MLR_ERR_UNSUPPORTED, "mlr_paged_prefill: too many work items");
+  // Workgroups per CU of this kernel, queried once per device (threads that
+  // race here store the same values).
+  constexpr int kMaxDevices = 64;
+  static std::atomic<int> per_cu_of[kMaxDevices];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
+    return set_error(MLR_ERR_HIP, "mlr_paged_prefill: no current device");
+  int per_cu = per_cu_of[dev].load(std::memory_order_acquire);
+  if (per_cu == 0) {
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &per_cu, reinterpret_cast<const void *>(prefill_mfma<T, D, BN, KS, kPad, kSplit>),
+            256 * KS, 0) != hipSuccess)
+      return set_error(MLR_ERR_HIP, "mlr_paged_prefill: device query failed");
+    per_cu_of[dev].store(per_cu, std::memory_order_release);
+  }
+  q.ncu = current_device_cus();
+  if (q.ncu <= 0) return set_error(MLR_ERR_HIP, "mlr_paged_prefill: device query failed");
+  q.pair_cu = per_cu == 2 ? 1 : 0;
+  prefill_mfma<T, D, BN, KS, kPad, kSplit>
+      <<<dim3(static_cast<unsigned>(blocks)), 256 * KS, 0, stream>>>(q);
+  const int rc = check_launch("mlr_paged_prefill(mfma)");
+  if (rc != MLR_OK || !kSplit) return rc;
+  prefill_merge<T, D, BN, kPad>
+      <<<dim3(static_cast<unsigned>(items * q.hq)), 256, 0, stream>>>(q);
+  return check_launch("mlr_paged_prefill(merge)");
 }
 
 template <typename T, int D, int BN, int KS, bool kPad>
 int launch(const PrefillParams &p, int64_t max_query_len, hipStream_t stream) {
+  static_assert(BN == kKeyTile, "key_splits counts tiles of kKeyTile keys");
   PrefillParams q = p;
   q.n_qtiles = static_cast<int>(ceil_div(max_query_len, kBM));
-  const int64_t blocks = static_cast<int64_t>(q.num_seqs) * q.n_qtiles * q.hq;
-  if (blocks > INT32_MAX)
-    return set_error(MLR_ERR_UNSUPPORTED, "mlr_paged_prefill: too many work items");
-  // CU count and workgroups per CU of this kernel, queried once per device
-  // (threads that race here store the same values).
-  constexpr int kMaxDevices = 64;
-  static std::atomic<int> ncu_of[kMaxDevices], per_cu_of[kMaxDevices];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
-    return set_error(MLR_ERR_HIP, "mlr_paged_prefill: no current device");
-  if (ncu_of[dev].load(std::memory_order_acquire) == 0) {
-    int ncu = 0, per_cu = 0;
-    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void *>(prefill_mfma<T, D, BN, KS, kPad>), 256 * KS, 0) !=
-            hipSuccess)
-      return set_error(MLR_ERR_HIP, "mlr_paged_prefill: device query failed");
-    per_cu_of[dev].store(per_cu, std::memory_order_relaxed);
-    ncu_of[dev].store(ncu, std::memory_order_release);
+  q.max_splits = q.split_tiles = 1;
+  const int64_t items = static_cast<int64_t>(q.num_seqs) * q.n_qtiles;
+  const int64_t context = p.qsl != nullptr ? p.max_blocks * p.block_size : p.s_ctx;
+  const KeySplits ks = key_splits(items, q.hq, ceil_div(context, kKeyTile), p.d);
+  if (ks.max_splits > 1 && p.ws != nullptr &&
+      p.ws_bytes >= split_bytes(items, q.hq, D, ks.max_splits)) {
+    q.max_splits = ks.max_splits;
+    q.split_tiles = ks.split_tiles;
+    return launch_kernel<T, D, BN, KS, kPad, true>(q, stream);
   }
-  q.ncu = ncu_of[dev].load(std::memory_order_acquire);
-  q.pair_cu = per_cu_of[dev].load(std::memory_order_relaxed) == 2 ? 1 : 0;
-  prefill_mfma<T, D, BN, KS, kPad><<<dim3(static_cast<unsigned>(blocks)), 256 * KS, 0, stream>>>(q);
-  return check_launch("mlr_paged_prefill(mfma)");
+  return launch_kernel<T, D, BN, KS, kPad, false>(q, stream);
 }
 
 }  // namespace
@@ -813,6 +961,19 @@ bool prefill_mfma_eligible(const PrefillParams &p, int dtype) {
          aligned &&
          p.bs_log2 >= 4 && p.max_blocks * p.block_size < k2g && p.num_blocks < k2g &&
          p.block_size * p.hkv * p.d * 2 < k2g && p.scale > 0.0 && p.scale < 1e30;
+}
+
+size_t prefill_mfma_workspace(int64_t num_seqs, int64_t max_query_len, int64_t max_context,
+                              int64_t num_q_heads, int64_t head_dim, int dtype) {
+  if ((dtype != MLR_DTYPE_BF16 && dtype != MLR_DTYPE_F16) || head_dim % 8 != 0 ||
+      head_dim > 128 || num_seqs <= 0 || max_query_len <= 0 || num_q_heads <= 0)
+    return 0;
+  const int64_t items = num_seqs * ceil_div(max_query_len, kBM);
+  const KeySplits ks =
+      key_splits(items, num_q_heads, ceil_div(max_context, kKeyTile), head_dim);
+  return ks.max_splits > 1
+             ? split_bytes(items, num_q_heads, head_dim <= 64 ? 64 : 128, ks.max_splits)
+             : 0;
 }
 
 template <typename T>

@@ -88,6 +88,20 @@ _PROTOTYPES = {
          _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_f64, _c_int,
          _c_i64, _c_ptr, _c_i64, _c_i64, _c_ptr],
     ),
+    "mlr_paged_prefill_split": (
+        _c_int,
+        [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64,
+         _c_i64, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_i64,
+         _c_i64, _c_f64, _c_int, _c_i64, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_size, _c_ptr],
+    ),
+    "mlr_paged_prefill_chunk_split": (
+        _c_int,
+        [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64,
+         _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_f64, _c_int,
+         _c_i64, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_size, _c_ptr],
+    ),
+    "mlr_paged_prefill_workspace_size": (
+        _c_size, [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int]),
     "mlr_qkv_rope_write": (
         _c_int,
         [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr,

@@ -356,6 +356,18 @@ def _validate_tables(block_tables: torch.Tensor, seq_lens: torch.Tensor,
         raise ValueError("block_tables contain an invalid physical block")
 
 
+def _prefill_workspace(lib, device, num_seqs, max_query_len, max_context, num_q_heads, head_dim,
+                       dcode) -> tuple[torch.Tensor | None, int]:
+    """Scratch of one prefill call whose key ranges are split over workgroups:
+    (tensor or None, bytes). It comes from torch's allocator on the current
+    stream, so calls on different streams never share one."""
+    nbytes = int(lib.mlr_paged_prefill_workspace_size(
+        num_seqs, max_query_len, max_context, num_q_heads, head_dim, dcode))
+    if not nbytes:
+        return None, 0
+    return torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes
+
+
 def paged_prefill_launch(q: torch.Tensor, k_cache: torch.Tensor,
                          v_cache: torch.Tensor, block_tables: torch.Tensor,
                          query_start_loc: torch.Tensor, context_lens: torch.Tensor,
@@ -383,17 +395,20 @@ def paged_prefill_launch(q: torch.Tensor, k_cache: torch.Tensor,
         scale = 1.0 / math.sqrt(head_dim)
     if total_q == 0:
         return out
+    dcode = _lib.dtype_code(q.dtype, "paged prefill")
     with torch.cuda.device(device):
-        status = lib.mlr_paged_prefill(
+        ws, ws_bytes = _prefill_workspace(
+            lib, device, context_lens.shape[0], int(max_query_len),
+            block_tables.shape[1] * block_size, num_q_heads, head_dim, dcode)
+        status = lib.mlr_paged_prefill_split(
             q.data_ptr(), q.stride(0), q.stride(1),
             k_cache.data_ptr(), v_cache.data_ptr(),
             num_blocks, block_size, num_kv_heads, head_dim,
             block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1],
             query_start_loc.data_ptr(), context_lens.data_ptr(),
             context_lens.shape[0], int(max_query_len), num_q_heads, float(scale),
-            _lib.dtype_code(q.dtype, "paged prefill"), int(tile_size),
-            out.data_ptr(), out.stride(0), out.stride(1),
-            _lib.stream_handle(device))
+            dcode, int(tile_size), out.data_ptr(), out.stride(0), out.stride(1),
+            ws.data_ptr() if ws is not None else None, ws_bytes, _lib.stream_handle(device))
     _lib.check(status, "mlr_paged_prefill")
     return out
 
@@ -457,16 +472,18 @@ def paged_attention_prefill_chunk_tiled(
         q = q.contiguous()
     out = torch.empty_like(q, memory_format=torch.contiguous_format)
     num_blocks, _, num_kv_heads, head_dim = k_cache.shape
+    dcode = _lib.dtype_code(q.dtype, "paged_attention_prefill_chunk_tiled")
     with torch.cuda.device(device):
-        status = lib.mlr_paged_prefill_chunk(
+        ws, ws_bytes = _prefill_workspace(lib, device, 1, chunk_len, int(context_len),
+                                          q_num_heads, head_dim, dcode)
+        status = lib.mlr_paged_prefill_chunk_split(
             q.data_ptr(), q.stride(0), q.stride(1),
             k_cache.data_ptr(), v_cache.data_ptr(),
             num_blocks, block_size, num_kv_heads, head_dim,
             table.data_ptr(), table.numel(), int(prefix_len), int(context_len),
             q_num_heads, 1.0 / math.sqrt(head_dim),
-            _lib.dtype_code(q.dtype, "paged_attention_prefill_chunk_tiled"),
-            int(tile_size), out.data_ptr(), out.stride(0), out.stride(1),
-            _lib.stream_handle(device))
+            dcode, int(tile_size), out.data_ptr(), out.stride(0), out.stride(1),
+            ws.data_ptr() if ws is not None else None, ws_bytes, _lib.stream_handle(device))
     _lib.check(status, "mlr_paged_prefill_chunk")
     return out
 
