@@ -413,6 +413,47 @@ int mlr_build_step_metadata(const int64_t *req_info, const int64_t *block_tables
                             int64_t *context_lens, void *stream);
 
 /*
+ * Checks of a step's metadata, in one launch: out[0 .. groups) receives words
+ * whose OR holds the flags below (groups = mlr_check_step_groups(...), 0 when
+ * num_tokens is more than the kernel takes). Request r has tokens
+ * [query_start_loc[r], query_start_loc[r + 1]) (null: token r alone) at
+ * positions context_lens[r] - its count + i; token slots follow
+ * block_tables[r, p / block_size] * block_size + p % block_size. `decoding`
+ * [num_reqs] (or null) sends a request's tokens to the decode flags, and
+ * repeats are looked for within each of the two kinds. With num_reqs == 0
+ * only the slots are checked (range and repeats), with num_tokens == 0 only
+ * the tables. With `detail`, query_start_loc, context_lens and one word per
+ * request (1: an invalid block id under its context) follow the flags. Every
+ * index is clamped, so malformed metadata is read in bounds.
+ *
+ * Replaces the checks of model/qwen2.py:578-602,
+ * kernels/reference/paged_attention.py:224-238 and
+ * runtime/paged_kv_cache.py:235-239.
+ */
+enum mlr_check_flags {
+  MLR_CHECK_CONTEXT = 1,       /* a context length <= 0 */
+  MLR_CHECK_WIDTH = 2,         /* a context past its block table */
+  MLR_CHECK_BLOCK = 4,         /* an invalid block id under a context */
+  MLR_CHECK_QSL_START = 8,     /* query_start_loc[0] != 0 */
+  MLR_CHECK_QSL_ORDER = 16,    /* a request without tokens */
+  MLR_CHECK_QSL_END = 32,      /* query_start_loc[num_reqs] != num_tokens */
+  MLR_CHECK_QUERY_LEN = 64,    /* more tokens than max_query_len */
+  MLR_CHECK_COVER = 128,       /* a context shorter than its tokens */
+  MLR_CHECK_SLOT_RANGE = 256,  /* a slot outside the pool */
+  MLR_CHECK_POSITION = 512,    /* a token's position */
+  MLR_CHECK_SLOT = 1024,       /* a token's slot */
+  MLR_CHECK_REPEAT = 2048,     /* a slot twice */
+  MLR_CHECK_DECODE_SHIFT = 3   /* the last three of decode tokens: << 3 */
+};
+int64_t mlr_check_step_groups(int64_t num_reqs, int64_t num_tokens);
+int mlr_check_step(const int64_t *block_tables, int64_t block_table_stride, int64_t max_blocks,
+                   const int64_t *context_lens, int64_t num_reqs,
+                   const int64_t *query_start_loc, const int64_t *positions,
+                   const int64_t *slot_mapping, int64_t num_tokens, const uint8_t *decoding,
+                   int64_t block_size, int64_t num_blocks, int64_t max_query_len, int detail,
+                   int64_t *out, int64_t out_len, void *stream);
+
+/*
  * RMSNorm of `rows` rows of `hidden` elements, after a residual add when
  * `residual` is given:
  *   r   = x + residual, rounded to the dtype and written to residual_out

@@ -24,6 +24,7 @@ from typing import Sequence
 import torch
 
 from .. import _lib
+from .step_checks import BLOCK, CONTEXT, WIDTH, step_flags
 
 _DEFAULT_TILE = 64
 
@@ -337,7 +338,11 @@ def paged_attention_decode_batch_parallel(
 
 def _validate_tables(block_tables: torch.Tensor, seq_lens: torch.Tensor,
                      block_size: int, num_blocks: int) -> None:
-    """One device reduction and one host sync for all table checks."""
+    """One launch and one host sync for all table checks."""
+    bits = step_flags(block_size, num_blocks, tables=block_tables, ctx=seq_lens)
+    if bits is not None:
+        _raise_table_errors(bits & CONTEXT, bits & WIDTH, bits & BLOCK)
+        return
     width = block_tables.shape[1]
     required = (seq_lens + block_size - 1) // block_size
     columns = torch.arange(width, device=block_tables.device)
@@ -348,11 +353,15 @@ def _validate_tables(block_tables: torch.Tensor, seq_lens: torch.Tensor,
         (required > width).any(),
         bad_ids.any(),
     ]).cpu()
-    if bool(flags[0]):
+    _raise_table_errors(*flags.tolist())
+
+
+def _raise_table_errors(context, width, block) -> None:
+    if context:
         raise ValueError("seq_lens must be greater than 0")
-    if bool(flags[1]):
+    if width:
         raise ValueError("block_tables have insufficient blocks for seq_lens")
-    if bool(flags[2]):
+    if block:
         raise ValueError("block_tables contain an invalid physical block")
 
 

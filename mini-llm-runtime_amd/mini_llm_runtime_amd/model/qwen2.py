@@ -29,6 +29,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ..kernels import layer_ops as kops
+from ..kernels import step_checks as kchk
 from ..runtime.paged_kv_cache import PagedKVCache
 from .qwen2_attention import Qwen2Attention, _raise_first
 
@@ -219,6 +220,23 @@ class Qwen2DecoderLayer(nn.Module):
                 layer_idx=layer_idx, slot_mapping=slot_mapping, block_tables=block_tables,
                 query_start_loc=query_start_loc, context_lens=context_lens,
                 max_query_len=max_query_len))
+
+
+def _raise_packed_errors(flags) -> None:
+    """The errors of a packed prefill's metadata, in order."""
+    _raise_first([
+        (flags[0], ValueError("query_start_loc must start at 0")),
+        (flags[1], ValueError("query_start_loc must be strictly increasing")),
+        (flags[2], ValueError("query_start_loc must end at the packed token count")),
+        (flags[3], ValueError("max_query_len is smaller than a request's token count")),
+        (flags[4], ValueError("context_lens must cover each request's tokens")),
+        (flags[5], ValueError("block_tables have insufficient blocks for context_lens")),
+        (flags[6], ValueError("block_tables contain an invalid physical block")),
+        (flags[7], ValueError("position_ids must run from context_len - num_tokens "
+                              "to context_len - 1 for each request")),
+        (flags[8], ValueError("slot_mapping must match block_tables and positions")),
+        (flags[9], ValueError("packed tokens must use distinct write slots")),
+    ])
 
 
 class TinyQwen2Model(nn.Module):
@@ -442,6 +460,14 @@ class TinyQwen2Model(nn.Module):
                                query_start_loc, context_lens, max_query_len,
                                num_tokens) -> None:
         bs, width = kv_cache.block_size, block_tables.shape[1]
+        bits = kchk.step_flags(bs, kv_cache.num_blocks, tables=block_tables, ctx=context_lens,
+                               qsl=query_start_loc, positions=position_ids, slots=slot_mapping,
+                               max_query_len=max_query_len)
+        if bits is not None:
+            _raise_packed_errors([bits & f for f in (
+                kchk.QSL_START, kchk.QSL_ORDER, kchk.QSL_END, kchk.QUERY_LEN, kchk.COVER,
+                kchk.WIDTH, kchk.BLOCK, kchk.POSITION, kchk.SLOT, kchk.REPEAT)])
+            return
         device = position_ids.device
         lens = query_start_loc[1:] - query_start_loc[:-1]
         # Request of each packed row: how many request ends lie at or before
@@ -470,19 +496,7 @@ class TinyQwen2Model(nn.Module):
             (slot_mapping != expected).any(),
             (ordered[1:] == ordered[:-1]).any(),
         ]).tolist()
-        _raise_first([
-            (flags[0], ValueError("query_start_loc must start at 0")),
-            (flags[1], ValueError("query_start_loc must be strictly increasing")),
-            (flags[2], ValueError("query_start_loc must end at the packed token count")),
-            (flags[3], ValueError("max_query_len is smaller than a request's token count")),
-            (flags[4], ValueError("context_lens must cover each request's tokens")),
-            (flags[5], ValueError("block_tables have insufficient blocks for context_lens")),
-            (flags[6], ValueError("block_tables contain an invalid physical block")),
-            (flags[7], ValueError("position_ids must run from context_len - num_tokens "
-                                  "to context_len - 1 for each request")),
-            (flags[8], ValueError("slot_mapping must match block_tables and positions")),
-            (flags[9], ValueError("packed tokens must use distinct write slots")),
-        ])
+        _raise_packed_errors(flags)
 
 
 class TinyQwen2ForCausalLM(nn.Module):

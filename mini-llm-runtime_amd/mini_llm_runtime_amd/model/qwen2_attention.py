@@ -40,6 +40,7 @@ import torch.nn as nn
 from ..kernels import layer_ops as kops
 from ..kernels import paged_attention as kpa
 from ..kernels import pre_attention as kpre
+from ..kernels import step_checks as kchk
 from ..runtime.paged_kv_cache import PagedKVCache
 
 
@@ -142,6 +143,18 @@ def _raise_first(checks) -> None:
     for failed, error in checks:
         if failed:
             raise error
+
+
+def _raise_decode_errors(flags) -> None:
+    """The reference's errors of a decode batch's metadata, in its order."""
+    _raise_first([
+        (flags[0], ValueError("context_lens must be greater than 0")),
+        (flags[1], ValueError("decode positions must equal context_lens - 1")),
+        (flags[2], ValueError("block_tables have insufficient blocks for context_lens")),
+        (flags[3], ValueError("block_tables contain an invalid physical block")),
+        (flags[4], ValueError("slot_mapping must match block_tables and positions")),
+        (flags[5], ValueError("decode requests must use distinct write slots")),
+    ])
 
 
 class Qwen2Attention(nn.Module):
@@ -398,6 +411,12 @@ class Qwen2Attention(nn.Module):
         width = block_tables.shape[1]
         batch = block_tables.shape[0]
         positions = position_ids[:, 0]
+        bits = kchk.step_flags(bs, nblocks, tables=block_tables, ctx=context_lens,
+                               positions=positions, slots=slot_mapping)
+        if bits is not None:
+            _raise_decode_errors([bits & kchk.CONTEXT, bits & kchk.POSITION, bits & kchk.WIDTH,
+                                  bits & kchk.BLOCK, bits & kchk.SLOT, bits & kchk.REPEAT])
+            return
         required = (context_lens + bs - 1) // bs
         columns = torch.arange(width, device=block_tables.device)
         used = columns[None, :] < required[:, None]
@@ -416,14 +435,7 @@ class Qwen2Attention(nn.Module):
             (ordered[1:] == ordered[:-1]).any() if batch > 1 else torch.zeros(
                 (), dtype=torch.bool, device=slot_mapping.device),
         ]).tolist()
-        _raise_first([
-            (flags[0], ValueError("context_lens must be greater than 0")),
-            (flags[1], ValueError("decode positions must equal context_lens - 1")),
-            (flags[2], ValueError("block_tables have insufficient blocks for context_lens")),
-            (flags[3], ValueError("block_tables contain an invalid physical block")),
-            (flags[4], ValueError("slot_mapping must match block_tables and positions")),
-            (flags[5], ValueError("decode requests must use distinct write slots")),
-        ])
+        _raise_decode_errors(flags)
 
     # ------------------------------------------------------------------
     # Packed prefill of several requests (no counterpart in the reference's

@@ -39,6 +39,7 @@ from dataclasses import dataclass
 import torch
 
 from ..kernels import paged_attention as kpa
+from ..kernels import step_checks as kchk
 from .paged_kv_cache import PagedKVCache
 from .request import Request, RequestStatus
 from .scheduler import Scheduler, SchedulerOutput
@@ -202,14 +203,14 @@ def _build_on_device(entries, block_size: int, dev: torch.device) -> ModelBatch:
     )
 
 
-def _upload(values, device: torch.device) -> torch.Tensor:
-    """A host list of ints as an int64 tensor on `device`. For a GPU the list
+def _upload(values, device: torch.device, dtype: torch.dtype = torch.long) -> torch.Tensor:
+    """A host list of ints as an int64 (or `dtype`) tensor on `device`. For a GPU the list
     is staged in pinned memory and copied asynchronously on the current
     stream, so the host does not wait for the kernels already queued there
     (a copy from pageable memory would)."""
     if device.type != "cuda":
-        return torch.tensor(values, dtype=torch.long, device=device)
-    staged = torch.tensor(values, dtype=torch.long, pin_memory=True)
+        return torch.tensor(values, dtype=dtype, device=device)
+    staged = torch.tensor(values, dtype=dtype, pin_memory=True)
     return staged.to(device, non_blocking=True)
 
 
@@ -275,16 +276,29 @@ def _check_batch(model, batch: ModelBatch, kv_cache: PagedKVCache) -> tuple[list
     # context uses lies outside the cache (blocks needed: ceil(ctx / bs), none
     # for ctx <= 0).
     bs, width = kv_cache.block_size, batch.block_tables.shape[1]
-    required_dev = torch.div(batch.context_lens + (bs - 1), bs,
-                             rounding_mode="floor").clamp_(min=0)
-    used = torch.arange(width, device=device)[None, :] < required_dev[:, None]
-    bad = (used & ((batch.block_tables < 0)
-                   | (batch.block_tables >= kv_cache.num_blocks))).any(dim=1)
-    flags = _step_metadata_flags(batch, bs, width, device)
-    host = torch.cat([batch.query_start_loc, batch.context_lens, bad.long(),
-                      flags.long()]).tolist()
-    qsl, ctx, bad_rows = host[:n + 1], host[n + 1:2 * n + 1], host[2 * n + 1:3 * n + 1]
-    flags = host[3 * n + 1:]
+    found = None
+    if num_tokens > 0:
+        decoding = _upload([ph is RequestStatus.DECODING for ph in batch.request_phases],
+                           device, torch.uint8)
+        found = kchk.step_flags(bs, kv_cache.num_blocks, tables=batch.block_tables,
+                                ctx=batch.context_lens, qsl=batch.query_start_loc,
+                                positions=batch.positions, slots=batch.slot_mapping,
+                                decoding=decoding, detail=True)
+    if found is not None:
+        bits, qsl, ctx, bad_rows = found
+        flags = [bits & (f << s) for s in (0, kchk.DECODE_SHIFT)
+                 for f in (kchk.POSITION, kchk.SLOT, kchk.REPEAT)]
+    else:
+        required_dev = torch.div(batch.context_lens + (bs - 1), bs,
+                                 rounding_mode="floor").clamp_(min=0)
+        used = torch.arange(width, device=device)[None, :] < required_dev[:, None]
+        bad = (used & ((batch.block_tables < 0)
+                       | (batch.block_tables >= kv_cache.num_blocks))).any(dim=1)
+        flags = _step_metadata_flags(batch, bs, width, device)
+        host = torch.cat([batch.query_start_loc, batch.context_lens, bad.long(),
+                          flags.long()]).tolist()
+        qsl, ctx, bad_rows = host[:n + 1], host[n + 1:2 * n + 1], host[2 * n + 1:3 * n + 1]
+        flags = host[3 * n + 1:]
     if qsl[0] != 0:
         raise ValueError("query_start_loc must start at 0")
     if any(b <= a for a, b in zip(qsl, qsl[1:])):

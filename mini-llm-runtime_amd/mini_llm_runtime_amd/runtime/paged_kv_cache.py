@@ -19,6 +19,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
+from ..kernels.step_checks import REPEAT, SLOT_RANGE, step_flags
 
 
 class PagedKVCache:
@@ -191,14 +192,22 @@ class PagedKVCache:
         if slot_mapping.numel() == 0:
             return
         num_slots = self.num_blocks * self.block_size
+        bits = step_flags(self.block_size, self.num_blocks, slots=slot_mapping.to(torch.long))
+        if bits is not None:
+            self._raise_slot_errors(bits & SLOT_RANGE, bits & REPEAT)
+            return
         ordered = slot_mapping.sort().values
         flags = torch.stack([
             ((ordered[0] < 0) | (ordered[-1] >= num_slots)),
             (ordered[1:] == ordered[:-1]).any(),
         ]).cpu()
-        if bool(flags[0]):
+        self._raise_slot_errors(*flags.tolist())
+
+    @staticmethod
+    def _raise_slot_errors(out_of_range, repeated) -> None:
+        if out_of_range:
             raise IndexError("slot_mapping contains an out-of-range slot")
-        if bool(flags[1]):
+        if repeated:
             raise ValueError("slot_mapping must contain distinct slots")
 
     def _launch_write(self, slot_mapping: torch.Tensor, k: torch.Tensor,
