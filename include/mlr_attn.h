@@ -413,6 +413,15 @@ int mlr_build_step_metadata(const int64_t *req_info, const int64_t *block_tables
                             int64_t *context_lens, void *stream);
 
 /*
+ * dst[i] = host_values[i] for i < n <= 3840, each within 32 bits: a short list
+ * in HOST memory to device memory as kernel arguments, without a wait; the
+ * list may be reused once the call returns. Stands for the
+ * torch.tensor(list, device=...) of the block table in
+ * kernels/reference/paged_attention.py:60-75.
+ */
+int mlr_stage_i64(const int64_t *host_values, int64_t n, int64_t *dst, void *stream);
+
+/*
  * Checks of a step's metadata, in one launch: out[0 .. groups) receives words
  * whose OR holds the flags below (groups = mlr_check_step_groups(...), 0 when
  * num_tokens is more than the kernel takes). Request r has tokens

@@ -114,6 +114,7 @@ _PROTOTYPES = {
         [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr,
          _c_ptr, _c_ptr, _c_ptr],
     ),
+    "mlr_stage_i64": (_c_int, [_c_ptr, _c_i64, _c_ptr, _c_ptr]),
     "mlr_check_step_groups": (_c_i64, [_c_i64, _c_i64]),
     "mlr_check_step": (
         _c_int,

@@ -19,6 +19,7 @@ Numerics (FP32 softmax statistics; P@V in FP32 for the chunk path):
 from __future__ import annotations
 
 import math
+from array import array
 from typing import Sequence
 
 import torch
@@ -35,6 +36,44 @@ def _as_index_tensor(values, device: torch.device) -> torch.Tensor:
     else:
         tensor = torch.as_tensor(list(values), dtype=torch.long, device=device)
     return tensor
+
+
+# Longest host list that mlr_stage_i64 takes (four launches).
+_STAGE_MAX = 3840
+
+
+def _host_blocks(entries, required: int, num_blocks: int) -> array | None:
+    """The first `required` block ids of a host table as an int64 array, or
+    None when one of them is out of range."""
+    try:
+        used = array("q", entries)
+    except TypeError:  # numpy or tensor elements
+        used = array("q", [int(b) for b in entries])
+    except OverflowError:
+        return None
+    del used[required:]
+    if used and (min(used) < 0 or max(used) >= num_blocks):
+        return None
+    return used
+
+
+def _device_ints(values: array, device: torch.device) -> torch.Tensor:
+    """An int64 array as a tensor on `device`, for the call that follows on
+    torch's current stream. A short one travels as kernel arguments; a copy
+    from host memory would wait for the work queued on the stream. Refused
+    under graph capture, as that copy is: a replay would see these values."""
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("a host block table cannot be captured into a graph; "
+                           "pass the table as a device tensor to a batched call")
+    n = len(values)
+    if n > _STAGE_MAX or (n and max(values) > 0x7FFFFFFF):
+        return torch.tensor(values, dtype=torch.long, device=device)
+    out = torch.empty(n, dtype=torch.long, device=device)
+    with torch.cuda.device(device):
+        status = _lib.load().mlr_stage_i64(values.buffer_info()[0], n, out.data_ptr(),
+                                           _lib.stream_handle(device))
+    _lib.check(status, "mlr_stage_i64")
+    return out
 
 
 def _check_cache_pair(k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
@@ -242,14 +281,16 @@ def paged_attention_decode(
         raise ValueError("block_table does not contain enough blocks for seq_len")
     if block_size != k_cache.shape[1]:
         raise ValueError("block_size does not match KV cache layout")
-    used = [int(b) for b in list(block_table)[:required_blocks]]
-    if any(b < 0 or b >= k_cache.shape[0] for b in used):
+    used = _host_blocks(list(block_table)[:required_blocks], required_blocks,
+                        k_cache.shape[0])
+    if used is None:
         raise ValueError("block_table contains an out-of-range physical block")
     _require_kernel_layout(q, k_cache, v_cache, "paged_attention_decode")
     device = _lib.require_hip(q, k_cache, v_cache, what="paged_attention_decode")
-    table = torch.tensor([used], dtype=torch.long, device=device)
-    lens = torch.tensor([seq_len], dtype=torch.long, device=device)
-    out = paged_decode_launch(q.unsqueeze(0), k_cache, v_cache, table, lens)
+    used.append(int(seq_len))
+    staged = _device_ints(used, device)
+    out = paged_decode_launch(q.unsqueeze(0), k_cache, v_cache, staged[:-1].unsqueeze(0),
+                              staged[-1:])
     return out.squeeze(0)
 
 
@@ -469,12 +510,13 @@ def paged_attention_prefill_chunk_tiled(
         if bool(((used < 0) | (used >= k_cache.shape[0])).any().cpu()):
             raise ValueError("block_table contains an out-of-range physical block")
     else:
-        entries = [int(b) for b in block_table]
+        entries = list(block_table)
         if len(entries) < required_blocks:
             raise IndexError("block_table does not cover context_len")
-        if any(b < 0 or b >= k_cache.shape[0] for b in entries[:required_blocks]):
+        used = _host_blocks(entries, required_blocks, k_cache.shape[0])
+        if used is None:
             raise ValueError("block_table contains an out-of-range physical block")
-        table = torch.tensor(entries[:required_blocks], dtype=torch.long, device=device)
+        table = _device_ints(used, device)
     table = table.contiguous()
     lib = _lib.load()
     if q.stride(-1) != 1:
@@ -532,8 +574,8 @@ def paged_attention_prefill_varlen(
     block_tables = _as_index_tensor(block_tables, device)
     query_start_loc = _as_index_tensor(query_start_loc, device)
     context_lens = _as_index_tensor(context_lens, device)
-    qlens = query_start_loc[1:] - query_start_loc[:-1]
     if max_query_len is None:
+        qlens = query_start_loc[1:] - query_start_loc[:-1]
         max_query_len = int(qlens.max().item()) if qlens.numel() else 0
     return paged_prefill_launch(q, k_cache, v_cache, block_tables, query_start_loc,
                                 context_lens, max_query_len, tile_size=tile_size)
