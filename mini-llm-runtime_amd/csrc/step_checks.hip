@@ -10,11 +10,11 @@
 // requests took 105 us for a 7 us kernel.
 //
 // Workgroup j takes the table rows j, j + G, ... (one row at a time, its 256
-// threads along the columns) and the tokens [256 j, 256 j + 256): it finds
-// each token's request by binary search in query_start_loc, compares position
-// and slot with what the table gives, and its slot with those of all earlier
-// tokens, which pass through LDS (n^2 / 2 broadcast reads: 4 us at 2,048
-// tokens, where a sort takes 24). Every workgroup writes one word of
+// threads along the columns) and the tokens [64 j, 64 j + 64): it finds each
+// token's request by binary search in query_start_loc, compares position and
+// slot with what the table gives, and its slot with those of all earlier
+// tokens, which pass through LDS as broadcast reads, a quarter per wave
+// (6.4 us at 1,021 tokens, 9.5 at 2,048, where a sort takes 22 and 27). Every workgroup writes one word of
 // flags of its own, so there is nothing to clear first and nothing to add
 // up; the host reads the words in the one transfer that it waits for anyway.
 #include <algorithm>
@@ -25,6 +25,7 @@ namespace mlr {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kTokens = 64;       // tokens per workgroup
 constexpr int kTile = 1024;       // earlier tokens staged at a time
 constexpr int kMaxGroups = 256;   // workgroups, unless the tokens need more
 constexpr int64_t kMaxTokens = 8192;  // past this a sort finds a repeat sooner
@@ -47,7 +48,8 @@ struct CheckParams {
 };
 
 __global__ __launch_bounds__(kThreads) void check_step(CheckParams p) {
-  __shared__ int64_t keys[kTile];
+  __shared__ __align__(16) int64_t keys[kTile];
+  __shared__ int64_t own[kTokens];
   __shared__ unsigned int wave_flags[kThreads / kWave];
   const int tid = threadIdx.x, groups = gridDim.x;
   const int64_t bs = p.block_size;
@@ -87,8 +89,10 @@ __global__ __launch_bounds__(kThreads) void check_step(CheckParams p) {
     if (p.qsl[p.reqs] != p.tokens) flags |= MLR_CHECK_QSL_END;
   }
 
-  const int t = blockIdx.x * kThreads + tid;
-  const int first = blockIdx.x * kThreads;
+  // Lane i of every wave holds token first + i; wave 0 checks it, and all four
+  // look for its slot among a quarter of the earlier tokens each.
+  const int first = blockIdx.x * kTokens, lane = tid % kWave, wave = tid / kWave;
+  const int t = first + lane;
   if (first < p.tokens) {  // uniform
     // The request of token u: how many request ends lie at or before it.
     auto owner = [&](int u) -> int {
@@ -109,15 +113,17 @@ __global__ __launch_bounds__(kThreads) void check_step(CheckParams p) {
     int64_t mine = 0;
     unsigned int shift = 0;
     if (t < p.tokens) {
-      const int64_t slot = p.slots[t];
       mine = key_of(t);
+      if (p.decoding != nullptr && p.decoding[owner(t)]) shift = MLR_CHECK_DECODE_SHIFT;
+    }
+    if (wave == 0 && t < p.tokens) {
+      const int64_t slot = p.slots[t];
       if (slot < 0 || slot >= p.num_blocks * bs) flags |= MLR_CHECK_SLOT_RANGE;
       if (p.reqs > 0) {
         const int r = owner(t);
         const int64_t start = p.qsl != nullptr ? p.qsl[r] : t;
         const int64_t len = p.qsl != nullptr ? p.qsl[r + 1] - start : 1;
         const int64_t pos = p.positions[t];
-        if (p.decoding != nullptr && p.decoding[r]) shift = MLR_CHECK_DECODE_SHIFT;
         if (pos != p.ctx[r] - len + (t - start)) flags |= MLR_CHECK_POSITION << shift;
         int64_t col = pos >= 0 ? pos / bs : 0;
         col = col > p.width - 1 ? p.width - 1 : col;
@@ -126,17 +132,26 @@ __global__ __launch_bounds__(kThreads) void check_step(CheckParams p) {
           flags |= MLR_CHECK_SLOT << shift;
       }
     }
-    const int last = min(p.tokens, first + kThreads);
-    for (int base = 0; base < last; base += kTile) {
-      const int n = min(kTile, last - base);
+    bool same = false;
+    // Whole workgroups of earlier tokens: no bounds, two keys a read.
+    for (int base = 0; base < first; base += kTile) {
+      const int n = min(kTile, first - base);  // a multiple of kTokens
       __syncthreads();
       for (int i = tid; i < n; i += kThreads) keys[i] = key_of(base + i);
       __syncthreads();
-      const int mine_n = t < p.tokens ? min(n, t - base) : 0;  // tokens before this one
-      bool same = false;
-      for (int i = 0; i < mine_n; ++i) same |= keys[i] == mine;
-      if (same) flags |= MLR_CHECK_REPEAT << shift;
+      const longlong2 *part = reinterpret_cast<const longlong2 *>(keys + wave * (n / 4));
+#pragma unroll 8
+      for (int i = 0; i < n / 8; ++i) {
+        const longlong2 k = part[i];
+        same |= k.x == mine || k.y == mine;
+      }
     }
+    if (wave == 0) {  // its own earlier lanes, through LDS within the wave
+      own[lane] = mine;
+      __builtin_amdgcn_wave_barrier();
+      for (int i = 0; i < kTokens; ++i) same |= i < lane && own[i] == mine;
+    }
+    if (same && t < p.tokens) flags |= MLR_CHECK_REPEAT << shift;
   }
 
 #pragma unroll
@@ -157,7 +172,7 @@ using namespace mlr;
 extern "C" int64_t mlr_check_step_groups(int64_t num_reqs, int64_t num_tokens) {
   if (num_reqs < 0 || num_tokens < 0 || num_tokens > kMaxTokens || num_reqs >= INT32_MAX) return 0;
   return std::max<int64_t>({1, std::min<int64_t>(num_reqs, kMaxGroups),
-                            ceil_div(num_tokens, kThreads)});
+                            ceil_div(num_tokens, kTokens)});
 }
 
 extern "C" int mlr_check_step(const int64_t *block_tables, int64_t block_table_stride,

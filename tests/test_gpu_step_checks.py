@@ -116,7 +116,7 @@ def test_same_errors_as_the_torch_checks(device, reqs):
     assert len(seen) > 3
 
 
-@pytest.mark.parametrize("tokens", [1, 255, 256, 257, 1025, 8192, 8193])
+@pytest.mark.parametrize("tokens", [1, 63, 64, 65, 257, 1025, 1089, 8192, 8193])
 def test_repeated_and_out_of_range_slots(device, tokens):
     rng = random.Random(tokens)
     caches = [PagedKVCache(1, 600, 16, 1, 8, device=d) for d in ("cpu", device)]
