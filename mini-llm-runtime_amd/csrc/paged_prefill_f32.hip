@@ -1,218 +1,370 @@
-// FP32 paged chunk prefill on gfx950 matrix cores (v_mfma_f32_16x16x4_f32).
+// FP32 paged chunk prefill on gfx950 matrix cores (v_mfma_f32_32x32x2_f32).
 //
-// One workgroup = 64 queries of one query head as four waves of 16 queries.
-// The waves share no LDS and no barrier: each runs its own key range, the
-// keys up to its last query's position. Per wave and block of 16 keys:
-//   S^T[16 keys x 16 queries] = K[16 keys x D] . Q^T[D x 16 queries] in D/4
-//     MFMAs. Step (j, e) takes dims 16j + 4g + e from lane group g = l/16:
-//     lane l holds key l%16's row chunk j (one 16-byte load per j) and query
-//     l%16's matching Q chunk, loaded once and pre-multiplied by
-//     scale*log2(e), so the scores come out in base-2 units.
-//   Lane l then holds S^T[keys 4g..4g+3][query l%16]. A query's 16 scores
-//     sit in the four lanes l%16 + 16g', so its row max is two lane swaps;
-//     its row sum is kept per lane and added across those lanes once, at the
-//     end.
-//   O^T += V^T . P^T in D/4 MFMAs: step i takes keys 4g + i, whose
-//     probabilities are the lane's four values; dim block c takes dims
-//     VC*m + c of row m (VC = D/16), so lane l loads VC consecutive floats of
-//     each of its four V rows with vector loads, and accumulator c holds
-//     O^T[dim VC*(4g + i) + c][query l%16]: VC consecutive dims per lane and
-//     i, one vector store per i at the end.
-// Each wave issues the next block's K and V loads before the current
-// block's MFMAs, so one block's loads are in flight while the matrix cores
-// work (8 x 512-token chunks in FP32: 665 us per call against 717 us without).
-// Keys past the last one the wave needs, and keys of an out-of-range block
-// id, load as zeros and are masked; so are keys past a query's position
-// (causal by absolute position). Rows the wave does not need are never
-// read, so unwritten rows of the pool (whatever they hold) never reach a
-// product.
+// One workgroup = 32 queries of one query head; its waves deal the 32-key
+// tiles of the context round-robin and merge their (m, l, O) through LDS at
+// the end. Per wave and tile:
+//   S^T[32 keys x 32 queries] = K[32 keys x D] . Q^T[D x 32 queries], D/2
+//     MFMAs. Lane l holds K row l%32 and Q row l%32, floats 8j + 4(l/32) ..
+//     +4 of 8-float block j (one 16-byte load each): MFMA e of block j takes
+//     element e of both, so the k pairs of an MFMA lie 4 floats apart in K and
+//     Q alike. Q is loaded once, pre-multiplied by scale*log2(e).
+//   Lane l then holds the scores of query l%32 and keys 8(i/4) + 4(l/32) + i%4,
+//     i < 16: the row max is 15 maxima and one swap with lane l^32; row sums
+//     stay per lane until the end. Online softmax in FP32, base 2.
+//   O^T[32 dims x 32 queries] += V^T[32 dims x 2 keys] . P^T[2 keys x 32
+//     queries], 16 steps for each of D/32 accumulators: step i takes the two
+//     keys whose probabilities lanes l and l^32 hold in register i. Dim m of
+//     accumulator c is dim VC*m + c (VC = D/32), so lane l loads VC
+//     consecutive floats of a V row.
+//
+// What bounds it: the FP32 matrix cores (152 TFLOP/s by a large product), if
+// the loads arrive in time. K and V of a tile are 16 KB (D = 64) for 8192
+// matrix-core cycles, so each wave reads them straight from L2 without LDS.
+// There is one buffer of each: the next tile's K is requested once this
+// tile's S^T has read K, and lands during the softmax and P.V; the next V
+// once P.V has read V, and lands during S^T. Block ids come 32 tiles at a
+// time, one per lane, so no load waits for a table lookup. The kernel before
+// this one (16 queries a wave, one 16-key block in flight behind a block id
+// load each) took 256 us for 4 sequences of 100..700 queries on prefixes up
+// to 1,500, 14/2 heads of 64 (36 TFLOP/s); this one takes 117 us (78 TFLOP/s), and 8
+// x 512 queries after 2,000 keys 454 and 334 us (99 TFLOP/s).
+//
+// K rows past the last key the workgroup needs are read as that key's row and
+// masked, V rows past it as zeros; so are the rows of an out-of-range block.
+// Unwritten pool rows never reach a product. Head sizes other than 32, 64 and 128 (multiples of 4 up to 128) run
+// in the next larger kernel with the dims past the head as zeros.
 //
 // Numerics: FP32 products and sums throughout (the reference's FP32 path,
-// kernels/reference/paged_attention.py:346-434), online softmax in base 2;
-// the scale is folded into q (one FP32 rounding). The reference's tile_size
-// only orders its FP32 accumulation, as here the 16-key blocks do.
+// kernels/reference/paged_attention.py:346-434); the scale is folded into q
+// (one FP32 rounding). The reference's tile_size only orders its FP32
+// accumulation, as the tiles and waves here do.
 //
-// Work: items are (sequence, 64-query tile) pairs, each run once per query
+// Work: items are (sequence, 32-query tile) pairs, each run once per query
 // head. Workgroup b goes to XCD b mod 8 (the dispatcher deals workgroups to
 // the XCDs in turn), and the query heads of one item get workgroups of one
 // residue mod 8, so the K/V rows a GQA group re-reads come from one L2.
-// Items start last query tile first: later tiles see more keys.
+// Items start with the most keys first: ranked by every workgroup where there
+// are at most 256 of several sequences, else last query tile first.
 #include "paged_prefill.h"
 
 namespace mlr {
 namespace {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 constexpr float kLog2eF32 = 1.4426950408889634f;
-constexpr int kQW = 16;      // queries per wave
-constexpr int kBMF = 64;     // queries per workgroup (four waves)
+constexpr int kBMF = 32;   // queries per workgroup
+constexpr int kBNF = 32;   // keys per tile
+// Work items ranked by their keys: at most kRankMax of them, and only where
+// contexts pass kRankKeys keys (the ranking takes 3 us: 25 us against 22 for
+// 4 x 300 tokens, but 117 against 173 for 4 ragged chunks on ragged prefixes).
+constexpr int kRankMax = 256;
+constexpr int kRankKeys = 512;
 
-__device__ __forceinline__ float swap_max(float x, int lanes) {
-  return fmaxf(x, __shfl_xor(x, lanes, 64));
+template <int VC> struct VecOf { typedef float type __attribute__((ext_vector_type(VC))); };
+template <> struct VecOf<1> { typedef float type; };
+
+__device__ __forceinline__ float other_half_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x),
+                                                  false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
-template <int D>
-__global__ __launch_bounds__(256) void prefill_f32_mfma(PrefillParams p) {
-  constexpr int QK = D / 16;  // 16-dim chunks of a row (S^T k-steps: 4 each)
-  constexpr int VC = D / 16;  // dims per lane and V row (O^T dim blocks)
+// kWaves waves per workgroup.
+template <int D, int kWaves, bool kPad>
+__global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p) {
+  constexpr int QK = D / 8;   // 8-float blocks of a row
+  constexpr int VC = D / 32;  // dims per lane and V row; O^T accumulators
+  typedef typename VecOf<VC>::type vec_t;
   const int nqt = p.n_qtiles;
   const int nitems = p.num_seqs * nqt;
   const int b = static_cast<int>(blockIdx.x);
-  const int t = b >> 3;
-  const int h = t % p.hq;
-  const int rank = (t / p.hq) * 8 + (b & 7);
+  const int tb = b >> 3;
+  const int h = tb % p.hq;
+  const int rank = (tb / p.hq) * 8 + (b & 7);
   if (rank >= nitems) return;  // uniform: the grid is padded to whole groups of 8
-  const int seq = rank % p.num_seqs;
-  const int qt = nqt - 1 - rank / p.num_seqs;
-  SeqRange rg = seq_range(p, seq);
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wq = qt * kBMF + kQW * wv;  // the wave's first query (chunk index)
+  int seq = rank % p.num_seqs, qt = nqt - 1 - rank / p.num_seqs;
+  if (kWaves >= 4 && p.num_seqs > 1 && nitems <= kRankMax &&
+      p.max_blocks * p.block_size > kRankKeys) {  // uniform
+    // The item with `rank` items of more keys (ties by index).
+    __shared__ __align__(16) int keys_s[kRankMax];
+    __shared__ int item_s;
+    const int i = threadIdx.x;
+    int mine = 0;
+    if (i < kRankMax) {
+      if (i < nitems) {
+        const SeqRange r = seq_range(p, i / nqt);
+        const int64_t lo = static_cast<int64_t>(i % nqt) * kBMF;
+        mine = lo < r.qlen ? static_cast<int>(r.prefix + min<int64_t>(r.qlen, lo + kBMF)) : 0;
+      }
+      keys_s[i] = mine;
+    }
+    __syncthreads();
+    if (i < nitems) {
+      int above = 0;
+      for (int j = 0; j < nitems; j += 4) {
+        const int4 o = *reinterpret_cast<const int4 *>(keys_s + j);
+        above += (o.x > mine || (o.x == mine && j < i)) + (o.y > mine || (o.y == mine && j + 1 < i)) +
+                 (o.z > mine || (o.z == mine && j + 2 < i)) +
+                 (o.w > mine || (o.w == mine && j + 3 < i));
+      }
+      if (above == rank) item_s = i;
+    }
+    __syncthreads();
+    const int item = __builtin_amdgcn_readfirstlane(item_s);
+    seq = item / nqt;
+    qt = item % nqt;
+  }
+  const int q0 = qt * kBMF;
+  const SeqRange rg = seq_range(p, seq);
   const int qlen = static_cast<int>(rg.qlen);
-  if (wq >= qlen) return;  // uniform per wave; no barrier follows
+  if (q0 >= qlen) return;  // uniform
   const int prefix = static_cast<int>(rg.prefix);
   const int kvh = h / p.group;
   const int lane = threadIdx.x & 63;
-  const int g = lane >> 4, m = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = lane & 31, half = lane >> 5;
+  const int d = kPad ? p.d : D;
 
-  // Q^T fragments of query wq + m (zeros past the chunk).
-  const int qi = wq + m;
+  // Q^T fragments of query q0 + m (zeros past the chunk and past the head).
+  const int qi = q0 + m;
   const bool q_ok = qi < qlen;
   const float c2 = static_cast<float>(p.scale) * kLog2eF32;
   f32x4_t qf[QK];
   {
     const float *qrow = static_cast<const float *>(p.q) +
-                        (rg.q0 + (q_ok ? qi : wq)) * p.q_st + static_cast<int64_t>(h) * p.q_sh;
+                        (rg.q0 + (q_ok ? qi : q0)) * p.q_st + static_cast<int64_t>(h) * p.q_sh;
 #pragma unroll
     for (int j = 0; j < QK; ++j) {
-      const f32x4_t v = *reinterpret_cast<const f32x4_t *>(qrow + 16 * j + 4 * g);
-      qf[j] = q_ok ? v * c2 : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      const int e = 8 * j + 4 * half;
+      const f32x4_t v = *reinterpret_cast<const f32x4_t *>(qrow + (kPad && e >= d ? 0 : e));
+      qf[j] = q_ok && !(kPad && e >= d) ? v * c2 : f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
   }
-  // Keys this wave needs: up to its last query's position.
-  const int kv_end = prefix + min(qlen, wq + kQW);
-  const int nkb = (kv_end + 15) >> 4;
-  // Lane l's query position for the causal mask (the S^T column).
-  const int qpos = prefix + wq + m;
-  const int first_masked = prefix + wq;  // blocks ending at or before it see no mask
+  // Keys the workgroup needs: up to its last query's position.
+  const int kv_end = prefix + min(qlen, q0 + kBMF);
+  const int ntiles = (kv_end + kBNF - 1) / kBNF;
+  const int qpos = prefix + qi;
+  const int first_masked = prefix + q0;  // tiles ending at or before it see no mask
   const int bs_log2 = p.bs_log2;
   const int bs_mask = (1 << bs_log2) - 1;
-  const int64_t row_elems = static_cast<int64_t>(p.hkv) * D;
-  const float *kc = static_cast<const float *>(p.kc) + static_cast<int64_t>(kvh) * D;
-  const float *vc = static_cast<const float *>(p.vc) + static_cast<int64_t>(kvh) * D;
+  const int64_t row_elems = static_cast<int64_t>(p.hkv) * d;
+  const uint32_t row_bytes = static_cast<uint32_t>(p.hkv) * d * 4;
+  // Lane offsets inside a span: K row m%16 (with 64-bit bases: a tile's rows lie
+  // in two spans), V row 4 half and the lane's dims.
+  const uint32_t k_lane = 16u * half;
+  const uint32_t v_lane = 4u * half * row_bytes + 4u * (kPad && VC * m >= d ? 0 : VC * m);
+  const float *kc = static_cast<const float *>(p.kc) + static_cast<int64_t>(kvh) * d;
+  const float *vc = static_cast<const float *>(p.vc) + static_cast<int64_t>(kvh) * d;
   const int64_t *bt_row = p.bt + static_cast<int64_t>(seq) * p.bt_stride;
 
-  f32x4_t acc[VC];
+  f32x16_t acc[VC];
 #pragma unroll
-  for (int c = 0; c < VC; ++c) acc[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_lane = 0.f;
+  for (int c = 0; c < VC; ++c) acc[c] = f32x16_t{};
+  float m_run = -INFINITY, l_run = 0.f;
 
-  // Block kb's K fragments and V rows into kf / vf; returns whether its
-  // block id is in range.
-  auto load_block = [&](int kb, f32x4_t (&kf)[QK], f32x4_t (&vf)[4][VC / 4]) -> bool {
-    const int key0 = kb * 16;
-    // 16 keys never straddle a cache block (block_size a power of two >= 16).
-    const int64_t raw = bt_row[key0 >> bs_log2];
-    const int64_t blk = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(raw))) |
-                        (static_cast<int64_t>(__builtin_amdgcn_readfirstlane(
-                             static_cast<uint32_t>(static_cast<uint64_t>(raw) >> 32))) << 32);
-    const bool blk_ok = blk >= 0 && blk < p.num_blocks;
-    const int64_t slot0 = (blk_ok ? blk : 0) * p.block_size + (key0 & bs_mask);
-    // K rows: lane l reads key key0 + m (zeros past kv_end or for a bad block).
-    {
-      const bool ok = blk_ok && key0 + m < kv_end;
-      const float *krow = kc + (slot0 + (ok ? m : 0)) * row_elems;
+  // The wave's tiles are wave, wave + kWaves, ...; lane 2u + s holds the block
+  // id of span s (16 keys) of its tile kb + u, kb a multiple of 32 (-1: out of
+  // range; spans past the last key repeat its block).
+  int64_t ids = 0;
+  auto load_ids = [&](int kb) __attribute__((always_inline)) {
+    const int64_t key =
+        static_cast<int64_t>(wave + kWaves * (kb + (lane >> 1))) * kBNF + 16 * (lane & 1);
+    const int64_t id = bt_row[(key < kv_end ? static_cast<int>(key) : kv_end - 1) >> bs_log2];
+    ids = id >= 0 && id < p.num_blocks ? id : -1;
+  };
+  struct TileAt {
+    int64_t slot[2];  // first row of each span in the pool (0 when bad)
+    int last[2];      // its last row that the workgroup needs
+    bool bad[2];
+    uint32_t vbytes[2];  // bytes of its V rows under a buffer resource (0 when bad)
+  };
+  auto tile_at = [&](int k) __attribute__((always_inline)) -> TileAt {
+    TileAt t;
+    const int key0 = (wave + kWaves * k) * kBNF;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int src = 2 * (k & 31) + s;
+      const int64_t id = static_cast<int64_t>(
+          static_cast<uint64_t>(static_cast<uint32_t>(
+              __builtin_amdgcn_readlane(static_cast<int>(ids), src))) |
+          (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(
+               static_cast<int>(ids >> 32), src)))
+           << 32));
+      // A span wholly past the last key re-reads that key's row.
+      const int key = min(key0 + 16 * s, kv_end - 1);
+      t.bad[s] = id < 0;
+      t.slot[s] = ((id < 0 ? 0 : id) << bs_log2) + (id < 0 ? 0 : key & bs_mask);
+      t.last[s] = id < 0 ? 0 : min(15, kv_end - 1 - key);
+      t.vbytes[s] = id < 0 ? 0u : static_cast<uint32_t>(t.last[s]) * row_bytes + 4u * d;
+    }
+    return t;
+  };
+  f32x4_t kf[QK];
+  vec_t vf[16];
+  auto load_k = [&](const TileAt &t) __attribute__((always_inline)) {
+    const int s = m >> 4;
+    const int64_t row = (s ? t.slot[1] : t.slot[0]) + min(m & 15, s ? t.last[1] : t.last[0]);
+    const char *krow = reinterpret_cast<const char *>(kc + row * row_elems) + k_lane;
+#pragma unroll
+    for (int j = 0; j < QK; ++j) {
+      const int e = 8 * j + 4 * half;
+      kf[j] = *reinterpret_cast<const f32x4_t *>(krow + (kPad && e >= d ? -4 * (e - 8 * j) : 32 * j));
+    }
+  };
+  // V rows through a buffer resource per span that ends with its last needed
+  // row: rows past it, and all rows of a bad block, read as zeros.
+  auto load_v = [&](const TileAt &t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<float *>(vc + t.slot[s] * row_elems), 0, t.vbytes[s], 0x00020000);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {  // keys 8 (i / 4) + 4 half + i % 4 of the span
+        const uint32_t row = (8u * (i >> 2) + (i & 3)) * row_bytes;
+        if constexpr (VC == 1)
+          vf[8 * s + i] = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(r, v_lane, row, 0));
+        else if constexpr (VC == 2)
+          vf[8 * s + i] = __builtin_bit_cast(
+              vec_t, __builtin_amdgcn_raw_buffer_load_b64(r, v_lane, row, 0));
+        else
+          vf[8 * s + i] = __builtin_bit_cast(
+              vec_t, __builtin_amdgcn_raw_buffer_load_b128(r, v_lane, row, 0));
+      }
+    }
+  };
+
+  const int nk = ntiles > wave ? (ntiles - wave + kWaves - 1) / kWaves : 0;
+  TileAt cur{};
+  if (nk > 0) {  // uniform per wave
+    load_ids(0);
+    cur = tile_at(0);
+    load_k(cur);
+    load_v(cur);
+  }
+  for (int k = 0; k < nk; ++k) {
+    const int key0 = (wave + kWaves * k) * kBNF;
+    TileAt next = cur;
+    if (k + 1 < nk) {
+      if (((k + 1) & 31) == 0) load_ids(k + 1);
+      next = tile_at(k + 1);
+    }
+    if constexpr (kPad) {  // dims past the head
 #pragma unroll
       for (int j = 0; j < QK; ++j)
-        kf[j] = ok ? *reinterpret_cast<const f32x4_t *>(krow + 16 * j + 4 * g)
-                   : f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (8 * j + 4 * half >= d) kf[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-    // V rows of keys key0 + 4g + i: VC consecutive dims each.
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int k = 4 * g + i;
-      const bool ok = blk_ok && key0 + k < kv_end;
-      const float *vrow = vc + (slot0 + (ok ? k : 0)) * row_elems + VC * m;
-#pragma unroll
-      for (int u = 0; u < VC / 4; ++u)
-        vf[i][u] = ok ? *reinterpret_cast<const f32x4_t *>(vrow + 4 * u)
-                      : f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
-    return blk_ok;
-  };
-  f32x4_t kf[QK], vf[4][VC / 4];
-  bool blk_ok = load_block(0, kf, vf);
-  for (int kb = 0; kb < nkb; ++kb) {
-    const int key0 = kb * 16;
-    f32x4_t nkf[QK], nvf[4][VC / 4];
-    bool nok = false;
-    if (kb + 1 < nkb) nok = load_block(kb + 1, nkf, nvf);
-    // S^T of the block.
-    f32x4_t s = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // S^T of the tile.
+    f32x16_t s = f32x16_t{};
 #pragma unroll
     for (int j = 0; j < QK; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][e], qf[j][e], s, 0, 0, 0);
+      for (int e = 0; e < 4; ++e)
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j][e], qf[j][e], s, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (k + 1 < nk) load_k(next);
+    __builtin_amdgcn_sched_barrier(0);
     // Mask: keys past the query's position, and all keys of a bad block.
-    if (!blk_ok || key0 + 15 > first_masked) {
+    const bool bad = cur.bad[0] || cur.bad[1];
+    if (bad || key0 + kBNF - 1 > first_masked) {  // uniform
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (!blk_ok || key0 + 4 * g + i > qpos) s[i] = -INFINITY;
+      for (int i = 0; i < 16; ++i)
+        if (cur.bad[i >> 3] || key0 + 8 * (i >> 2) + 4 * half + (i & 3) > qpos) s[i] = -INFINITY;
     }
     // Online softmax (base 2). The reference point stays 0 until the query
     // has seen a key, so masked scores give exactly zero probabilities.
-    float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-    mx = swap_max(mx, 16);
-    mx = swap_max(mx, 32);
+    float mx = s[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+    mx = other_half_max(mx);
     const float m_new = fmaxf(m_run, mx);
     const float ref = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = __builtin_amdgcn_exp2f(m_run - ref);  // 0 while m_run is -inf
-    float pr[4];
+    if (__any(m_new > m_run)) {
+      const float alpha = __builtin_amdgcn_exp2f(m_run - ref);  // 0 while m_run is -inf
+      l_run *= alpha;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) pr[i] = __builtin_amdgcn_exp2f(s[i] - ref);
-    l_lane = l_lane * alpha + ((pr[0] + pr[1]) + (pr[2] + pr[3]));
+      for (int c = 0; c < VC; ++c) acc[c] *= alpha;
+    }
     m_run = m_new;
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int c = 0; c < VC; ++c) acc[c] *= alpha;
+    for (int i = 0; i < 16; ++i) {
+      s[i] = __builtin_amdgcn_exp2f(s[i] - ref);
+      sum[i & 3] += s[i];
+    }
+    l_run += (sum[0] + sum[1]) + (sum[2] + sum[3]);
     // O^T += V^T P^T.
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 16; ++i)
 #pragma unroll
-      for (int c = 0; c < VC; ++c)
-        acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][c >> 2][c & 3], pr[i], acc[c], 0, 0, 0);
-    if (kb + 1 < nkb) {
-#pragma unroll
-      for (int j = 0; j < QK; ++j) kf[j] = nkf[j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int u = 0; u < VC / 4; ++u) vf[i][u] = nvf[i][u];
-      blk_ok = nok;
-    }
+      for (int c = 0; c < VC; ++c) {
+        float v;
+        if constexpr (VC == 1) v = vf[i];
+        else v = vf[i][c];
+        acc[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, s[i], acc[c], 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    if (k + 1 < nk) load_v(next);
+    __builtin_amdgcn_sched_barrier(0);
+    cur = next;
   }
 
-  // Row sum across the query's four lanes, then the output rows.
-  float l_tot = l_lane + __shfl_xor(l_lane, 16, 64);
-  l_tot = l_tot + __shfl_xor(l_tot, 32, 64);
-  if (q_ok) {
-    const float inv = 1.f / l_tot;
-    float *orow = static_cast<float *>(p.out) + (rg.q0 + qi) * p.o_st +
-                  static_cast<int64_t>(h) * p.o_sh;
+  // The waves' parts: (O^T, m, l) of each, lane-major, then wave w adds and
+  // stores the registers w, w + kWaves, ... (acc[c][i] = O[query m][dim
+  // VC * (8 (i / 4) + 4 half + i % 4) + c]).
+  constexpr int A = 16 * VC;
+  __shared__ float part[kWaves][A][64];
+  __shared__ float m_s[kWaves][64], l_s[kWaves][64];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      // acc[c][i] = O[query qi][dim VC*(4g + i) + c].
+  for (int c = 0; c < VC; ++c)
 #pragma unroll
-      for (int u = 0; u < VC / 4; ++u) {
-        f32x4_t o;
+    for (int i = 0; i < 16; ++i) part[wave][i * VC + c][lane] = acc[c][i];
+  m_s[wave][lane] = m_run;
+  l_s[wave][lane] = l_run;
+  __syncthreads();
+  float mx = m_s[0][lane];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = acc[4 * u + e][i] * inv;
-        *reinterpret_cast<f32x4_t *>(orow + VC * (4 * g + i) + 4 * u) = o;
-      }
+  for (int w = 1; w < kWaves; ++w) mx = fmaxf(mx, m_s[w][lane]);
+  const float ref = mx == -INFINITY ? 0.f : mx;
+  float f[kWaves], l = 0.f;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    f[w] = __builtin_amdgcn_exp2f(m_s[w][lane] - ref);  // 0 for a wave without keys
+    l += f[w] * (l_s[w][lane] + l_s[w][lane ^ 32]);
+  }
+  if (!q_ok) return;
+  const float inv = 1.f / l;
+  float *orow = static_cast<float *>(p.out) + (rg.q0 + qi) * p.o_st +
+                static_cast<int64_t>(h) * p.o_sh;
+  // Register i of every accumulator: VC consecutive dims, one store.
+#pragma unroll
+  for (int u = 0; u < 16 / kWaves; ++u) {
+    const int i = wave + kWaves * u;
+    const int e = VC * (8 * (i >> 2) + 4 * half + (i & 3));
+    if (kPad && e >= d) continue;
+    vec_t o;
+#pragma unroll
+    for (int c = 0; c < VC; ++c) {
+      float x = 0.f;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) x += f[w] * part[w][i * VC + c][lane];
+      if constexpr (VC == 1) o = x * inv;
+      else o[c] = x * inv;
     }
+    *reinterpret_cast<vec_t *>(orow + e) = o;
   }
 }
 
-template <int D>
+template <int D, int kWaves, bool kPad>
+int launch_waves(const PrefillParams &q, int64_t blocks, hipStream_t stream) {
+  prefill_f32_mfma<D, kWaves, kPad>
+      <<<dim3(static_cast<unsigned>(blocks)), 64 * kWaves, 0, stream>>>(q);
+  return check_launch("mlr_paged_prefill(fp32 mfma)");
+}
+
+template <int D, bool kPad>
 int launch_f32(const PrefillParams &p, int64_t max_query_len, hipStream_t stream) {
   PrefillParams q = p;
   q.n_qtiles = static_cast<int>(ceil_div(max_query_len, kBMF));
@@ -220,8 +372,20 @@ int launch_f32(const PrefillParams &p, int64_t max_query_len, hipStream_t stream
   const int64_t blocks = ceil_div(items, 8) * 8 * q.hq;
   if (blocks > INT32_MAX)
     return set_error(MLR_ERR_UNSUPPORTED, "mlr_paged_prefill: too many work items");
-  prefill_f32_mfma<D><<<dim3(static_cast<unsigned>(blocks)), 256, 0, stream>>>(q);
-  return check_launch("mlr_paged_prefill(fp32 mfma)");
+  const int64_t groups = items * q.hq, cus = current_device_cus();
+  if constexpr (D < 128) {
+    // A grid of fewer workgroups than CUs: eight waves each, half the keys a
+    // wave (at 128 their registers would spill).
+    if (groups <= cus) return launch_waves<D, 8, kPad>(q, blocks, stream);
+  }
+  // Short contexts in a grid that fills the GPU: fewer waves, so that each has
+  // some tiles between its first load and the merge. us per call with 1 / 2 /
+  // 4 waves: 16 x 200 tokens (7 tiles), 28/4 heads of 128 88 / 109 / 160; 4 x 300
+  // (10 tiles) 54 / 53 / 70; 300 after 1000 (41 tiles) x 4 300 / 252 / 240.
+  const int64_t context = p.qsl != nullptr ? p.max_blocks * p.block_size : p.s_ctx;
+  if (groups >= 4 * cus && context <= 8 * kBNF) return launch_waves<D, 1, kPad>(q, blocks, stream);
+  if (groups >= 4 * cus && context <= 16 * kBNF) return launch_waves<D, 2, kPad>(q, blocks, stream);
+  return launch_waves<D, 4, kPad>(q, blocks, stream);
 }
 
 }  // namespace
@@ -235,13 +399,17 @@ bool prefill_f32_eligible(const PrefillParams &p, int dtype) {
                        p.o_sh % 4 == 0;
   // Positions are 32-bit inside the kernel.
   constexpr int64_t k2g = int64_t(1) << 31;
-  return dtype == MLR_DTYPE_F32 && (p.d == 64 || p.d == 128) && aligned && p.bs_log2 >= 4 &&
-         p.max_blocks * p.block_size < k2g && p.scale > 0.0 && p.scale < 1e30;
+  return dtype == MLR_DTYPE_F32 && p.d % 4 == 0 && p.d <= 128 && aligned && p.bs_log2 >= 4 &&
+         p.max_blocks * p.block_size < k2g && 16 * static_cast<int64_t>(p.hkv) * p.d * 4 < k2g &&
+         p.scale > 0.0 && p.scale < 1e30;
 }
 
 int launch_prefill_f32(const PrefillParams &p, int64_t max_query_len, hipStream_t stream) {
-  if (p.d == 64) return launch_f32<64>(p, max_query_len, stream);
-  return launch_f32<128>(p, max_query_len, stream);
+  if (p.d <= 32) return launch_f32<32, true>(p, max_query_len, stream);
+  if (p.d == 64) return launch_f32<64, false>(p, max_query_len, stream);
+  if (p.d < 64) return launch_f32<64, true>(p, max_query_len, stream);
+  if (p.d == 128) return launch_f32<128, false>(p, max_query_len, stream);
+  return launch_f32<128, true>(p, max_query_len, stream);
 }
 
 }  // namespace mlr

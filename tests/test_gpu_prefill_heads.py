@@ -7,6 +7,9 @@ which moves a probability by that much relative; exp2 and the sums add a few
 2^-22, and the probability operand of the matrix cores carries at least 16
 bits (two 8-bit bf16 parts): 2^-16. The weighted mean of V is then off by
 under 2^-13 max |V|, and the result is rounded once (2^-8 bf16, 2^-11 fp16).
+FP32 inputs stay FP32 throughout: errors of independent roundings, about
+sqrt(d) 2^-24 |q||k| in a score, stay under the 1e-5 that the FP32 paths are
+held to.
 """
 
 from __future__ import annotations
@@ -20,22 +23,31 @@ from mini_llm_runtime_amd.kernels import paged_attention as kpa
 
 pytestmark = pytest.mark.gpu
 
-HALF_ULP = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+HALF_ULP = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}
+
+
+def _slack(dtype, vmax):
+    return 1e-5 if dtype is torch.float32 else 2.0 ** -13 * vmax
 
 
 def _attend(q, k, v, prefix):
     group = q.shape[1] // k.shape[1]
     k, v = (t.repeat_interleave(group, dim=1).transpose(0, 1) for t in (k, v))
     scores = torch.matmul(q.transpose(0, 1), k.transpose(1, 2).contiguous()) / math.sqrt(q.shape[2])
-    seen = torch.arange(k.shape[1])[None, :] <= prefix + torch.arange(q.shape[0])[:, None]
+    seen = (torch.arange(k.shape[1], device=q.device)[None, :]
+            <= prefix + torch.arange(q.shape[0], device=q.device)[:, None])
     probs = torch.softmax(scores.masked_fill(~seen, float("-inf")), dim=-1)
     return torch.matmul(probs, v.contiguous()).transpose(0, 1)
 
 
-@pytest.mark.parametrize("dtype", list(HALF_ULP), ids=lambda t: str(t)[6:])
-@pytest.mark.parametrize("d,hq,hkv,bs", [(8, 4, 2, 16), (16, 4, 2, 16), (24, 6, 6, 32),
-                                         (40, 5, 1, 16), (56, 4, 2, 64), (72, 4, 4, 16),
-                                         (80, 10, 2, 16), (96, 8, 2, 16), (120, 3, 1, 32)])
+SHAPES = [(8, 4, 2, 16), (16, 4, 2, 16), (24, 6, 6, 32), (32, 6, 3, 16), (40, 5, 1, 16),
+          (56, 4, 2, 64), (72, 4, 4, 16), (80, 10, 2, 16), (96, 8, 2, 16), (120, 3, 1, 32)]
+# The 16-bit kernels pre-scale q at 64 and 128, another bound than this one.
+CASES = [(t, *s) for t in HALF_ULP for s in SHAPES]
+CASES += [(torch.float32, 64, 14, 2, 16), (torch.float32, 128, 4, 1, 16)]
+
+
+@pytest.mark.parametrize("dtype,d,hq,hkv,bs", CASES, ids=lambda v: str(v).split(".")[-1])
 def test_other_head_sizes_match_float64(device, dtype, d, hq, hkv, bs):
     gen = torch.Generator().manual_seed(d)
     seqs = [(0, 1), (130, 33), (0, 129), (700, 200), (15, 64)]  # (prefix, queries)
@@ -66,7 +78,36 @@ def test_other_head_sizes_match_float64(device, dtype, d, hq, hkv, bs):
             torch.tensor([p + n for p, n in seqs]).to(device), bs)
     got = kpa.paged_attention_prefill_varlen(wide.to(device)[..., :d], *args).double().cpu()
     vmax = float(torch.nan_to_num(vc.float()).abs().max())
-    bound = HALF_ULP[dtype] * 1.01 * want.abs() + 2.0 ** -13 * vmax
+    bound = HALF_ULP[dtype] * 1.01 * want.abs() + _slack(dtype, vmax)
     assert bool(((got - want).abs() <= bound).all()), ((got - want).abs() - bound).max()
     assert torch.equal(
         kpa.paged_attention_prefill_varlen(torch.cat(qs).to(device), *args).double().cpu(), got)
+
+
+@pytest.mark.parametrize("seqs,longest,prefix,hq,hkv,d", [
+    (16, 200, 0, 28, 4, 128),   # one wave per workgroup
+    (10, 330, 60, 28, 4, 128),  # two
+    (16, 180, 30, 14, 2, 64), (4, 300, 900, 14, 2, 64),  # four, items ranked
+    (2, 40, 700, 4, 2, 32)])    # eight
+def test_fp32_workgroup_shapes_match_float64(device, seqs, longest, prefix, hq, hkv, d):
+    """FP32: every wave count of the launcher, ragged chunks and prefixes."""
+    gen = torch.Generator().manual_seed(seqs)
+    n = torch.randint(1, longest + 1, (seqs,), generator=gen).tolist()
+    n[-1] = longest
+    p = torch.randint(0, prefix + 1, (seqs,), generator=gen).tolist()
+    need = [-(-(a + b) // 16) for a, b in zip(n, p)]
+    perm = torch.randperm(sum(need), generator=gen).tolist()
+    kc, vc = (torch.randn(sum(need), 16, hkv, d, generator=gen).to(device) for _ in range(2))
+    q = torch.randn(sum(n), hq, d, generator=gen).to(device)
+    tables = [perm[sum(need[:i]):sum(need[:i + 1])] for i in range(seqs)]
+    bt = torch.tensor([t + [-1] * (max(need) - len(t)) for t in tables]).to(device)
+    qsl = [sum(n[:i]) for i in range(seqs + 1)]
+    ctx = [a + b for a, b in zip(n, p)]
+    got = kpa.paged_attention_prefill_varlen(q, kc, vc, bt, torch.tensor(qsl).to(device),
+                                             torch.tensor(ctx).to(device), 16)
+    for i, t in enumerate(tables):
+        k, v = (c[torch.tensor(t, device=device)].reshape(-1, hkv, d)[:ctx[i]].double()
+                for c in (kc, vc))
+        want = _attend(q[qsl[i]:qsl[i + 1]].double(), k, v, p[i])
+        off = (got[qsl[i]:qsl[i + 1]].double() - want).abs().max().item()
+        assert off <= 1e-5, (i, off)
