@@ -379,6 +379,23 @@ int mlr_qkv_rope_write(const void *qkv, int64_t qkv_stride_t, const void *bias,
                        int64_t num_kv_heads, int64_t head_dim, int dtype, void *stream);
 
 /*
+ * mlr_qkv_rope_write for a whole prompt with separate projections: q, k and v
+ * [num_tokens, heads * head_dim] with their own row strides, bias already
+ * added. The rotated k and the v rows also go to fresh_k and fresh_v
+ * [num_tokens, num_kv_heads, head_dim], every row whatever its slot. Results
+ * are those of Qwen2RotaryEmbedding + apply_rotary_pos_emb + write_slots
+ * (model/qwen2.py:125-209, 427-439) bit for bit.
+ */
+int mlr_qkv_rope_write_prompt(const void *q, int64_t q_stride_t, const void *k,
+                              int64_t k_stride_t, const void *v, int64_t v_stride_t,
+                              const int64_t *positions, const float *inv_freq,
+                              const void *slot_mapping, int index_dtype, void *q_out,
+                              int64_t q_out_stride_t, void *k_cache, void *v_cache,
+                              void *fresh_k, void *fresh_v, int64_t num_slots,
+                              int64_t num_tokens, int64_t num_q_heads, int64_t num_kv_heads,
+                              int64_t head_dim, int dtype, void *stream);
+
+/*
  * Batched weighted row sum in FP32, out[b, d] = sum_n p[b, n] * v[b, n, d],
  * with p [batch, 64], v [batch, 64, 256] and out [batch, 256], all
  * contiguous; v and out 16-byte aligned. Sums run in row order with fma.

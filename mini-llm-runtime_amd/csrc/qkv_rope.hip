@@ -65,6 +65,16 @@ struct alignas(VEC * sizeof(T)) Vec {
   T v[VEC];
 };
 
+// With separate projections (kSep): the k and v sources (qkv is then q's own
+// buffer), and a second destination of the token's k and v rows, row t of
+// two [num_tokens, hkv, d] buffers.
+template <typename T>
+struct Separate {
+  const T *k, *v;
+  int64_t k_st, v_st;
+  T *fresh_k, *fresh_v;
+};
+
 // One wave per token (grid-stride over tokens; a workgroup holds one wave,
 // or four for large launches). A token's row is cut into
 // chunks of VEC elements: a rotary chunk is VEC elements of the first half of
@@ -74,13 +84,13 @@ struct alignas(VEC * sizeof(T)) Vec {
 // pass is issued unconditionally (clamped index), so the loads are in flight
 // together and the cos/sin table is built under their latency; only the
 // stores depend on the chunk kind.
-template <typename T, typename I, int VEC, int K>
+template <typename T, typename I, int VEC, int K, bool kSep>
 __global__ __launch_bounds__(256) void qkv_rope_write_kernel(
     const T *__restrict__ qkv, int64_t qkv_st, const T *__restrict__ bias,
     const int64_t *__restrict__ positions, const float *__restrict__ inv_freq,
     const void *__restrict__ slots, T *__restrict__ q_out, int64_t q_st,
     T *__restrict__ kc, T *__restrict__ vc, int64_t num_slots, int64_t num_tokens, int hq,
-    int hkv, int d) {
+    int hkv, int d, Separate<T> sep) {
 #pragma clang fp contract(off)
   using V = Vec<T, VEC>;
   // Per wave: [d/2] cos then [d/2] sin, dtype-rounded. The wave's own rows:
@@ -111,8 +121,13 @@ __global__ __launch_bounds__(256) void qkv_rope_write_kernel(
         const int c = min(c0 + 64 * k + lane, n_chunks - 1);
         const bool rope = c < n_rope;
         elo[k] = rope ? (c / cph) * d + (c % cph) * VEC : v_base + (c - n_rope) * VEC;
-        lo[k] = *reinterpret_cast<const V *>(row + elo[k]);
-        hi[k] = *reinterpret_cast<const V *>(row + (rope ? elo[k] + half : elo[k]));
+        const T *src = row + elo[k];
+        if constexpr (kSep) {
+          if (elo[k] >= v_base) src = sep.v + t * sep.v_st + (elo[k] - v_base);
+          else if (elo[k] >= hq * d) src = sep.k + t * sep.k_st + (elo[k] - hq * d);
+        }
+        lo[k] = *reinterpret_cast<const V *>(src);
+        hi[k] = *reinterpret_cast<const V *>(rope ? src + half : src);
       }
       if (c0 == 0) {
         // sincosf: one argument reduction for both; its results are those
@@ -160,7 +175,12 @@ __global__ __launch_bounds__(256) void qkv_rope_write_kernel(
             *reinterpret_cast<V *>(o + i0) = olo;
             *reinterpret_cast<V *>(o + i0 + half) = ohi;
           }
-        } else if (write_kv) {
+          if (kSep && h >= hq) {
+            T *f = sep.fresh_k + (t * hkv + (h - hq)) * d;
+            *reinterpret_cast<V *>(f + i0) = olo;
+            *reinterpret_cast<V *>(f + i0 + half) = ohi;
+          }
+        } else if (kSep || write_kv) {
           const int ev = elo[k] - v_base;  // element within the token's v heads
           V ov = lo[k];
           if (bias != nullptr) {
@@ -169,7 +189,8 @@ __global__ __launch_bounds__(256) void qkv_rope_write_kernel(
               ov.v[j] = Elem<T>::from_f32(Elem<T>::to_f32(lo[k].v[j]) +
                                           load_f(bias + v_base + ev + j));
           }
-          *reinterpret_cast<V *>(vc + slot * hkv * d + ev) = ov;
+          if (write_kv) *reinterpret_cast<V *>(vc + slot * hkv * d + ev) = ov;
+          if (kSep) *reinterpret_cast<V *>(sep.fresh_v + t * hkv * d + ev) = ov;
         }
       }
     }
@@ -181,13 +202,13 @@ __global__ __launch_bounds__(256) void qkv_rope_write_kernel(
 // the chunk-to-head map by shifts). The token index is made wave-uniform, so
 // its position and slot are scalar loads, and a pass's row loads are issued
 // before anything waits: the cos/sin table is built while they are in flight.
-template <typename T, typename I, int D, int K>
+template <typename T, typename I, int D, int K, bool kSep>
 __global__ __launch_bounds__(256) void qkv_rope_write_wide_kernel(
     const T *__restrict__ qkv, int64_t qkv_st, const T *__restrict__ bias,
     const int64_t *__restrict__ positions, const float *__restrict__ inv_freq,
     const void *__restrict__ slots, T *__restrict__ q_out, int64_t q_st,
     T *__restrict__ kc, T *__restrict__ vc, int64_t num_slots, int64_t num_tokens, int hq,
-    int hkv) {
+    int hkv, Separate<T> sep) {
 #pragma clang fp contract(off)
   constexpr int kVec = 16 / sizeof(T);
   constexpr int kHalf = D / 2;
@@ -216,8 +237,13 @@ __global__ __launch_bounds__(256) void qkv_rope_write_wide_kernel(
         const int c = min(c0 + 64 * k + lane, n_chunks - 1);
         const bool rope = c < n_rope;
         const int e = rope ? (c / kCph) * D + (c % kCph) * kVec : v_base + (c - n_rope) * kVec;
-        lo[k] = *reinterpret_cast<const V *>(row + e);
-        hi[k] = *reinterpret_cast<const V *>(row + (rope ? e + kHalf : e));
+        const T *src = row + e;
+        if constexpr (kSep) {
+          if (e >= v_base) src = sep.v + t * sep.v_st + (e - v_base);
+          else if (e >= hq * D) src = sep.k + t * sep.k_st + (e - hq * D);
+        }
+        lo[k] = *reinterpret_cast<const V *>(src);
+        hi[k] = *reinterpret_cast<const V *>(rope ? src + kHalf : src);
       }
     };
     load_pass(0);
@@ -262,7 +288,12 @@ __global__ __launch_bounds__(256) void qkv_rope_write_wide_kernel(
             *reinterpret_cast<V *>(o + i0) = olo;
             *reinterpret_cast<V *>(o + i0 + kHalf) = ohi;
           }
-        } else if (write_kv) {
+          if (kSep && h >= hq) {
+            T *f = sep.fresh_k + (t * hkv + (h - hq)) * D;
+            *reinterpret_cast<V *>(f + i0) = olo;
+            *reinterpret_cast<V *>(f + i0 + kHalf) = ohi;
+          }
+        } else if (kSep || write_kv) {
           const int ev = (c - n_rope) * kVec;  // element within the token's v heads
           V ov = lo[k];
           if (bias != nullptr) {
@@ -271,7 +302,8 @@ __global__ __launch_bounds__(256) void qkv_rope_write_wide_kernel(
               ov.v[j] = Elem<T>::from_f32(Elem<T>::to_f32(lo[k].v[j]) +
                                           load_f(bias + v_base + ev + j));
           }
-          *reinterpret_cast<V *>(vc + slot * hkv * D + ev) = ov;
+          if (write_kv) *reinterpret_cast<V *>(vc + slot * hkv * D + ev) = ov;
+          if (kSep) *reinterpret_cast<V *>(sep.fresh_v + t * hkv * D + ev) = ov;
         }
       }
       c0 += 64 * K;
@@ -282,11 +314,11 @@ __global__ __launch_bounds__(256) void qkv_rope_write_wide_kernel(
   }
 }
 
-template <typename T, typename I, int VEC>
+template <typename T, typename I, int VEC, bool kSep>
 void launch_vec(const void *qkv, int64_t qkv_st, const void *bias, const int64_t *positions,
                 const float *inv_freq, const void *slots, void *q_out, int64_t q_st, void *kc,
                 void *vc, int64_t num_slots, int64_t num_tokens, int hq, int hkv, int d,
-                hipStream_t stream) {
+                const Separate<T> &sep, hipStream_t stream) {
   // Four tokens (waves) per workgroup from 1024 tokens on, one below it.
   // Measured at a Qwen2.5-0.5B layer, bf16, in 100-call graphs: 2048
   // tokens 4.39 us against 4.53 us with one wave per workgroup (eight per
@@ -295,33 +327,33 @@ void launch_vec(const void *qkv, int64_t qkv_st, const void *bias, const int64_t
   const int64_t wgs = (num_tokens + waves - 1) / waves;
   const int64_t blocks = wgs < 65536 ? wgs : 65536;
   const size_t lds = static_cast<size_t>(waves) * d * sizeof(float);
-  qkv_rope_write_kernel<T, I, VEC, 4><<<static_cast<unsigned>(blocks), 64 * waves, lds, stream>>>(
+  qkv_rope_write_kernel<T, I, VEC, 4, kSep><<<static_cast<unsigned>(blocks), 64 * waves, lds, stream>>>(
       static_cast<const T *>(qkv), qkv_st, static_cast<const T *>(bias), positions, inv_freq,
       slots, static_cast<T *>(q_out), q_st, static_cast<T *>(kc), static_cast<T *>(vc),
-      num_slots, num_tokens, hq, hkv, d);
+      num_slots, num_tokens, hq, hkv, d, sep);
 }
 
-template <typename T, typename I, int D>
+template <typename T, typename I, int D, bool kSep>
 void launch_wide(const void *qkv, int64_t qkv_st, const void *bias, const int64_t *positions,
                  const float *inv_freq, const void *slots, void *q_out, int64_t q_st, void *kc,
                  void *vc, int64_t num_slots, int64_t num_tokens, int hq, int hkv,
-                 hipStream_t stream) {
+                 const Separate<T> &sep, hipStream_t stream) {
   const int waves = num_tokens >= 1024 ? 4 : 1;
   const int64_t wgs = (num_tokens + waves - 1) / waves;
   const int64_t blocks = wgs < 65536 ? wgs : 65536;
   const size_t lds = static_cast<size_t>(waves) * D * sizeof(float);
-  qkv_rope_write_wide_kernel<T, I, D, 2>
+  qkv_rope_write_wide_kernel<T, I, D, 2, kSep>
       <<<static_cast<unsigned>(blocks), 64 * waves, lds, stream>>>(
           static_cast<const T *>(qkv), qkv_st, static_cast<const T *>(bias), positions,
           inv_freq, slots, static_cast<T *>(q_out), q_st, static_cast<T *>(kc),
-          static_cast<T *>(vc), num_slots, num_tokens, hq, hkv);
+          static_cast<T *>(vc), num_slots, num_tokens, hq, hkv, sep);
 }
 
-template <typename T>
+template <typename T, bool kSep>
 int launch(const void *qkv, int64_t qkv_st, const void *bias, const int64_t *positions,
            const float *inv_freq, const void *slots, int index_dtype, void *q_out,
            int64_t q_st, void *kc, void *vc, int64_t num_slots, int64_t num_tokens, int hq,
-           int hkv, int d, hipStream_t stream) {
+           int hkv, int d, const Separate<T> &sep, hipStream_t stream) {
   // 16-byte chunks at head sizes 64 and 128; otherwise four-element chunks.
   // Either needs half a head to be whole chunks and every row start aligned
   // to the chunk size.
@@ -331,7 +363,11 @@ int launch(const void *qkv, int64_t qkv_st, const void *bias, const int64_t *pos
            (reinterpret_cast<uintptr_t>(qkv) & align) == 0 &&
            (reinterpret_cast<uintptr_t>(q_out) & align) == 0 &&
            (reinterpret_cast<uintptr_t>(kc) & align) == 0 &&
-           (reinterpret_cast<uintptr_t>(vc) & align) == 0;
+           (reinterpret_cast<uintptr_t>(vc) & align) == 0 &&
+           (!kSep || (sep.k_st % vec == 0 && sep.v_st % vec == 0 &&
+                      ((reinterpret_cast<uintptr_t>(sep.k) | reinterpret_cast<uintptr_t>(sep.v) |
+                        reinterpret_cast<uintptr_t>(sep.fresh_k) |
+                        reinterpret_cast<uintptr_t>(sep.fresh_v)) & align) == 0));
   };
   constexpr int kWide = 16 / sizeof(T);
   constexpr int kVec = 4;
@@ -339,11 +375,11 @@ int launch(const void *qkv, int64_t qkv_st, const void *bias, const int64_t *pos
   const bool vec = aligned_to(kVec);
   const bool i32 = index_dtype == MLR_INDEX_I32;
 #define MLR_QKV_WIDE(I, D)                                                                  \
-  launch_wide<T, I, D>(qkv, qkv_st, bias, positions, inv_freq, slots, q_out, q_st, kc, vc, \
-                       num_slots, num_tokens, hq, hkv, stream)
+  launch_wide<T, I, D, kSep>(qkv, qkv_st, bias, positions, inv_freq, slots, q_out, q_st, kc, vc, \
+                       num_slots, num_tokens, hq, hkv, sep, stream)
 #define MLR_QKV_LAUNCH(I, V)                                                                  \
-  launch_vec<T, I, V>(qkv, qkv_st, bias, positions, inv_freq, slots, q_out, q_st, kc, vc,   \
-                      num_slots, num_tokens, hq, hkv, d, stream)
+  launch_vec<T, I, V, kSep>(qkv, qkv_st, bias, positions, inv_freq, slots, q_out, q_st, kc, vc,   \
+                      num_slots, num_tokens, hq, hkv, d, sep, stream)
   if (wide && d == 64) {
     if (i32) MLR_QKV_WIDE(int32_t, 64); else MLR_QKV_WIDE(int64_t, 64);
   } else if (wide) {
@@ -392,18 +428,72 @@ extern "C" int mlr_qkv_rope_write(const void *qkv, int64_t qkv_stride_t, const v
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dtype) {
     case MLR_DTYPE_F32:
-      return launch<float>(qkv, qkv_stride_t, bias, positions, inv_freq, slot_mapping,
+      return launch<float, false>(qkv, qkv_stride_t, bias, positions, inv_freq, slot_mapping,
                            index_dtype, q_out, q_out_stride_t, k_cache, v_cache, num_slots,
-                           num_tokens, hq, hkv, d, s);
+                           num_tokens, hq, hkv, d, {}, s);
     case MLR_DTYPE_F16:
-      return launch<f16_t>(qkv, qkv_stride_t, bias, positions, inv_freq, slot_mapping,
+      return launch<f16_t, false>(qkv, qkv_stride_t, bias, positions, inv_freq, slot_mapping,
                            index_dtype, q_out, q_out_stride_t, k_cache, v_cache, num_slots,
-                           num_tokens, hq, hkv, d, s);
+                           num_tokens, hq, hkv, d, {}, s);
     case MLR_DTYPE_BF16:
-      return launch<bf16_t>(qkv, qkv_stride_t, bias, positions, inv_freq, slot_mapping,
+      return launch<bf16_t, false>(qkv, qkv_stride_t, bias, positions, inv_freq, slot_mapping,
                             index_dtype, q_out, q_out_stride_t, k_cache, v_cache, num_slots,
-                            num_tokens, hq, hkv, d, s);
+                            num_tokens, hq, hkv, d, {}, s);
     default:
       return set_error(MLR_ERR_UNSUPPORTED, "mlr_qkv_rope_write: unsupported dtype %d", dtype);
+  }
+}
+
+// The same step for a whole prompt whose q, k and v come from three
+// projections, with the rotated k and v written to two fresh buffers as well:
+// the prompt then attends over those, and the cache keeps its rows. In place
+// of 25 launches of torch's rotation (positions to FP32, cos, sin, two
+// rotate_half with their copies), the cache write and the copies into a
+// padded pool: one layer over a 1,021-token prompt (896 wide, 14/2 heads,
+// bf16) takes 310 us, 506 before; the launch itself 5.1 us.
+extern "C" int mlr_qkv_rope_write_prompt(
+    const void *q, int64_t q_stride_t, const void *k, int64_t k_stride_t, const void *v,
+    int64_t v_stride_t, const int64_t *positions, const float *inv_freq, const void *slot_mapping,
+    int index_dtype, void *q_out, int64_t q_out_stride_t, void *k_cache, void *v_cache,
+    void *fresh_k, void *fresh_v, int64_t num_slots, int64_t num_tokens, int64_t num_q_heads,
+    int64_t num_kv_heads, int64_t head_dim, int dtype, void *stream) {
+  using namespace mlr;
+  clear_error();
+  MLR_REQUIRE(num_tokens >= 0, "mlr_qkv_rope_write_prompt: num_tokens must be >= 0");
+  MLR_REQUIRE(num_q_heads > 0 && num_kv_heads > 0,
+              "mlr_qkv_rope_write_prompt: head counts must be positive");
+  MLR_REQUIRE(head_dim > 0 && head_dim % 2 == 0 && head_dim <= 1024,
+              "mlr_qkv_rope_write_prompt: head_dim must be even and in (0, 1024]");
+  MLR_REQUIRE((num_q_heads + 2 * num_kv_heads) * head_dim < (int64_t(1) << 30),
+              "mlr_qkv_rope_write_prompt: row too wide");
+  MLR_REQUIRE(q_stride_t >= num_q_heads * head_dim && k_stride_t >= num_kv_heads * head_dim &&
+                  v_stride_t >= num_kv_heads * head_dim &&
+                  q_out_stride_t >= num_q_heads * head_dim,
+              "mlr_qkv_rope_write_prompt: a row stride smaller than its row");
+  MLR_REQUIRE(num_slots >= 0, "mlr_qkv_rope_write_prompt: num_slots must be >= 0");
+  MLR_REQUIRE(index_dtype == MLR_INDEX_I32 || index_dtype == MLR_INDEX_I64,
+              "mlr_qkv_rope_write_prompt: unknown index dtype %d", index_dtype);
+  if (num_tokens == 0) return MLR_OK;
+  MLR_REQUIRE(q && k && v && positions && inv_freq && slot_mapping && q_out && k_cache &&
+                  v_cache && fresh_k && fresh_v,
+              "mlr_qkv_rope_write_prompt: null pointer");
+  const int hq = static_cast<int>(num_q_heads), hkv = static_cast<int>(num_kv_heads);
+  const int d = static_cast<int>(head_dim);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  auto run = [&](auto tag) {
+    using T = decltype(tag);
+    const Separate<T> sep{static_cast<const T *>(k), static_cast<const T *>(v), k_stride_t,
+                          v_stride_t, static_cast<T *>(fresh_k), static_cast<T *>(fresh_v)};
+    return launch<T, true>(q, q_stride_t, nullptr, positions, inv_freq, slot_mapping, index_dtype,
+                           q_out, q_out_stride_t, k_cache, v_cache, num_slots, num_tokens, hq,
+                           hkv, d, sep, s);
+  };
+  switch (dtype) {
+    case MLR_DTYPE_F32: return run(float{});
+    case MLR_DTYPE_F16: return run(f16_t{});
+    case MLR_DTYPE_BF16: return run(bf16_t{});
+    default:
+      return set_error(MLR_ERR_UNSUPPORTED, "mlr_qkv_rope_write_prompt: unsupported dtype %d",
+                       dtype);
   }
 }

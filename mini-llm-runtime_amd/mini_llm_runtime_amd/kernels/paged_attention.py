@@ -463,6 +463,34 @@ def paged_prefill_launch(q: torch.Tensor, k_cache: torch.Tensor,
     return out
 
 
+def paged_prefill_chunk_launch(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                               table: torch.Tensor, prefix_len: int, context_len: int, *,
+                               tile_size: int = _DEFAULT_TILE) -> torch.Tensor:
+    """One sequence's chunk prefill on already-validated operands: q [C, Hq, D]
+    with C = context_len - prefix_len > 0, table int64 covering context_len."""
+    device = _lib.require_hip(q, k_cache, v_cache, table, what="paged chunk prefill")
+    table = table.contiguous()
+    lib = _lib.load()
+    if q.stride(-1) != 1:
+        q = q.contiguous()
+    out = torch.empty_like(q, memory_format=torch.contiguous_format)
+    num_blocks, block_size, num_kv_heads, head_dim = k_cache.shape
+    dcode = _lib.dtype_code(q.dtype, "paged_attention_prefill_chunk_tiled")
+    with torch.cuda.device(device):
+        ws, ws_bytes = _prefill_workspace(lib, device, 1, q.shape[0], context_len, q.shape[1],
+                                          head_dim, dcode)
+        status = lib.mlr_paged_prefill_chunk_split(
+            q.data_ptr(), q.stride(0), q.stride(1),
+            k_cache.data_ptr(), v_cache.data_ptr(),
+            num_blocks, block_size, num_kv_heads, head_dim,
+            table.data_ptr(), table.numel(), prefix_len, context_len,
+            q.shape[1], 1.0 / math.sqrt(head_dim), dcode, tile_size,
+            out.data_ptr(), out.stride(0), out.stride(1),
+            ws.data_ptr() if ws is not None else None, ws_bytes, _lib.stream_handle(device))
+    _lib.check(status, "mlr_paged_prefill_chunk")
+    return out
+
+
 def paged_attention_prefill_chunk_tiled(
     q: torch.Tensor,
     k_cache: torch.Tensor,
@@ -517,26 +545,8 @@ def paged_attention_prefill_chunk_tiled(
         if used is None:
             raise ValueError("block_table contains an out-of-range physical block")
         table = _device_ints(used, device)
-    table = table.contiguous()
-    lib = _lib.load()
-    if q.stride(-1) != 1:
-        q = q.contiguous()
-    out = torch.empty_like(q, memory_format=torch.contiguous_format)
-    num_blocks, _, num_kv_heads, head_dim = k_cache.shape
-    dcode = _lib.dtype_code(q.dtype, "paged_attention_prefill_chunk_tiled")
-    with torch.cuda.device(device):
-        ws, ws_bytes = _prefill_workspace(lib, device, 1, chunk_len, int(context_len),
-                                          q_num_heads, head_dim, dcode)
-        status = lib.mlr_paged_prefill_chunk_split(
-            q.data_ptr(), q.stride(0), q.stride(1),
-            k_cache.data_ptr(), v_cache.data_ptr(),
-            num_blocks, block_size, num_kv_heads, head_dim,
-            table.data_ptr(), table.numel(), int(prefix_len), int(context_len),
-            q_num_heads, 1.0 / math.sqrt(head_dim),
-            dcode, int(tile_size), out.data_ptr(), out.stride(0), out.stride(1),
-            ws.data_ptr() if ws is not None else None, ws_bytes, _lib.stream_handle(device))
-    _lib.check(status, "mlr_paged_prefill_chunk")
-    return out
+    return paged_prefill_chunk_launch(q, k_cache, v_cache, table, int(prefix_len),
+                                      int(context_len), tile_size=int(tile_size))
 
 
 def paged_attention_prefill_varlen(

@@ -114,6 +114,46 @@ def qkv_rope_write(qkv: torch.Tensor, positions: torch.Tensor, inv_freq: torch.T
     return out
 
 
+def qkv_rope_write_prompt(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                          positions: torch.Tensor, inv_freq: torch.Tensor,
+                          kv_cache: PagedKVCache, layer_idx: int, slot_mapping: torch.Tensor,
+                          pool_rows: int) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """A whole prompt's projections q [T, Hq, D], k and v [T, Hkv, D] (unit
+    stride within a row) -> rotated q [T, Hq, D] and the rotated k and v as the
+    first T rows of two new [pool_rows, Hkv, D] buffers (later rows are not
+    written); k and v also go to slot_mapping of the layer's cache, whose shape
+    and dtype they have. positions int64 [T]; slot_mapping int32/int64 [T]."""
+    tokens, hq, d = q.shape
+    hkv = k.shape[1]
+    device = _lib.require_hip(q, k, v, positions, inv_freq, slot_mapping, kv_cache.k_cache,
+                              what="qkv_rope_write_prompt")
+    layer_k, layer_v = kv_cache.get_layer_cache(layer_idx)
+    if not (layer_k.is_contiguous() and layer_v.is_contiguous()):
+        raise ValueError("KV cache layers must be contiguous")
+
+    def rows(t):
+        return t if t.stride(2) == 1 and t.stride(1) == d else t.contiguous()
+
+    q, k, v = rows(q), rows(k), rows(v)
+    positions, slot_mapping = positions.contiguous(), slot_mapping.contiguous()
+    freq = _freq_fp32(inv_freq)
+    out = torch.empty((tokens, hq, d), dtype=q.dtype, device=device)
+    fresh = torch.empty((2, pool_rows, hkv, d), dtype=q.dtype, device=device)
+    if tokens == 0:
+        return out, fresh[0], fresh[1]
+    lib = _lib.load()
+    with torch.cuda.device(device):
+        status = lib.mlr_qkv_rope_write_prompt(
+            q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
+            positions.data_ptr(), freq.data_ptr(), slot_mapping.data_ptr(),
+            _lib.INDEX_CODES[slot_mapping.dtype], out.data_ptr(), hq * d, layer_k.data_ptr(),
+            layer_v.data_ptr(), fresh[0].data_ptr(), fresh[1].data_ptr(),
+            kv_cache.num_blocks * kv_cache.block_size, tokens, hq, hkv, d,
+            _lib.dtype_code(q.dtype, "qkv_rope_write_prompt"), _lib.stream_handle(device))
+    _lib.check(status, "mlr_qkv_rope_write_prompt")
+    return out, fresh[0], fresh[1]
+
+
 def qkv_rope_decode_fusable(qkv_dtype: torch.dtype, kv_cache: PagedKVCache,
                             num_q_heads: int) -> bool:
     """Shapes ``qkv_rope_decode`` covers: bf16 or fp16, head_dim 64 or 128, at

@@ -324,7 +324,7 @@ class TinyQwen2Model(nn.Module):
         return self._run(input_ids, lambda layer, i: lambda h:
                          layer.self_attn.forward_prefill_with_cache(
                              hidden_states=h, position_ids=position_ids, kv_cache=kv_cache,
-                             layer_idx=i, slot_mapping=slot_mapping))
+                             layer_idx=i, slot_mapping=slot_mapping, slots_checked=i > 0))
 
     def forward_decode_with_cache(self, input_ids, position_ids, kv_cache, slot_mapping,
                                   block_table, context_len) -> torch.Tensor:

@@ -21,10 +21,11 @@ the reference's rounding; then the attention kernel:
   the fused step and one varlen prefill.
 - ``forward_prefill_chunk_with_cache`` runs the fused step and the tiled
   chunk prefill (reference :737-767).
-- ``forward_prefill_with_cache`` keeps PyTorch projections and rotation,
-  writes the prompt's rows and attends over the fresh K/V with the chunk
-  kernel at prefix 0, viewing them as a pool of 16-row blocks (the reference
-  uses its dense attention here, :427-439).
+- ``forward_prefill_with_cache`` keeps its three projections; one
+  ``mlr_qkv_rope_write_prompt`` launch rotates them, writes the prompt's rows
+  and lays them out once more, and the chunk kernel attends over those at
+  prefix 0 as a pool of 16-row blocks (the reference uses its dense attention
+  here, :427-439). A cache of another dtype takes PyTorch's rotation.
 - ``forward_decode_with_cache`` is the single-request decode (:441-536), on
   the fused step.
 
@@ -280,7 +281,11 @@ class Qwen2Attention(nn.Module):
     # ------------------------------------------------------------------
     def forward_prefill_with_cache(self, hidden_states: torch.Tensor,
                                    position_ids: torch.Tensor, kv_cache: PagedKVCache,
-                                   layer_idx: int, slot_mapping: torch.Tensor) -> torch.Tensor:
+                                   layer_idx: int, slot_mapping: torch.Tensor, *,
+                                   slots_checked: bool = False) -> torch.Tensor:
+        """slots_checked: this slot_mapping already passed the value checks
+        against this cache (the model's first layer makes them), so they are
+        not repeated; every other check still runs."""
         self._check_hidden(hidden_states, "[1, seq_len, hidden_size]", "prefill with cache")
         self._check_width_and_positions(hidden_states, position_ids)
         if slot_mapping.ndim != 1:
@@ -289,11 +294,65 @@ class Qwen2Attention(nn.Module):
         if slot_mapping.shape[0] != hidden_states.shape[1]:
             raise ValueError("slot_mapping length must match sequence length "
                              f"({hidden_states.shape[1]}), got {slot_mapping.shape[0]}")
-        query, key, value = self._qkv_rope(hidden_states, position_ids)
+        if self._prompt_fusable(hidden_states, position_ids, kv_cache, layer_idx, slot_mapping):
+            if not slots_checked:
+                kv_cache.check_slots(slot_mapping)
+                slots_checked = True
+            query, key, value = self.qkv_proj(hidden_states)
+            if query.dtype == key.dtype == value.dtype == kv_cache.dtype:
+                return self._prompt_attention(query[0], key[0], value[0], position_ids[0],
+                                              kv_cache, layer_idx, slot_mapping)
+            cos, sin = self.rotary_embedding(query, position_ids)
+            query, key = apply_rotary_pos_emb(query, key, cos, sin)
+        else:
+            query, key, value = self._qkv_rope(hidden_states, position_ids)
         kv_cache.write_slots(slot_mapping=slot_mapping, k=key.squeeze(0),
-                             v=value.squeeze(0), layer_idx=layer_idx)
+                             v=value.squeeze(0), layer_idx=layer_idx,
+                             validate=not slots_checked)
         out = self._attend_fresh(query.squeeze(0), key.squeeze(0), value.squeeze(0))
         return kops.apply_linear(self.o_proj, out.reshape(1, -1, self.hidden_size))
+
+    def _prompt_attention(self, query, key, value, positions, kv_cache, layer_idx,
+                          slot_mapping) -> torch.Tensor:
+        """The prompt's projections [T, heads, D] -> the layer's output
+        [1, T, hidden]: rotation and cache write in one launch, then causal
+        attention over the prompt's own rows, a pool of 16-row blocks in
+        order."""
+        seq_len, block = query.shape[0], 16
+        blocks = -(-seq_len // block)
+        query, pool_k, pool_v = kpre.qkv_rope_write_prompt(
+            query, key, value, positions.to(torch.long), self.rotary_embedding.inv_freq,
+            kv_cache, layer_idx, slot_mapping, blocks * block)
+        out = kpa.paged_prefill_chunk_launch(
+            query, pool_k.view(blocks, block, *pool_k.shape[1:]),
+            pool_v.view(blocks, block, *pool_v.shape[1:]),
+            torch.arange(blocks, dtype=torch.long, device=query.device), 0, seq_len)
+        return kops.apply_linear(self.o_proj, out.reshape(1, -1, self.hidden_size))
+
+    def _prompt_fusable(self, hidden_states, position_ids, kv_cache, layer_idx,
+                        slot_mapping) -> bool:
+        """Whether the prompt's rotation and cache write go through
+        mlr_qkv_rope_write_prompt: a HIP cache of the model's shape and dtype,
+        integer positions and slots on its device, and a plain rotary module.
+        Anything else takes the PyTorch rotation and write_slots, with their
+        conversions and errors."""
+        rotary, dtype = self.rotary_embedding, hidden_states.dtype
+        return (hidden_states.is_cuda and hidden_states.shape[1] > 0
+                and dtype in (torch.float32, torch.float16, torch.bfloat16)
+                and kv_cache.dtype == dtype and kv_cache.device == hidden_states.device
+                and kv_cache.k_cache.device == hidden_states.device
+                and self.qkv_proj.q_proj.weight.dtype == dtype
+                and 0 <= layer_idx < kv_cache.num_layers
+                and kv_cache.num_kv_heads == self.num_key_value_heads
+                and kv_cache.head_dim == self.head_dim
+                and position_ids.dtype in (torch.int32, torch.int64)
+                and slot_mapping.dtype in (torch.int32, torch.int64)
+                and position_ids.device == hidden_states.device
+                and slot_mapping.device == hidden_states.device
+                and type(rotary) is Qwen2RotaryEmbedding and not rotary._forward_hooks
+                and not rotary._forward_pre_hooks and "forward" not in rotary.__dict__
+                and not nn.modules.module._has_any_global_hook()
+                and not kops._transformed())
 
     def _attend_fresh(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         """Causal attention of a whole prompt over its own K/V with the chunk
