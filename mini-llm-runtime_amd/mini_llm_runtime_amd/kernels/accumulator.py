@@ -34,7 +34,7 @@ def paged_attention_accumulator_cuda(p: torch.Tensor, v: torch.Tensor) -> torch.
     if p.shape[0] == 0:
         return out
     lib = _lib.load()
-    with torch.cuda.device(p.device):
+    with _lib.on(p.device):
         status = lib.mlr_pa_accumulate(p.data_ptr(), v.data_ptr(), out.data_ptr(), p.shape[0],
                                        _lib.stream_handle(p.device))
     _lib.check(status, "mlr_pa_accumulate")

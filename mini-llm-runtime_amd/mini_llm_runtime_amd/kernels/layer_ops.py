@@ -52,20 +52,19 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     xr = _rows(x, "x")
     weight = weight.contiguous()
     out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    res_out = None
+    rows = xr.shape[0]
+    xs = xr.stride(0) if rows else hidden
+    rp = rs = res_out = ro = None
     if residual is not None:
         rr = _rows(residual, "residual")
+        rp, rs = rr.data_ptr(), rr.stride(0) if rows else hidden
         res_out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    rows = xr.shape[0]
-    lib = _lib.load()
-    with torch.cuda.device(x.device):
-        status = lib.mlr_rms_norm(
-            xr.data_ptr(), xr.stride(0) if rows else hidden,
-            rr.data_ptr() if residual is not None else None,
-            rr.stride(0) if residual is not None and rows else hidden,
-            res_out.data_ptr() if residual is not None else None, hidden,
-            weight.data_ptr(), out.data_ptr(), hidden, rows, hidden, float(eps),
-            _lib.dtype_code(x.dtype, "rms_norm"), _lib.stream_handle(x.device))
+        ro = res_out.data_ptr()
+    device = x.device
+    with _lib.on(device):
+        status = _lib.load().mlr_rms_norm(
+            xr.data_ptr(), xs, rp, rs or hidden, ro, hidden, weight.data_ptr(), out.data_ptr(),
+            hidden, rows, hidden, eps, _lib.DTYPE_CODES[x.dtype], _lib.stream_handle(device))
     _lib.check(status, "mlr_rms_norm")
     return out if residual is None else (out, res_out)
 
@@ -82,7 +81,7 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     out = torch.empty(*gate_up.shape[:-1], inter, dtype=gate_up.dtype, device=gate_up.device)
     rows = g.shape[0]
     lib = _lib.load()
-    with torch.cuda.device(gate_up.device):
+    with _lib.on(gate_up.device):
         status = lib.mlr_silu_mul(g.data_ptr(), g.stride(0) if rows else 2 * inter,
                                   out.data_ptr(), inter, rows, inter,
                                   _lib.dtype_code(gate_up.dtype, "silu_mul"),
@@ -164,7 +163,7 @@ def _rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
     code = _lib.DTYPE_CODES[dtype]
     nbytes = lib.mlr_rows_linear_workspace_size(rows, n_out, k, gated, code)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
-    with torch.cuda.device(device):
+    with _lib.on(device):
         status = lib.mlr_rows_linear(
             xp, stride, wp, bias.data_ptr() if bias is not None else None, out.data_ptr(), n_out,
             rows, n_out, k, gated, code, ws.data_ptr() if ws is not None else None, nbytes,

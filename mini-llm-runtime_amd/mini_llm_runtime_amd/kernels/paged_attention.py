@@ -69,7 +69,7 @@ def _device_ints(values: array, device: torch.device) -> torch.Tensor:
     if n > _STAGE_MAX or (n and max(values) > 0x7FFFFFFF):
         return torch.tensor(values, dtype=torch.long, device=device)
     out = torch.empty(n, dtype=torch.long, device=device)
-    with torch.cuda.device(device):
+    with _lib.on(device):
         status = _lib.load().mlr_stage_i64(values.buffer_info()[0], n, out.data_ptr(),
                                            _lib.stream_handle(device))
     _lib.check(status, "mlr_stage_i64")
@@ -120,7 +120,7 @@ def decode_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     and asks for an eager call of the same size first, or an explicit
     workspace.
     """
-    stream = torch.cuda.current_stream(device).cuda_stream
+    stream = _lib.stream_handle(device)
     key = (device.index, stream)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
@@ -145,7 +145,7 @@ def check_workspace(workspace: torch.Tensor) -> None:
     (check_decode_workspaces synchronises the device for that)."""
     lib = _lib.load()
     device = workspace.device
-    with torch.cuda.device(device):
+    with _lib.on(device):
         status = lib.mlr_paged_decode_workspace_check(
             workspace.data_ptr(), workspace.numel(), _lib.stream_handle(device))
     if status == _lib.MLR_ERR_MERGE:
@@ -236,7 +236,7 @@ def paged_decode_launch(q: torch.Tensor, k_cache: torch.Tensor,
               int(tokens_per_split), workspace.data_ptr(), workspace.numel())
     tail = (out.data_ptr(), out.stride(0), out.stride(1), stream)
     if new_k is None:
-        with torch.cuda.device(device):
+        with _lib.on(device):
             status = lib.mlr_paged_decode(*common, *tail)
         _lib.check(status, "mlr_paged_decode")
         return out
@@ -245,7 +245,7 @@ def paged_decode_launch(q: torch.Tensor, k_cache: torch.Tensor,
     if new_k.stride(-1) != 1 or new_k.stride() != new_v.stride():
         new_k, new_v = new_k.contiguous(), new_v.contiguous()
     slot_mapping = slot_mapping.to(torch.long).contiguous()
-    with torch.cuda.device(device):
+    with _lib.on(device):
         status = lib.mlr_paged_decode_append(
             *common, new_k.data_ptr(), new_v.data_ptr(), new_k.stride(0),
             new_k.stride(1), slot_mapping.data_ptr(), *tail)
@@ -446,7 +446,7 @@ def paged_prefill_launch(q: torch.Tensor, k_cache: torch.Tensor,
     if total_q == 0:
         return out
     dcode = _lib.dtype_code(q.dtype, "paged prefill")
-    with torch.cuda.device(device):
+    with _lib.on(device):
         ws, ws_bytes = _prefill_workspace(
             lib, device, context_lens.shape[0], int(max_query_len),
             block_tables.shape[1] * block_size, num_q_heads, head_dim, dcode)
@@ -476,7 +476,7 @@ def paged_prefill_chunk_launch(q: torch.Tensor, k_cache: torch.Tensor, v_cache: 
     out = torch.empty_like(q, memory_format=torch.contiguous_format)
     num_blocks, block_size, num_kv_heads, head_dim = k_cache.shape
     dcode = _lib.dtype_code(q.dtype, "paged_attention_prefill_chunk_tiled")
-    with torch.cuda.device(device):
+    with _lib.on(device):
         ws, ws_bytes = _prefill_workspace(lib, device, 1, q.shape[0], context_len, q.shape[1],
                                           head_dim, dcode)
         status = lib.mlr_paged_prefill_chunk_split(
@@ -611,7 +611,7 @@ def paged_kv_read_floor(k_cache: torch.Tensor, v_cache: torch.Tensor,
     n = int(lib.mlr_paged_kv_read_floor_outputs(batch, width, block_size, tokens_per_item))
     if out is None:
         out = torch.empty(max(n, 1), dtype=torch.int32, device=device)
-    with torch.cuda.device(device):
+    with _lib.on(device):
         status = lib.mlr_paged_kv_read_floor(
             k_cache.data_ptr(), v_cache.data_ptr(), num_blocks, block_size, row_bytes,
             block_tables.data_ptr(), block_tables.stride(0), width, context_lens.data_ptr(),

@@ -102,7 +102,7 @@ def qkv_rope_write(qkv: torch.Tensor, positions: torch.Tensor, inv_freq: torch.T
     freq = _freq_fp32(inv_freq)
     bias_c = bias.contiguous() if bias is not None else None
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _lib.on(device):
         status = lib.mlr_qkv_rope_write(
             qkv.data_ptr(), qkv.stride(0), bias_c.data_ptr() if bias_c is not None else None,
             positions.data_ptr(), freq.data_ptr(), slot_mapping.data_ptr(),
@@ -142,7 +142,7 @@ def qkv_rope_write_prompt(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if tokens == 0:
         return out, fresh[0], fresh[1]
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _lib.on(device):
         status = lib.mlr_qkv_rope_write_prompt(
             q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
             positions.data_ptr(), freq.data_ptr(), slot_mapping.data_ptr(),
@@ -230,7 +230,7 @@ def qkv_rope_decode(qkv: torch.Tensor, inv_freq: torch.Tensor, kv_cache: PagedKV
     elif workspace.numel() < ws_bytes:
         raise ValueError(f"decode workspace of {workspace.numel()} bytes is smaller than "
                          f"the {ws_bytes} bytes required")
-    with torch.cuda.device(device):
+    with _lib.on(device):
         status = lib.mlr_paged_decode_qkv(
             qkv.data_ptr(), qkv.stride(0), freq.data_ptr(), layer_k.data_ptr(), layer_v.data_ptr(), kv_cache.num_blocks,
             kv_cache.block_size, hkv, d, block_tables.data_ptr(), block_tables.stride(0),

@@ -63,7 +63,7 @@ def step_flags(block_size: int, num_blocks: int, *, tables: torch.Tensor | None 
     def ptr(t):
         return None if t is None else t.data_ptr()
 
-    with torch.cuda.device(device):
+    with _lib.on(device):
         status = lib.mlr_check_step(
             ptr(tables), stride, width, ptr(ctx), reqs, ptr(qsl), ptr(positions), ptr(slots),
             tokens, ptr(decoding), block_size, num_blocks, max_query_len, detail,

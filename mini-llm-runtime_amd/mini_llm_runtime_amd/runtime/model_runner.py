@@ -185,7 +185,7 @@ def _build_on_device(entries, block_size: int, dev: torch.device) -> ModelBatch:
     ctx = out[2 * num_tokens + num_reqs + 1:]
     tables = buf[num_tokens + 2 * num_reqs:].view(num_reqs, width)
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         status = lib.mlr_build_step_metadata(
             buf[num_tokens:].data_ptr(), tables.data_ptr(), width, width, num_reqs,
             num_tokens, block_size, positions.data_ptr(), slots.data_ptr(), qsl.data_ptr(),

@@ -219,7 +219,7 @@ class PagedKVCache:
         layer_v = self.v_cache[layer_idx]
         if not (layer_k.is_contiguous() and layer_v.is_contiguous()):
             raise ValueError("KV cache layers must be contiguous")
-        with torch.cuda.device(device):
+        with _lib.on(device):
             status = lib.mlr_kv_write(
                 k.data_ptr(), v.data_ptr(), _lib.dtype_code(k.dtype, "write_slots"),
                 k.shape[0], k.stride(0), k.stride(1), k.stride(2),
