@@ -531,6 +531,42 @@ class Qwen2Attention(nn.Module):
         return kops.apply_linear(self.o_proj, out.reshape(-1, self.hidden_size))
 
     # ------------------------------------------------------------------
+    # A step's prefills and decodes together (no counterpart in the reference)
+    # ------------------------------------------------------------------
+    def forward_mixed_with_cache(self, hidden_states: torch.Tensor, position_ids: torch.Tensor,
+                                 kv_cache: PagedKVCache, layer_idx: int, num_prefill: int,
+                                 prefill: tuple, decode: tuple) -> torch.Tensor:
+        """hidden_states [T, hidden]: num_prefill packed prefill tokens, then
+        one token per decode request. One projection and one o_proj for all of
+        them; each kind attends as in forward_prefill_packed_with_cache and
+        forward_decode_batch_with_cache, the prefill first.
+
+        prefill: (slot_mapping, block_tables, query_start_loc, context_lens,
+        max_query_len); decode: (slot_mapping, block_tables, context_lens). The
+        caller has run both forwards' checks (the runner does)."""
+        weight, bias = self._qkv_weights()
+        qkv = torch.nn.functional.linear(hidden_states, weight, bias)
+        k_layer, v_layer = kv_cache.get_layer_cache(layer_idx)
+        heads, freq = self.num_attention_heads, self.rotary_embedding.inv_freq
+        out = torch.empty((hidden_states.shape[0], heads, self.head_dim), dtype=qkv.dtype,
+                          device=qkv.device)
+        slots, tables, query_start_loc, context_lens, max_query_len = prefill
+        query = kpre.qkv_rope_write(qkv[:num_prefill], position_ids[:num_prefill], freq, kv_cache,
+                                    layer_idx, slots, heads)
+        kpa.paged_prefill_launch(query, k_layer, v_layer, tables, query_start_loc, context_lens,
+                                 max_query_len, out=out[:num_prefill])
+        slots, tables, context_lens = decode
+        if kpre.qkv_rope_decode_fusable(qkv.dtype, kv_cache, heads):
+            kpre.qkv_rope_decode(qkv[num_prefill:], freq, kv_cache, layer_idx, slots, tables,
+                                 context_lens, heads, out=out[num_prefill:])
+        else:
+            query = kpre.qkv_rope_write(qkv[num_prefill:], position_ids[num_prefill:], freq,
+                                        kv_cache, layer_idx, slots, heads)
+            kpa.paged_decode_launch(query, k_layer, v_layer, tables, context_lens,
+                                    out=out[num_prefill:])
+        return kops.apply_linear(self.o_proj, out.reshape(-1, self.hidden_size))
+
+    # ------------------------------------------------------------------
     # Chunk prefill (reference :624-767)
     # ------------------------------------------------------------------
     def forward_prefill_chunk_with_cache(self, hidden_states: torch.Tensor,

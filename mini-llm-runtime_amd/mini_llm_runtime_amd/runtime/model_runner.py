@@ -6,8 +6,9 @@ decodes) into flat token/position arrays with ``query_start_loc`` offsets and
 the paged-attention metadata: right-padded (-1) block tables, context lengths
 and the slot of every scheduled token, slot = table[pos // B] * B + pos % B.
 
-``execute_model_batch`` runs the model on those metadata. The reference runs
-one ``forward_prefill_with_cache`` per prefill request; here every prefill of
+``execute_model_batch`` runs the model on those metadata. A step with both
+prefills and decodes runs them in one pass over the layers
+(``forward_mixed_with_cache``). The reference runs one ``forward_prefill_with_cache`` per prefill request; here every prefill of
 the step goes through one packed forward (``forward_prefill_packed_with_cache``:
 one varlen prefill launch per layer), and the decodes through one batched
 decode forward, as in the reference. Logits come back in packed token order
@@ -376,6 +377,46 @@ def _step_metadata_flags(batch: ModelBatch, bs: int, width: int,
                         (bad_slot & dec).any(), (repeat & repeat_dec).any()])
 
 
+def _takes_mixed_steps(model, device: torch.device) -> bool:
+    from ..model.qwen2 import TinyQwen2ForCausalLM
+
+    return (device.type == "cuda" and type(model) is TinyQwen2ForCausalLM
+            and "logits" not in model.__dict__ and hasattr(model.model, "takes_mixed_steps")
+            and model.model.takes_mixed_steps())
+
+
+def _execute_mixed(model, batch: ModelBatch, kv_cache: PagedKVCache, qsl: list[int],
+                   prefill: list[int], decode: list[int], logits: torch.Tensor) -> torch.Tensor:
+    """A checked step of prefills and decodes in one pass over the layers, the
+    prefill tokens first; fills and returns `logits`."""
+    model.model._check_cache(kv_cache)
+    device, split = logits.device, len(prefill)
+    lens = [qsl[i + 1] - qsl[i] for i in prefill]
+    count = sum(lens)
+    if prefill[-1] == split - 1:  # build_model_batch's order: rows as they are
+        tables, ctx = batch.block_tables, batch.context_lens
+        hidden = model.model.forward_mixed_with_cache(
+            batch.input_token_ids, batch.positions, kv_cache, count,
+            (batch.slot_mapping[:count], tables[:split], batch.query_start_loc[:split + 1],
+             ctx[:split], max(lens)),
+            (batch.slot_mapping[count:], tables[split:], ctx[split:]))
+        return model.logits(hidden, logits)
+    rows = _upload([t for i in prefill + decode for t in range(qsl[i], qsl[i + 1])], device)
+    order = _upload(prefill + decode, device)
+    offsets = [0]
+    for n in lens:
+        offsets.append(offsets[-1] + n)
+    slots = batch.slot_mapping.index_select(0, rows)
+    tables = batch.block_tables.index_select(0, order)
+    ctx = batch.context_lens.index_select(0, order)
+    hidden = model.model.forward_mixed_with_cache(
+        batch.input_token_ids.index_select(0, rows), batch.positions.index_select(0, rows),
+        kv_cache, count,
+        (slots[:count], tables[:split], _upload(offsets, device), ctx[:split], max(lens)),
+        (slots[count:], tables[split:], ctx[split:]))
+    return logits.index_copy_(0, rows, model.logits(hidden))
+
+
 def execute_model_batch(model, batch: ModelBatch, kv_cache: PagedKVCache,
                         decode_graphs=None, prefill_graphs=None) -> torch.Tensor:
     """[num_packed_tokens, vocab_size] logits in packed token order.
@@ -392,6 +433,10 @@ def execute_model_batch(model, batch: ModelBatch, kv_cache: PagedKVCache,
     logits = model.lm_head.weight.new_empty((num_tokens, model.lm_head.out_features))
     prefill = [i for i, ph in enumerate(batch.request_phases) if ph is RequestStatus.PREFILLING]
     decode = [i for i, ph in enumerate(batch.request_phases) if ph is RequestStatus.DECODING]
+
+    if (prefill and decode and decode_graphs is None and prefill_graphs is None
+            and _takes_mixed_steps(model, device)):
+        return _execute_mixed(model, batch, kv_cache, qsl, prefill, decode, logits)
 
     packed = step = None
     if prefill:

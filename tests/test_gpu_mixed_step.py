@@ -1,0 +1,99 @@
+"""A step's prefills and decodes in one pass over the layers against the two
+forwards run one after the other.
+
+The two differ only in the row count of the library GEMMs (which may pick
+another kernel, i.e. another order of FP32 sums): FP32 logits within 1e-4
+relative, 16-bit logits within the rounding that a layer's output carries on
+(relative 2-norm 2e-2). Cache rows outside the step's slots keep their bits."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from mini_llm_runtime_amd.model.qwen2 import TinyQwen2Config, TinyQwen2ForCausalLM
+from mini_llm_runtime_amd.runtime import model_runner
+from mini_llm_runtime_amd.runtime.paged_kv_cache import PagedKVCache
+from mini_llm_runtime_amd.runtime.request import RequestStatus
+
+pytestmark = pytest.mark.gpu
+P, D = RequestStatus.PREFILLING, RequestStatus.DECODING
+
+
+def _setup(config, dtype, device, order, block_size):
+    """order: (phase, context, tokens) per request."""
+    torch.manual_seed(1)
+    with device:
+        model = TinyQwen2ForCausalLM(config).to(dtype).eval()
+    gen = torch.Generator().manual_seed(len(order))
+    need = [-(-n // block_size) for _, n, _ in order]
+    perm = torch.randperm(sum(need) + 2, generator=gen).tolist()
+    caches = []
+    for _ in range(2):
+        cache = PagedKVCache(config.num_hidden_layers, sum(need) + 2, block_size,
+                             config.num_key_value_heads, config.head_dim, dtype=dtype,
+                             device=device)
+        for c in (cache.k_cache, cache.v_cache):
+            c.copy_(torch.randn(c.shape, generator=torch.Generator().manual_seed(5)).to(dtype))
+        caches.append(cache)
+    tables, pos, slots, qsl = [], [], [], [0]
+    for i, (_, n, count) in enumerate(order):
+        tables.append(perm[sum(need[:i]):sum(need[:i + 1])])
+        pos += range(n - count, n)
+        slots += [tables[-1][p // block_size] * block_size + p % block_size
+                  for p in range(n - count, n)]
+        qsl.append(qsl[-1] + count)
+    t = lambda v: torch.tensor(v, dtype=torch.long, device=device)  # noqa: E731
+    width = max(need)
+    batch = model_runner.ModelBatch(
+        [f"r{i}" for i in range(len(order))],
+        torch.randint(0, config.vocab_size, (qsl[-1],), generator=gen).to(device), t(pos), t(qsl),
+        [phase for phase, _, _ in order], t([n for _, n, _ in order]),
+        t([x + [-1] * (width - len(x)) for x in tables]), t(slots))
+    return model, batch, caches
+
+
+SMALL = TinyQwen2Config()
+WIDE = TinyQwen2Config(vocab_size=515, hidden_size=896, intermediate_size=300, num_hidden_layers=2,
+                       num_attention_heads=14, num_key_value_heads=2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16],
+                         ids=lambda t: str(t)[6:])
+@pytest.mark.parametrize("config,block_size,order", [
+    (SMALL, 16, [(P, 5, 5), (D, 9, 1)]),
+    (SMALL, 4, [(D, 1, 1), (P, 30, 30), (D, 33, 1), (P, 20, 7)]),
+    (WIDE, 16, [(P, 300, 300), (P, 90, 40), (D, 700, 1), (D, 16, 1), (D, 17, 1)]),
+    (WIDE, 16, [(P, 300, 300), (D, 200, 1), (P, 1, 1), (D, 33, 1)])])
+def test_mixed_step_equals_the_two_forwards(device, monkeypatch, dtype, config, block_size, order):
+    model, batch, caches = _setup(config, dtype, device, order, block_size)
+    assert model_runner._takes_mixed_steps(model, device)
+    with torch.no_grad():
+        got = model_runner.execute_model_batch(model, batch, caches[0])
+        monkeypatch.setattr(model_runner, "_takes_mixed_steps", lambda *a: False)
+        want = model_runner.execute_model_batch(model, batch, caches[1])
+    tol = 1e-4 if dtype is torch.float32 else 2e-2
+    assert ((got - want).double().norm() / want.double().norm()).item() <= tol
+    slots = batch.slot_mapping.tolist()
+    kept = torch.ones(caches[0].num_blocks * block_size, dtype=torch.bool)
+    kept[slots] = False
+    for a, b in ((caches[0].k_cache, caches[1].k_cache), (caches[0].v_cache, caches[1].v_cache)):
+        a, b = (c.flatten(1, 2).cpu().double() for c in (a, b))
+        assert torch.equal(a[:, kept], b[:, kept])
+        assert ((a - b).norm() / b[:, slots].norm()).item() <= tol
+
+
+def test_steps_that_keep_the_two_forwards(device):
+    model, batch, caches = _setup(SMALL, torch.float32, device, [(P, 5, 5), (D, 9, 1)], 16)
+    seen = []
+    handle = model.model.layers[1].mlp.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+    with torch.no_grad():
+        model_runner.execute_model_batch(model, batch, caches[0])
+        assert len(seen) == 2
+        handle.remove()
+        layer = model.model.layers[0]
+        layer.self_attn.forward_decode_batch_with_cache = (
+            lambda *a, **k: seen.append(1) or type(layer.self_attn).forward_decode_batch_with_cache(
+                layer.self_attn, *a, **k))
+        model_runner.execute_model_batch(model, batch, caches[1])
+        assert seen[2:] == [1]
