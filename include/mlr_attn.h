@@ -478,6 +478,16 @@ int mlr_check_step(const int64_t *block_tables, int64_t block_table_stride, int6
                    const int64_t *slot_mapping, int64_t num_tokens, const uint8_t *decoding,
                    int64_t block_size, int64_t num_blocks, int64_t max_query_len, int detail,
                    int64_t *out, int64_t out_len, void *stream);
+/* The same, with `out` in HOST memory that the device can write (pinned), and
+ * a wait for `stream`: the words are there when the call returns. Refused
+ * under graph capture. */
+int mlr_check_step_wait(const int64_t *block_tables, int64_t block_table_stride,
+                        int64_t max_blocks, const int64_t *context_lens, int64_t num_reqs,
+                        const int64_t *query_start_loc, const int64_t *positions,
+                        const int64_t *slot_mapping, int64_t num_tokens,
+                        const uint8_t *decoding, int64_t block_size, int64_t num_blocks,
+                        int64_t max_query_len, int detail, int64_t *out, int64_t out_len,
+                        void *stream);
 
 /*
  * RMSNorm of `rows` rows of `hidden` elements, after a residual add when

@@ -207,3 +207,27 @@ extern "C" int mlr_check_step(const int64_t *block_tables, int64_t block_table_s
   check_step<<<static_cast<unsigned>(groups), kThreads, 0, static_cast<hipStream_t>(stream)>>>(p);
   return check_launch("mlr_check_step");
 }
+
+extern "C" int mlr_check_step_wait(const int64_t *block_tables, int64_t block_table_stride,
+                                   int64_t max_blocks, const int64_t *context_lens,
+                                   int64_t num_reqs, const int64_t *query_start_loc,
+                                   const int64_t *positions, const int64_t *slot_mapping,
+                                   int64_t num_tokens, const uint8_t *decoding,
+                                   int64_t block_size, int64_t num_blocks,
+                                   int64_t max_query_len, int detail, int64_t *out,
+                                   int64_t out_len, void *stream) {
+  clear_error();
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone)
+    return set_error(MLR_ERR_INVALID, "mlr_check_step_wait: the stream is being captured");
+  const int rc = mlr_check_step(block_tables, block_table_stride, max_blocks, context_lens,
+                                num_reqs, query_start_loc, positions, slot_mapping, num_tokens,
+                                decoding, block_size, num_blocks, max_query_len, detail, out,
+                                out_len, stream);
+  if (rc != MLR_OK) return rc;
+  const hipError_t err = hipStreamSynchronize(s);
+  if (err != hipSuccess)
+    return set_error(MLR_ERR_HIP, "mlr_check_step_wait: %s", hipGetErrorString(err));
+  return MLR_OK;
+}

@@ -128,6 +128,11 @@ _PROTOTYPES = {
         [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr,
          _c_i64, _c_i64, _c_i64, _c_int, _c_ptr, _c_i64, _c_ptr],
     ),
+    "mlr_check_step_wait": (
+        _c_int,
+        [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr,
+         _c_i64, _c_i64, _c_i64, _c_int, _c_ptr, _c_i64, _c_ptr],
+    ),
     "mlr_rms_norm": (
         _c_int,
         [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_i64,

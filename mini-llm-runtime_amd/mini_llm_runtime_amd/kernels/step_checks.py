@@ -58,17 +58,21 @@ def step_flags(block_size: int, num_blocks: int, *, tables: torch.Tensor | None 
             stride = width
     ctx, qsl, positions, slots, decoding = (
         None if t is None else t.contiguous() for t in (ctx, qsl, positions, slots, decoding))
-    out = torch.empty(groups + (3 * reqs + 1 if detail else 0), dtype=torch.long, device=device)
+    # The kernel writes its words straight to pinned host memory, read after
+    # the wait that the checks cost anyway: no copy behind the kernel. The
+    # buffer is this call's own until the wait has ended.
+    out = torch.empty(groups + (3 * reqs + 1 if detail else 0), dtype=torch.long,
+                      pin_memory=True)
 
     def ptr(t):
         return None if t is None else t.data_ptr()
 
     with _lib.on(device):
-        status = lib.mlr_check_step(
+        status = lib.mlr_check_step_wait(
             ptr(tables), stride, width, ptr(ctx), reqs, ptr(qsl), ptr(positions), ptr(slots),
             tokens, ptr(decoding), block_size, num_blocks, max_query_len, detail,
             out.data_ptr(), out.numel(), _lib.stream_handle(device))
-    _lib.check(status, "mlr_check_step")
+    _lib.check(status, "mlr_check_step_wait")
     host = out.tolist()
     flags = 0
     for word in host[:groups]:
