@@ -543,6 +543,29 @@ int mlr_rows_linear(const void *x, int64_t x_stride, const void *weight, const v
                     int gated, int dtype, void *workspace, size_t workspace_bytes,
                     void *stream);
 size_t mlr_rows_linear_workspace_size(int64_t rows, int64_t n, int64_t k, int gated, int dtype);
+/* With out == NULL and a workspace size above 0 the call stops at the FP32 sums
+ * [splits, rows, n] in the workspace (splits = size / (4 rows n)), which
+ * mlr_rms_norm_sums reads: mlr_rms_norm of residual + T(sum of the parts) with
+ * its residual_out, both [rows, hidden] contiguous. Equal to mlr_rows_linear
+ * then mlr_rms_norm bit for bit. */
+int mlr_rms_norm_sums(const float *sums, int64_t splits, const void *residual,
+                      int64_t residual_stride, void *residual_out, const void *weight,
+                      void *out, int64_t rows, int64_t hidden, double eps, int dtype,
+                      void *stream);
+/*
+ * mlr_rms_norm of x with `residual`, then the gated mlr_rows_linear of the
+ * normalised rows, in one launch and bit for bit: out [rows, n] for weight
+ * [2 n, k], and residual_out [rows, k] contiguous, a buffer of its own. bf16
+ * and fp16, rows <= 32, k a multiple of 8 up to 1024 (1008 past 16 rows), 16-byte aligned
+ * operands and row starts.
+ *
+ * Replaces the post-attention half of Qwen2DecoderLayer up to the activation
+ * (model/qwen2.py:768-792, 794-940) for a decode step's few rows.
+ */
+int mlr_norm_rows_linear(const void *x, int64_t x_stride, const void *residual,
+                         int64_t residual_stride, void *residual_out, const void *norm_weight,
+                         double eps, const void *weight, void *out, int64_t out_stride,
+                         int64_t rows, int64_t n, int64_t k, int dtype, void *stream);
 
 /*
  * Diagnostics. No counterpart in the reference: a read-only pass that

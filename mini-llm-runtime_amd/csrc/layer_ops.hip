@@ -187,6 +187,71 @@ __global__ __launch_bounds__(256) void rms_norm_rows_kernel(
   }
 }
 
+// The same norm after residual + x where x is a product still in `splits` FP32
+// parts [splits, rows, hidden] (mlr_rows_linear without out): the parts are
+// added in split order and rounded as that product's own reduction rounds
+// them, so a decode step saves the reduction's launch. One row per workgroup's
+// wave; latency, as above.
+template <typename T, int N, int K>
+__global__ __launch_bounds__(256) void rms_norm_sums_kernel(
+    const float *__restrict__ sums, int splits, const T *__restrict__ residual,
+    int64_t res_stride, T *__restrict__ residual_out, const T *__restrict__ weight,
+    T *__restrict__ out, int64_t rows, int hidden, float factor, float eps) {
+  using E = Elem<T>;
+  using C = Chunk<T, N>;
+  const int lane = threadIdx.x & 63;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;  // whole waves
+  const int chunks = hidden / N;
+  C r[K], w[K];
+  float x[K][N];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int c = min(lane + kWave * k, chunks - 1);
+    r[k] = reinterpret_cast<const C *>(residual + row * res_stride)[c];
+    w[k] = reinterpret_cast<const C *>(weight)[c];
+#pragma unroll
+    for (int e = 0; e < N; ++e) x[k][e] = sums[row * hidden + c * N + e];
+  }
+  for (int s = 1; s < splits; ++s) {
+    const float *part = sums + (s * rows + row) * hidden;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = min(lane + kWave * k, chunks - 1);
+#pragma unroll
+      for (int e = 0; e < N; ++e) x[k][e] += part[c * N + e];
+    }
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    if (lane + kWave * k < chunks) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        r[k].v[e] = E::from_f32(E::to_f32(r[k].v[e]) + E::to_f32(E::from_f32(x[k][e])));
+        const float f = E::to_f32(r[k].v[e]);
+        sum += f * f;
+      }
+      reinterpret_cast<C *>(residual_out + row * hidden)[lane + kWave * k] = r[k];
+    }
+  sum = wave_sum(sum);
+  const float inv = rsqrtf(sum * factor + eps);
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    if (lane + kWave * k < chunks) {
+      C o;
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        float f = E::to_f32(r[k].v[e]) * inv;
+        // The FP32 rounding of the product stays, as in rms_norm_kernel.
+        if constexpr (std::is_same<T, f16_t>::value) asm volatile("" : "+v"(f));
+        const T n = E::from_f32(f);
+        o.v[e] = E::from_f32(E::to_f32(w[k].v[e]) * E::to_f32(n));
+      }
+      reinterpret_cast<C *>(out + row * hidden)[lane + kWave * k] = o;
+    }
+}
+
 template <typename T, int N>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const T *__restrict__ gate_up,
                                                        int64_t gu_stride, T *__restrict__ out,
@@ -339,4 +404,49 @@ extern "C" int mlr_silu_mul(const void *gate_up, int64_t gate_up_stride, void *o
       return set_error(MLR_ERR_INVALID, "mlr_silu_mul: dtype %d not supported (bf16, fp16, "
                        "fp32)", dtype);
   }
+}
+
+extern "C" int mlr_rms_norm_sums(const float *sums, int64_t splits, const void *residual,
+                                 int64_t residual_stride, void *residual_out,
+                                 const void *weight, void *out, int64_t rows, int64_t hidden,
+                                 double eps, int dtype, void *stream) {
+  clear_error();
+  MLR_REQUIRE(rows >= 0 && rows < INT32_MAX, "mlr_rms_norm_sums: bad rows");
+  MLR_REQUIRE(splits > 0 && splits <= 64, "mlr_rms_norm_sums: splits must be in [1, 64]");
+  const int64_t size = dtype_size(dtype);
+  MLR_REQUIRE(dtype == MLR_DTYPE_BF16 || dtype == MLR_DTYPE_F16 || dtype == MLR_DTYPE_F32,
+              "mlr_rms_norm_sums: dtype %d not supported (bf16, fp16, fp32)", dtype);
+  MLR_REQUIRE(hidden > 0 && hidden * size % 16 == 0 && hidden * size <= 4 * kWave * 16,
+              "mlr_rms_norm_sums: hidden must be whole 16-byte chunks, 256 at most");
+  MLR_REQUIRE(eps > 0, "mlr_rms_norm_sums: eps must be > 0");
+  if (rows == 0) return MLR_OK;
+  MLR_REQUIRE(sums && residual && residual_out && weight && out,
+              "mlr_rms_norm_sums: null pointer argument");
+  MLR_REQUIRE(residual_stride >= hidden && residual_stride * size % 16 == 0,
+              "mlr_rms_norm_sums: bad residual stride");
+  MLR_REQUIRE(aligned16(sums) && aligned16(residual) && aligned16(residual_out) &&
+                  aligned16(weight) && aligned16(out),
+              "mlr_rms_norm_sums: operands must be 16-byte aligned");
+  const float factor = static_cast<float>(rows) / static_cast<float>(rows * hidden);
+  const float e = static_cast<float>(eps);
+  const unsigned grid = static_cast<unsigned>(ceil_div(rows, 4));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  auto run = [&](auto tag) {
+    using T = decltype(tag);
+    constexpr int N = Vec16<T>::n;
+    auto go = [&](auto kernel) {
+      kernel<<<grid, 256, 0, s>>>(sums, static_cast<int>(splits), static_cast<const T *>(residual),
+                                  residual_stride, static_cast<T *>(residual_out),
+                                  static_cast<const T *>(weight), static_cast<T *>(out), rows,
+                                  static_cast<int>(hidden), factor, e);
+    };
+    const int64_t chunks = hidden / N;
+    if (chunks <= kWave) go(rms_norm_sums_kernel<T, N, 1>);
+    else if (chunks <= 2 * kWave) go(rms_norm_sums_kernel<T, N, 2>);
+    else go(rms_norm_sums_kernel<T, N, 4>);
+    return check_launch("mlr_rms_norm_sums");
+  };
+  if (dtype == MLR_DTYPE_BF16) return run(bf16_t{});
+  if (dtype == MLR_DTYPE_F16) return run(f16_t{});
+  return run(float{});
 }

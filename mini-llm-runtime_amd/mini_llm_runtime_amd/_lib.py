@@ -144,6 +144,14 @@ _PROTOTYPES = {
         _c_int,
         [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_int,
          _c_int, _c_ptr, _c_size, _c_ptr]),
+    "mlr_rms_norm_sums": (
+        _c_int,
+        [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_f64, _c_int,
+         _c_ptr]),
+    "mlr_norm_rows_linear": (
+        _c_int,
+        [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_f64, _c_ptr, _c_ptr, _c_i64, _c_i64,
+         _c_i64, _c_i64, _c_int, _c_ptr]),
     "mlr_rows_linear_workspace_size": (_c_size, [_c_i64, _c_i64, _c_i64, _c_int, _c_int]),
     "mlr_paged_kv_read_floor_outputs": (_c_size, [_c_i64, _c_i64, _c_i64, _c_i64]),
     "mlr_paged_kv_read_floor": (

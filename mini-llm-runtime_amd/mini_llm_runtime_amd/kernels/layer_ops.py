@@ -125,9 +125,10 @@ def _transformed() -> bool:
 
 
 def _rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
-                 gated: bool) -> torch.Tensor | None:
+                 gated: bool, sums: bool = False) -> torch.Tensor | RowSums | None:
     """The product by mlr_rows_linear, or None for a call that it does not
-    take (the caller then runs the PyTorch operations)."""
+    take (the caller then runs the PyTorch operations). With ``sums`` a product
+    whose k is split over workgroups comes back as its parts."""
     dtype = x.dtype
     if not x.is_cuda or weight.dtype != dtype or dtype not in DTYPES or weight.ndim != 2:
         return None
@@ -158,18 +159,103 @@ def _rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
         return None
     n_out = n // 2 if gated else n
     device = x.device
-    out = torch.empty((*x.shape[:-1], n_out), dtype=dtype, device=device)
     lib = _lib.load()
     code = _lib.DTYPE_CODES[dtype]
     nbytes = lib.mlr_rows_linear_workspace_size(rows, n_out, k, gated, code)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
+    out = None
+    if not (sums and nbytes):
+        sums = False
+        out = torch.empty((*x.shape[:-1], n_out), dtype=dtype, device=device)
     with _lib.on(device):
         status = lib.mlr_rows_linear(
-            xp, stride, wp, bias.data_ptr() if bias is not None else None, out.data_ptr(), n_out,
+            xp, stride, wp, bias.data_ptr() if bias is not None else None,
+            out.data_ptr() if out is not None else None, n_out,
             rows, n_out, k, gated, code, ws.data_ptr() if ws is not None else None, nbytes,
             _lib.stream_handle(device))
     _lib.check(status, "mlr_rows_linear")
+    if sums:
+        return RowSums(ws.view(torch.float32).view(-1, rows, n_out), (*x.shape[:-1], n_out), dtype)
     return out
+
+
+class RowSums:
+    """A product of a few rows still in its FP32 parts [splits, rows, n], for
+    the norm that follows it (rms_norm_sums); ``tensor()`` is the product."""
+
+    def __init__(self, parts: torch.Tensor, shape, dtype: torch.dtype) -> None:
+        self.parts, self.shape, self.dtype = parts, torch.Size(shape), dtype
+
+    def tensor(self) -> torch.Tensor:
+        total = self.parts[0]
+        for part in self.parts[1:]:  # in split order, as the kernels add
+            total = total + part
+        return total.to(self.dtype).view(self.shape)
+
+
+def rms_norm_sums(x: RowSums, weight: torch.Tensor, eps: float, residual: torch.Tensor):
+    """rms_norm(x.tensor(), weight, eps, residual) from the parts in one launch,
+    or None for operands that the kernel does not take."""
+    splits, rows, hidden = x.parts.shape
+    size = x.dtype.itemsize
+    if (weight.dtype != x.dtype or weight.shape != (hidden,) or residual.dtype != x.dtype
+            or residual.shape != x.shape or hidden * size % 16 or hidden * size > 4096):
+        return None
+    rr, weight = _rows(residual, "residual"), weight.contiguous()
+    if (rr.data_ptr() | weight.data_ptr()) & 15 or rr.stride(0) * size % 16 or rr.stride(0) < hidden:
+        return None
+    device = residual.device
+    out, res_out = torch.empty((2, *x.shape), dtype=x.dtype, device=device)
+    if (res_out.data_ptr() | x.parts.data_ptr()) & 15:
+        return None
+    with _lib.on(device):
+        status = _lib.load().mlr_rms_norm_sums(
+            x.parts.data_ptr(), splits, rr.data_ptr(), rr.stride(0), res_out.data_ptr(),
+            weight.data_ptr(), out.data_ptr(), rows, hidden, eps, _lib.DTYPE_CODES[x.dtype],
+            _lib.stream_handle(device))
+    _lib.check(status, "mlr_rms_norm_sums")
+    return out, res_out
+
+
+def norm_silu_mul(x: torch.Tensor, residual: torch.Tensor, norm_weight: torch.Tensor, eps: float,
+                  gate_up_weight: torch.Tensor):
+    """(linear_silu_mul(n, gate_up_weight), r) for (n, r) = rms_norm(x,
+    norm_weight, eps, residual) in one launch, or None for a call that
+    mlr_norm_rows_linear does not take (16-bit types, at most 32 rows of at most
+    1024)."""
+    dtype, k = x.dtype, x.shape[-1]
+    if (dtype not in (torch.bfloat16, torch.float16) or not x.is_cuda or k % 8 or k == 0
+            or gate_up_weight.ndim != 2 or gate_up_weight.shape[1] != k
+            or gate_up_weight.shape[0] % 2):
+        return None
+    rows, n = x.numel() // k, gate_up_weight.shape[0] // 2
+    if (rows == 0 or rows > 32 or k > (1024 if rows <= 16 else 1008)
+            or 2 * n * k * 2 > _ROWS_LIMIT[True, rows > 16, True]
+            or x.shape != residual.shape or norm_weight.shape != (k,)):
+        return None
+    for t in (x, residual, norm_weight, gate_up_weight):
+        if (t.dtype != dtype or t.device != x.device or t.stride(-1) != 1
+                or type(t) not in (torch.Tensor, nn.Parameter) or t.data_ptr() & 15):
+            return None
+    if not gate_up_weight.is_contiguous() or _transformed():
+        return None
+    if torch.is_grad_enabled() and (x.requires_grad or residual.requires_grad
+                                    or norm_weight.requires_grad):
+        return None
+    xr, rr = x.reshape(rows, k), residual.reshape(rows, k)
+    xs, rs = (xr.stride(0), rr.stride(0)) if rows > 1 else (k, k)
+    if xs < k or rs < k or xs % 8 or rs % 8 or (xr.data_ptr() | rr.data_ptr()) & 15:
+        return None
+    device = x.device
+    out = torch.empty((*x.shape[:-1], n), dtype=dtype, device=device)
+    res_out = torch.empty(x.shape, dtype=dtype, device=device)
+    with _lib.on(device):
+        status = _lib.load().mlr_norm_rows_linear(
+            xr.data_ptr(), xs, rr.data_ptr(), rs, res_out.data_ptr(), norm_weight.data_ptr(), eps,
+            gate_up_weight.data_ptr(), out.data_ptr(), n, rows, n, k, _lib.DTYPE_CODES[dtype],
+            _lib.stream_handle(device))
+    _lib.check(status, "mlr_norm_rows_linear")
+    return out, res_out
 
 
 def linear_silu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor) -> torch.Tensor:
@@ -182,13 +268,19 @@ def linear_silu_mul(x: torch.Tensor, gate_up_weight: torch.Tensor) -> torch.Tens
     return silu_mul(F.linear(x, gate_up_weight)) if out is None else out
 
 
-def apply_linear(module: nn.Module, x: torch.Tensor) -> torch.Tensor:
-    """module(x) for a projection of the model: a plain nn.Linear without
-    hooks goes through linear(), anything else is called as it is."""
-    if (type(module) is nn.Linear and not module._forward_hooks
+def plain(module: nn.Module, kind: type) -> bool:
+    """Whether `module` is a `kind` that computes what its class says: no
+    subclass, hook or replaced forward."""
+    return (type(module) is kind and not module._forward_hooks
             and not module._forward_pre_hooks and not module._backward_hooks
             and not module._backward_pre_hooks and "forward" not in module.__dict__
-            and not nn.modules.module._has_any_global_hook()):
+            and not nn.modules.module._has_any_global_hook())
+
+
+def apply_linear(module: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """module(x) for a projection of the model: a plain nn.Linear over a few
+    rows goes through mlr_rows_linear, anything else is called as it is."""
+    if plain(module, nn.Linear):
         out = _rows_linear(x, module.weight, module.bias, False)
         if out is not None:
             return out

@@ -109,6 +109,15 @@ class Qwen2RMSNorm(nn.Module):
         """(self(residual + hidden_states), residual + hidden_states): the
         decoder layer's residual add and the norm after it, in one launch on a
         HIP device."""
+        if isinstance(hidden_states, kops.RowSums):
+            # A down projection's parts (Qwen2DecoderLayer._few_rows_tail).
+            got = None
+            if type(self.weight) is nn.Parameter and hidden_states.shape == residual.shape:
+                got = kops.rms_norm_sums(hidden_states, self.weight, self.variance_epsilon,
+                                         residual)
+            if got is not None:
+                return got
+            hidden_states = hidden_states.tensor()
         if hidden_states.shape != residual.shape:
             raise ValueError("hidden_states and residual must have the same shape")
         if hidden_states.shape[-1] != self.weight.shape[0]:
@@ -176,13 +185,37 @@ class Qwen2DecoderLayer(nn.Module):
             normed = self.input_layernorm(residual)
         else:
             normed, residual = self.input_layernorm.forward_with_residual(delta, residual)
-        normed, residual = self.post_attention_layernorm.forward_with_residual(
-            attend(normed), residual)
+        attended = attend(normed)
+        tail = self._few_rows_tail(attended, residual)
+        if tail is not None:
+            return tail
+        normed, residual = self.post_attention_layernorm.forward_with_residual(attended, residual)
         return residual, self.mlp(normed)
+
+    def _few_rows_tail(self, attended: torch.Tensor, residual: torch.Tensor):
+        """The layer after its attention for a decode step's few rows: add, norm,
+        gate/up and activation in one launch, then the down projection, whose
+        parts stay unsummed for the next norm (RowSums). (residual', delta')
+        with the bits of the separate modules, or None where those run (other
+        sizes and dtypes, hooks, gradients)."""
+        norm, mlp = self.post_attention_layernorm, self.mlp
+        if (attended.shape[-1] > 1024 or attended.numel() > 32 * attended.shape[-1]
+                or not kops.plain(norm, Qwen2RMSNorm) or not kops.plain(mlp, Qwen2MLP)
+                or "forward_with_residual" in norm.__dict__
+                or not kops.plain(mlp.down_proj, nn.Linear)):
+            return None
+        got = kops.norm_silu_mul(attended, residual, norm.weight, norm.variance_epsilon,
+                                 mlp._gate_up_weight())
+        if got is None:
+            return None
+        gated, residual = got
+        down = mlp.down_proj
+        delta = kops._rows_linear(gated, down.weight, down.bias, False, sums=True)
+        return residual, (mlp.down_proj(gated) if delta is None else delta)
 
     def _block(self, hidden_states: torch.Tensor, attend) -> torch.Tensor:
         residual, delta = self._block_parts(hidden_states, None, attend)
-        return residual + delta
+        return residual + (delta.tensor() if isinstance(delta, kops.RowSums) else delta)
 
     def forward(self, hidden_states: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
         return self._block(hidden_states, lambda h: self.self_attn(h, position_ids))
