@@ -48,12 +48,11 @@ __device__ __forceinline__ float bf16_bits_to_float(uint32_t b) {
 
 // fp32 -> bf16 with round-to-nearest-even; every NaN becomes the canonical
 // quiet NaN 0x7FC0, which is what Tensor.to(torch.bfloat16) produces.
+// The hardware conversion (v_cvt_pk_bf16_f32) rounds so; it keeps a NaN's
+// payload, hence the select.
 __device__ __forceinline__ uint16_t float_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return 0x7fc0u;
-  // Add 0x7fff plus the lowest kept bit, then truncate: ties go to even.
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<uint16_t>(u >> 16);
+  const uint16_t h = __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
+  return f != f ? uint16_t(0x7fc0u) : h;
 }
 
 __device__ __forceinline__ float f16_bits_to_float(uint16_t b) {
