@@ -14,7 +14,7 @@
 // scale (rounded again), then an FP32 softmax over positions t < seq_len;
 // positions past seq_len and padded block-table entries never contribute.
 //
-// bf16, fp16 and FP32 inputs with head_dim 64 or 128, at most 16 query heads
+// bf16, fp16 and FP32 inputs with a head_dim of whole 8s up to 128, at most 16 query heads
 // per KV head and block_size a multiple of 16 take the matrix-core kernel in
 // paged_decode_mfma.hip (one launch, splits merged in it); everything else
 // takes the generic kernels below.
@@ -388,8 +388,17 @@ int run_decode(const void *q, int64_t q_stride_b, int64_t q_stride_h,
                        q_stride_b % 8 == 0 && q_stride_h % 8 == 0;
   // The matrix-core kernel keeps token positions in 32 bits, and the byte
   // offsets of a GQA group's q rows (group x q_stride_h elements).
+  // Head sizes other than 64 and 128 take its padded form for the splits that the
+  // generic kernel takes too (any other is refused there, as it always was),
+  // and not the rotary one; their block offsets are 30-bit.
+  const bool padded = head_dim != 64 && head_dim != 128;
+  const bool padded_ok =
+      (tokens_per_split <= 0 || (tokens_per_split % 16 == 0 && tokens_per_split <= kGenMaxSplit)) &&
+      (app == nullptr || app->inv_freq == nullptr) &&
+      block_size * num_kv_heads * head_dim * dtype_size(dtype) < (int64_t(1) << 28);
   const bool mfma =
       aligned && max_context < (int64_t(1) << 31) && q_stride_h < (int64_t(1) << 20) &&
+      (!padded || padded_ok) &&
       decode_mfma_eligible(dtype, head_dim, num_q_heads / num_kv_heads, block_size);
   int64_t ts = tokens_per_split > 0 ? tokens_per_split
                                     : default_tokens_per_split(mfma, head_dim, max_context, dtype);

@@ -286,7 +286,11 @@ struct LaneOffsets {
   int k;       // K row of token m16, chunk 0 of lane group g: ((m16 * hkv + kvh) * D) * size + 16g
   int v;       // V row of token 4g, dims VC*m16..: ((4g * hkv + kvh) * D + VC*m16) * size
   int v_step;  // bytes between consecutive token rows (hkv * D * size)
+  int k_dim;   // first dim of chunk 0 (padded head sizes only, with head)
+  int head;    // the head size
 };
+// An offset past every block, also after the row steps of a V load.
+constexpr int kPastBlock = 0x40000000;
 
 // Raw buffer resource over one physical block (gfx9 descriptor word 3). The
 // base is wave-uniform, so the loads use a scalar descriptor plus 32-bit lane
@@ -296,7 +300,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t block_rsrc(const void *base,
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);
 }
 
-template <typename T, int D>
+template <typename T, int D, bool kPad>
 __device__ __forceinline__ void load_tile(Tile<T, D> &t, const typename TileTraits<T, D>::S *kc,
                                           const typename TileTraits<T, D>::S *vc,
                                           int64_t block_elems, int tile_off_bytes, int blk,
@@ -317,9 +321,13 @@ __device__ __forceinline__ void load_tile(Tile<T, D> &t, const typename TileTrai
   const __amdgpu_buffer_rsrc_t rk = block_rsrc(kc + base, bytes);
   const __amdgpu_buffer_rsrc_t rv = block_rsrc(vc + base, bytes);
 #pragma unroll
-  for (int j = 0; j < QK; ++j)
+  for (int j = 0; j < QK; ++j) {
+    // Chunks past a padded head read as zeros.
+    const bool past = kPad && o.k_dim + 64 / kSize * j >= o.head;
     t.k[j] = __builtin_bit_cast(
-        uint4, __builtin_amdgcn_raw_buffer_load_b128(rk, o.k + 64 * j, tile_off_bytes, 0));
+        uint4, __builtin_amdgcn_raw_buffer_load_b128(rk, past ? kPastBlock : o.k + 64 * j,
+                                                     tile_off_bytes, 0));
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     if constexpr (sizeof(VT) == 8) {
@@ -416,7 +424,7 @@ __device__ __forceinline__ void softmax_update(DecodeState<D> &st, const float (
 // read from the cache; the substitution is a per-lane select at compute time,
 // so it never waits on the tile's loads and holds no registers before.
 // bf16 and fp16 (Half16 gives the dtype's rounding and MFMAs).
-template <int D, bool kAppend, typename T>
+template <int D, bool kAppend, bool kPad, typename T>
 __device__ __forceinline__ void compute_tile(DecodeState<D> &st, Tile<T, D> &t,
                                              const typename Half16<T>::v8 *qf, float scale,
                                              int live, int g, int m16,
@@ -462,6 +470,17 @@ __device__ __forceinline__ void compute_tile(DecodeState<D> &st, Tile<T, D> &t,
   }
   const s16x4_t pb = __builtin_bit_cast(
       s16x4_t, make_uint2(H::pack2(pr[0], pr[1]), H::pack2(pr[2], pr[3])));
+  // With kPad the rounded-off part of each probability goes through a second
+  // MFMA: the generic kernel these head sizes ran on keeps them FP32.
+  s16x4_t pl{};
+  if constexpr (kPad) {
+    float lo4[4] = {pr[0], pr[1], pr[2], pr[3]};
+    H::round2(lo4[0], lo4[1]);
+    H::round2(lo4[2], lo4[3]);
+    pl = __builtin_bit_cast(s16x4_t,
+                            make_uint2(H::pack2(pr[0] - lo4[0], pr[1] - lo4[1]),
+                                       H::pack2(pr[2] - lo4[2], pr[3] - lo4[3])));
+  }
 #pragma unroll
   for (int n = 0; n < VC; ++n) {
     const int c = n >> 1, h = n & 1;
@@ -471,6 +490,7 @@ __device__ __forceinline__ void compute_tile(DecodeState<D> &st, Tile<T, D> &t,
     const uint32_t hi = __builtin_amdgcn_perm(vword<D>(t.v[3], c), vword<D>(t.v[2], c), sel);
     const s16x4_t va = __builtin_bit_cast(s16x4_t, make_uint2(lo, hi));
     st.acc[n] = H::pv(va, pb, st.acc[n]);
+    if constexpr (kPad) st.acc[n] = H::pv(va, pl, st.acc[n]);
   }
 }
 
@@ -483,7 +503,7 @@ __device__ __forceinline__ void compute_tile(DecodeState<D> &st, Tile<T, D> &t,
 // accumulator c holds O[dim VC*(4g + i) + c][head l%16], as in the bf16
 // tile. Scores are q.k times scale in FP32, as the reference's FP32 matmul
 // and scale give them (kernels/reference/paged_attention.py:246-247).
-template <int D, bool kAppend>
+template <int D, bool kAppend, bool kPad>
 __device__ __forceinline__ void compute_tile(DecodeState<D> &st, Tile<float, D> &t,
                                              const f32x4_t *qf, float scale, int live, int g,
                                              int m16, const float *new_row) {
@@ -648,7 +668,7 @@ __device__ __forceinline__ float unpublish(uint32_t w) { return __uint_as_float(
 // tiles, so with kH = 2 both halves of every slot row are requested by one
 // workgroup at the same time.
 template <typename T, int D, int kBatch, bool kDouble, bool kAppend, bool kLds, int kH,
-          bool kRope, int kW>
+          bool kRope, int kW, bool kPad>
 __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkItem &it,
                                             int kvh_base) {
   constexpr bool kF32 = std::is_same<T, float>::value;
@@ -663,6 +683,8 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
   constexpr int kRowChunks = D / kE;      // 16-byte chunks per K (or V) row of one head
   constexpr int VC = D / 16;
   constexpr int kThreads = 64 * kW * kH;
+  static_assert(!kPad || (!kLds && !kRope), "padded head sizes: the plain layouts only");
+  const int hd = kPad ? p.d : D;  // head size: with kPad any multiple of 8 up to D
   const int lane = threadIdx.x & 63;
   // The wave index is uniform within a wave; saying so keeps every value
   // derived from it (tile counts, block ids, descriptors) in SGPRs.
@@ -687,15 +709,18 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
   // variant: one more memory round trip ahead of the tile loads).
   const bool head_ok = m16 < p.group;
   const uint32_t q_bytes =
-      static_cast<uint32_t>(((int64_t)(p.group - 1) * p.q_sh + D) * kSize);
+      static_cast<uint32_t>(((int64_t)(p.group - 1) * p.q_sh + hd) * kSize);
   const __amdgpu_buffer_rsrc_t q_r = block_rsrc(
       static_cast<const S *>(p.q) + b * p.q_sb + (int64_t)(kvh * p.group) * p.q_sh, q_bytes);
   const uint32_t q_off = head_ok ? static_cast<uint32_t>(m16 * p.q_sh * kSize) : q_bytes;
   uint4 qraw[QK];
 #pragma unroll
-  for (int j = 0; j < QK; ++j)
-    qraw[j] = __builtin_bit_cast(
-        uint4, __builtin_amdgcn_raw_buffer_load_b128(q_r, q_off + (4 * kE * j + kE * g) * kSize, 0, 0));
+  for (int j = 0; j < QK; ++j) {
+    const int dim = 4 * kE * j + kE * g;
+    const uint32_t off = kPad && dim >= hd ? q_bytes : q_off + dim * kSize;
+    qraw[j] =
+        __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(q_r, off, 0, 0));
+  }
   // Token positions fit in 32 bits here (max_blocks * block_size < 2^31;
   // speculative tile positions stay below 2^32): block index and offset by
   // shift and mask when block_size is a power of two, else 32-bit division.
@@ -729,7 +754,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
   const bool new_is_v = lane >= kRowChunks;
   const int new_off = kE * (new_is_v ? lane - kRowChunks : lane);
   uint4 new_chunk = make_uint4(0, 0, 0, 0);
-  if (new_owner && lane < 2 * kRowChunks)
+  if (new_owner && lane < 2 * kRowChunks && (!kPad || new_off < hd))
     new_chunk = *reinterpret_cast<const uint4 *>(
         static_cast<const S *>(new_is_v ? p.new_v : p.new_k) + b * p.new_sb +
         (int64_t)kvh * p.new_sh + new_off);
@@ -815,11 +840,14 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
     const int k = kbase + lane;
     blk_reg = valid_id(k, k < nk ? raw_block_id(k) : int64_t(-1));
   };
-  const int row_elems = p.hkv * D;  // elements of one slot (token row)
+  const int row_elems = p.hkv * hd;  // elements of one slot (token row)
   const int64_t block_elems = p.block_size * row_elems;
   LaneOffsets lo;
-  lo.k = (m16 * p.hkv + kvh) * D * kSize + 16 * g;
-  lo.v = ((4 * g * p.hkv + kvh) * D + VC * m16) * kSize;
+  lo.k = (m16 * p.hkv + kvh) * hd * kSize + 16 * g;
+  lo.v = kPad && VC * m16 >= hd ? kPastBlock
+                                : ((4 * g * p.hkv + kvh) * hd + VC * m16) * kSize;
+  lo.k_dim = kE * g;
+  lo.head = hd;
   lo.v_step = row_elems * kSize;
   const int live = static_cast<int>(t1 - t0);
   // The owning wave stores the new K/V rows to slot new_slots[b] and to LDS,
@@ -861,9 +889,9 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
     if (lane < 2 * kRowChunks) {
       *reinterpret_cast<uint4 *>(new_row_s[hs] + (new_is_v ? D : 0) + new_off) = v;
       const int64_t num_slots = p.num_blocks * p.block_size;
-      if (new_slot >= 0 && new_slot < num_slots) {
+      if (new_slot >= 0 && new_slot < num_slots && (!kPad || new_off < hd)) {
         S *dst = static_cast<S *>(new_is_v ? p.vc_w : p.kc_w) +
-                 (new_slot * p.hkv + kvh) * D + new_off;
+                 (new_slot * p.hkv + kvh) * hd + new_off;
         *reinterpret_cast<uint4 *>(dst) = v;
       }
     }
@@ -889,7 +917,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
       // Byte offset of the tile's first token inside its block.
       const int tile_off =
           static_cast<int>(in_block(static_cast<uint32_t>(t0) + rel)) * row_elems * kSize;
-      load_tile<T, D>(buf[u], kc, vc, block_elems, tile_off, blk, rel, lo);
+      load_tile<T, D, kPad>(buf[u], kc, vc, block_elems, tile_off, blk, rel, lo);
     }
     if (append_here) {
 #pragma unroll
@@ -902,7 +930,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
   auto compute = [&](Tile<T, D>(&buf)[kBatch]) {
 #pragma unroll
     for (int u = 0; u < kBatch; ++u)
-      compute_tile<D, kAppend>(st, buf[u], qf, scale, live, g, m16, new_row_s[hs]);
+      compute_tile<D, kAppend, kPad>(st, buf[u], qf, scale, live, g, m16, new_row_s[hs]);
   };
 
   // The wave holding the new token stages its rows once, after its first
@@ -943,7 +971,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
     if (kBatch < nk) {  // uniform
       read_tile_from_lds(buf[0], lds_tiles[wave], blk4, rel4, m16, g);
       if (append_here && rel4 == last_rel) mark_new_row(buf[0]);
-      compute_tile<D, kAppend>(st, buf[0], qf, scale, live, g, m16, new_row_s[hs]);
+      compute_tile<D, kAppend, kPad>(st, buf[0], qf, scale, live, g, m16, new_row_s[hs]);
     }
   } else {
     // Issued whatever nk is (absent tiles read zeros), so that every path
@@ -996,8 +1024,8 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
   const int64_t row_b = (int64_t)b * p.hq + head0;
   const int rows_g = ngh * p.split_stride;
   const __amdgpu_buffer_rsrc_t acc_r = __builtin_amdgcn_make_buffer_rsrc(
-      static_cast<float *>(p.ws_acc) + row_b * p.split_stride * D, 0,
-      static_cast<uint32_t>(rows_g) * D * 4u, 0x00020000);
+      static_cast<float *>(p.ws_acc) + row_b * p.split_stride * hd, 0,
+      static_cast<uint32_t>(rows_g) * hd * 4u, 0x00020000);
   const __amdgpu_buffer_rsrc_t ml_r = __builtin_amdgcn_make_buffer_rsrc(
       reinterpret_cast<float *>(p.ws_ml) + row_b * p.split_stride * 2, 0,
       static_cast<uint32_t>(rows_g) * 8u, 0x00020000);
@@ -1005,7 +1033,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
   // Outputs per thread, at most (at least the merge's kPre per pass).
   constexpr int kMaxOut = (16 * D + kThreads - 1) / kThreads < 2 ? 2
                                                                   : (16 * D + kThreads - 1) / kThreads;
-  const int nout = ngh * D;
+  const int nout = ngh * hd;
   float own[kMaxOut];
   __shared__ float own_m_s[16], own_l_s[16];
 #pragma unroll
@@ -1013,7 +1041,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
     const int idx = threadIdx.x + kThreads * r;
     own[r] = 0.f;
     if (idx < nout) {
-      const int h = idx / D, d = idx % D;
+      const int h = idx / hd, d = idx % hd;
       // Waves w0 .. w0 + kW - 1 hold head h (head hg of their group).
       const int w0 = kH == 1 ? 0 : (h / p.group) * kW;
       const int hg = kH == 1 ? h : h % p.group;
@@ -1037,7 +1065,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
         }
       } else {
         const uint32_t row = static_cast<uint32_t>(h * p.split_stride + split);
-        publish(acc_r, (row * D + d) * 4u, num);
+        publish(acc_r, (row * hd + d) * 4u, num);
         if (d == 0) {
           publish(ml_r, row * 8u, M);
           publish(ml_r, row * 8u + 4u, den);
@@ -1109,8 +1137,8 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
 #pragma unroll
       for (int r = 0; r < kPre; ++r) {
         const int idx = threadIdx.x + kThreads * (pass * kPre + r);
-        const int h = idx < nout ? idx / D : 0, d = idx % D;
-        abase[r] = ((h * p.split_stride + s0) * D + d) * 4;
+        const int h = idx < nout ? idx / hd : 0, d = idx % hd;
+        abase[r] = ((h * p.split_stride + s0) * hd + d) * 4;
       }
       uint32_t a[kPre][kChunk], mw = 0, lw = 0;
       for (int tries = 0;; ++tries) {
@@ -1123,7 +1151,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
         for (int s = 0; s < kChunk; ++s) {
 #pragma unroll
           for (int r = 0; r < kPre; ++r)
-            a[r][s] = __builtin_amdgcn_raw_buffer_load_b32(acc_r, abase[r] + s * D * 4, 0,
+            a[r][s] = __builtin_amdgcn_raw_buffer_load_b32(acc_r, abase[r] + s * hd * 4, 0,
                                                            kCoherent);
         }
         if (pass == 0) {
@@ -1180,7 +1208,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
         if (s < cnt) {  // uniform
 #pragma unroll
           for (int r = 0; r < kPre; ++r)
-            __builtin_amdgcn_raw_buffer_store_b32(0u, acc_r, abase[r] + s * D * 4, 0, kCoherent);
+            __builtin_amdgcn_raw_buffer_store_b32(0u, acc_r, abase[r] + s * hd * 4, 0, kCoherent);
         }
       }
       if (pass == 0) {
@@ -1217,7 +1245,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
       for (int r = 0; r < kPre; ++r) {
         const int idx = threadIdx.x + kThreads * (pass * kPre + r);
         if (idx < nout) {
-          const int h = idx / D;
+          const int h = idx / hd;
           float acc = num[pass * kPre + r] * rescale_s[h];
 #pragma unroll
           for (int s = 0; s < kChunk; ++s)
@@ -1234,7 +1262,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
     for (int r = 0; r < kMaxOut; ++r) {
       const int idx = threadIdx.x + kThreads * r;
       if (idx < nout)
-        out[b * p.o_sb + (int64_t)(head0 + idx / D) * p.o_sh + idx % D] = store_out(__builtin_nanf(""));
+        out[b * p.o_sb + (int64_t)(head0 + idx / hd) * p.o_sh + idx % hd] = store_out(__builtin_nanf(""));
     }
     return;
   }
@@ -1242,7 +1270,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
   for (int r = 0; r < kMaxOut; ++r) {
     const int idx = threadIdx.x + kThreads * r;
     if (idx < nout) {
-      const int h = idx / D, d = idx % D;
+      const int h = idx / hd, d = idx % hd;
       out[b * p.o_sb + (int64_t)(head0 + h) * p.o_sh + d] = store_out(num[r] / den_s[h]);
     }
   }
@@ -1253,14 +1281,14 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
 // table and the workgroups past the live items exit after the context
 // lengths.
 template <typename T, int D, int kBatch, bool kDouble, bool kAppend, bool kLds, int kH,
-          bool kRope, int kW>
+          bool kRope, int kW, bool kPad>
 __global__ __launch_bounds__(64 * kW * kH) void decode_mfma(DecodeParams p) {
   const int64_t cap = p.max_blocks * p.block_size;
   const int nhg = p.hkv / kH;  // KV-head groups per item
   const WorkItem it = find_item(p, blockIdx.x / nhg, cap);
   if (it.b < 0) return;  // uniform
-  decode_item<T, D, kBatch, kDouble, kAppend, kLds, kH, kRope, kW>(p, it,
-                                                                  (blockIdx.x % nhg) * kH);
+  decode_item<T, D, kBatch, kDouble, kAppend, kLds, kH, kRope, kW, kPad>(
+      p, it, (blockIdx.x % nhg) * kH);
 }
 
 }  // namespace
@@ -1268,19 +1296,19 @@ __global__ __launch_bounds__(64 * kW * kH) void decode_mfma(DecodeParams p) {
 bool decode_mfma_eligible(int dtype, int64_t head_dim, int64_t group,
                           int64_t block_size) {
   return (dtype == MLR_DTYPE_BF16 || dtype == MLR_DTYPE_F16 || dtype == MLR_DTYPE_F32) &&
-         (head_dim == 64 || head_dim == 128) && group >= 1 && group <= 16 &&
+         head_dim % 8 == 0 && head_dim >= 8 && head_dim <= 128 && group >= 1 && group <= 16 &&
          block_size % 16 == 0;
 }
 
-template <typename T, int D, int B, bool DB, bool A, bool L, int H, bool R, int W>
+template <typename T, int D, int B, bool DB, bool A, bool L, int H, bool R, int W, bool P = false>
 int launch_one(const DecodeParams &p, hipStream_t stream) {
   // Every (sequence, split) item that can exist, times the KV-head groups.
   const int64_t items = (int64_t)p.batch * p.max_splits * (p.hkv / H);
   if (items > 0x7fffffff)
     return set_error(MLR_ERR_UNSUPPORTED, "mlr_paged_decode: %lld work items exceed the grid",
                      (long long)items);
-  decode_mfma<T, D, B, DB, A, L, H, R, W><<<dim3(static_cast<unsigned>(items)), 64 * W * H,
-                                            0, stream>>>(p);
+  decode_mfma<T, D, B, DB, A, L, H, R, W, P><<<dim3(static_cast<unsigned>(items)), 64 * W * H,
+                                               0, stream>>>(p);
   return check_launch("mlr_paged_decode(mfma)");
 }
 
@@ -1317,7 +1345,33 @@ int launch_16bit(const DecodeParams &p, int tiles_per_wave, bool pairs, hipStrea
   return launch_variant<T, 128, 2, true, false>(p, stream);
 }
 
+// Head sizes other than 64 and 128 (multiples of 8 up to 128): the next larger
+// layout with the dims past the head as zeros, double-buffered, one KV head
+// per workgroup. The generic kernel they ran on walks a split's tokens in
+// FP32 on the VALU and combines in a second launch: 13 bf16 requests of up to
+// 2,011 tokens, 10/2 heads of 80, checked call 193 us, here 34; 83 of up to 337,
+// 6/3 heads of 32, 38 and 12 us; 3 fp16 of up to 747, 4/2 heads of 16, 36 and 13.
+template <typename T>
+int launch_padded(const DecodeParams &p, hipStream_t stream) {
+  constexpr bool kF32 = std::is_same<T, float>::value;
+  if (p.d < 64) {
+    constexpr int B = kF32 ? 2 : 4;
+    if (p.new_k == nullptr)
+      return launch_one<T, 64, B, true, false, false, 1, false, kWaves, true>(p, stream);
+    return launch_one<T, 64, B, true, true, false, 1, false, kWaves, true>(p, stream);
+  }
+  constexpr int B = kF32 ? 1 : 2;
+  if (p.new_k == nullptr)
+    return launch_one<T, 128, B, true, false, false, 1, false, kWaves, true>(p, stream);
+  return launch_one<T, 128, B, true, true, false, 1, false, kWaves, true>(p, stream);
+}
+
 int launch_decode_mfma(const DecodeParams &p, hipStream_t stream) {
+  if (p.d != 64 && p.d != 128) {
+    if (p.dtype == MLR_DTYPE_F32) return launch_padded<float>(p, stream);
+    if (p.dtype == MLR_DTYPE_F16) return launch_padded<f16_t>(p, stream);
+    return launch_padded<bf16_t>(p, stream);
+  }
   // Tiles per wave: ceil(ts / 16 / 4). A split whose tiles fit one load batch
   // needs no second register buffer (fewer VGPRs, more waves per SIMD); at
   // head_dim 64 a 320-token split lands its fifth tile per wave in LDS.

@@ -1,0 +1,111 @@
+"""Decode at head sizes other than 64 and 128: the padded matrix-core kernel
+against the generic kernel (which a split of 24 tokens still takes) and
+against attention in 64 bits.
+
+Both kernels round each score to the input type, as the reference does; their
+FP32 sums run in another order, so a score may round to its neighbour: one
+unit (2^-8 bf16, 2^-11 fp16 relative) of a score of up to about 6 moves its
+probability by that much. Outputs are weighted means of |V| < 5, so 2e-2 holds
+them for 16-bit types, and 1e-5 for FP32, the bounds of the other head sizes.
+Against 64 bits the new kernel may not be further off than the generic one."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from mini_llm_runtime_amd import _lib
+from mini_llm_runtime_amd.kernels import paged_attention as kpa
+
+pytestmark = pytest.mark.gpu
+DTYPES = [torch.bfloat16, torch.float16, torch.float32]
+
+
+def _case(dtype, d, hq, hkv, bs, lens, seed):
+    gen = torch.Generator().manual_seed(seed)
+    need = [-(-n // bs) for n in lens]
+    perm = torch.randperm(sum(need) + 3, generator=gen).tolist()
+    kc = torch.full((sum(need) + 3, bs, hkv, d), float("nan"), dtype=dtype)
+    vc = kc.clone()
+    tables, at = [], 0
+    for n, nb in zip(lens, need):
+        tables.append(perm[at:at + nb])
+        at += nb
+        pos = torch.arange(n)
+        blocks = torch.tensor(tables[-1])[pos // bs]
+        kc[blocks, pos % bs] = torch.randn(n, hkv, d, generator=gen).to(dtype)
+        vc[blocks, pos % bs] = torch.randn(n, hkv, d, generator=gen).to(dtype)
+    q = torch.randn(len(lens), hq, d, generator=gen).to(dtype)
+    bt = torch.tensor([t + [-1] * (max(need) - len(t)) for t in tables])
+    return q, kc, vc, bt, tables
+
+
+def _exact(q, kc, vc, tables, lens):
+    out = []
+    for i, (t, n) in enumerate(zip(tables, lens)):
+        k, v = (c[torch.tensor(t)].flatten(0, 1)[:n].double() for c in (kc, vc))
+        group = q.shape[1] // k.shape[1]
+        k, v = (x.repeat_interleave(group, dim=1) for x in (k, v))
+        s = (q[i].double()[None] * k).sum(-1) / math.sqrt(q.shape[2])
+        out.append((torch.softmax(s, dim=0)[..., None] * v).sum(0))
+    return torch.stack(out)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda t: str(t)[6:])
+@pytest.mark.parametrize("d,hq,hkv,bs,lens", [
+    (8, 4, 2, 16, [1, 40, 333]), (16, 4, 2, 16, [5] * 40), (24, 6, 6, 32, [64, 65, 1000]),
+    (32, 6, 3, 16, [300] * 50), (56, 16, 1, 64, [2000, 17]), (72, 4, 4, 16, [700, 1, 129]),
+    (80, 10, 2, 16, [2011, 103, 900]), (96, 8, 2, 16, [4000] * 3 + [7]), (120, 3, 1, 16, [513])])
+def test_padded_heads_match_generic_and_float64(device, dtype, d, hq, hkv, bs, lens):
+    q, kc, vc, bt, tables = _case(dtype, d, hq, hkv, bs, lens, seed=d)
+    wide = torch.zeros(len(lens), hq, d + 8, dtype=dtype)
+    wide[..., :d] = q
+    args = (kc.to(device), vc.to(device), bt.to(device), torch.tensor(lens).to(device))
+    got = kpa.paged_decode_launch(wide.to(device)[..., :d], *args)
+    again = kpa.paged_decode_launch(q.to(device), *args)
+    assert torch.equal(got, again)  # and the workspace came back zero
+    generic = kpa.paged_decode_launch(q.to(device), *args, tokens_per_split=24)
+    assert not any(w.any() for w in kpa._WORKSPACES.values())
+    tol = 1e-5 if dtype is torch.float32 else 2e-2
+    assert (got.double() - generic.double()).abs().max().item() <= tol
+    want = _exact(q, kc, vc, tables, lens)
+    off, was = ((x.double().cpu() - want).norm().item() for x in (got, generic))
+    assert off <= 1.1 * was + 1e-6 * want.norm().item()
+    for split in (16, 64, 512):
+        other = kpa.paged_decode_launch(q.to(device), *args, tokens_per_split=split)
+        assert (other.double() - got.double()).abs().max().item() <= tol
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda t: str(t)[6:])
+@pytest.mark.parametrize("d,hq,hkv", [(16, 4, 2), (40, 5, 1), (96, 8, 2), (120, 4, 4)])
+def test_append_equals_write_then_decode(device, dtype, d, hq, hkv):
+    lens = [1, 16, 17, 700]
+    q, kc, vc, bt, tables = _case(dtype, d, hq, hkv, 16, lens, seed=d + 1)
+    gen = torch.Generator().manual_seed(9)
+    new_k, new_v = (torch.randn(4, hkv, d, generator=gen).to(dtype).to(device) for _ in range(2))
+    slots = torch.tensor([t[(n - 1) // 16] * 16 + (n - 1) % 16 for t, n in zip(tables, lens)])
+    ctx, bt, q = torch.tensor(lens).to(device), bt.to(device), q.to(device)
+    pools = [(kc.to(device), vc.to(device)) for _ in range(2)]
+    got = kpa.paged_decode_launch(q, *pools[0], bt, ctx, new_k=new_k, new_v=new_v,
+                                  slot_mapping=slots.to(device))
+    for pool, rows in zip(pools[1], (new_k, new_v)):
+        pool.view(-1, hkv, d)[slots.to(device)] = rows
+    want = kpa.paged_decode_launch(q, *pools[1], bt, ctx)
+    assert torch.equal(got, want)
+    for a, b in zip(*pools):
+        assert torch.equal(a.nan_to_num(9.0), b.nan_to_num(9.0))
+
+
+def test_out_of_range_block_and_refusals(device):
+    q, kc, vc, bt, _ = _case(torch.float16, 80, 4, 2, 16, [100, 100], seed=1)
+    bt[0, 3] = kc.shape[0] + 5
+    args = (q.to(device), kc.to(device), vc.to(device), bt.to(device),
+            torch.tensor([100, 100]).to(device))
+    got = kpa.paged_decode_launch(*args)
+    generic = kpa.paged_decode_launch(*args, tokens_per_split=24)
+    assert (got.double() - generic.double()).abs().max().item() <= 2e-2
+    for split in (528, 1024):  # the generic kernel's limit stays these sizes' limit
+        with pytest.raises(_lib.KernelError):
+            kpa.paged_decode_launch(*args, tokens_per_split=split)
