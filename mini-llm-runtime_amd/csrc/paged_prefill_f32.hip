@@ -32,7 +32,9 @@
 // K rows past the last key the workgroup needs are read as that key's row and
 // masked, V rows past it as zeros; so are the rows of an out-of-range block.
 // Unwritten pool rows never reach a product. Head sizes other than 32, 64 and 128 (multiples of 4 up to 128) run
-// in the next larger kernel with the dims past the head as zeros.
+// in the next larger kernel with the dims past the head as zeros, each score in
+// four chains, and q unscaled (the score is scaled instead): as close to 64
+// bits as the generic kernel they ran on at short contexts, closer at long ones.
 //
 // Numerics: FP32 products and sums throughout (the reference's FP32 path,
 // kernels/reference/paged_attention.py:346-434); the scale is folded into q
@@ -139,7 +141,8 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
     for (int j = 0; j < QK; ++j) {
       const int e = 8 * j + 4 * half;
       const f32x4_t v = *reinterpret_cast<const f32x4_t *>(qrow + (kPad && e >= d ? 0 : e));
-      qf[j] = q_ok && !(kPad && e >= d) ? v * c2 : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      qf[j] = q_ok && !(kPad && e >= d) ? (kPad ? v : v * c2)
+                                            : f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
   }
   // Keys the workgroup needs: up to its last query's position.
@@ -258,11 +261,26 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
     }
     // S^T of the tile.
     f32x16_t s = f32x16_t{};
+    if constexpr (kPad) {
+      // Four chains: the generic kernel these head sizes ran on adds a score in
+      // eight parts, and one chain of D/2 steps was further from 64 bits than
+      // that at short contexts (2.5e-7 against 1.5e-7 at head size 96).
+      f32x16_t part[4];
 #pragma unroll
-    for (int j = 0; j < QK; ++j)
+      for (int j = 0; j < QK; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j][e], qf[j][e], s, 0, 0, 0);
+        for (int e = 0; e < 4; ++e)
+          part[j & 3] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+              kf[j][e], qf[j][e], j < 4 && e == 0 ? f32x16_t{} : part[j & 3], 0, 0, 0);
+      // q is not pre-scaled here: one FP32 rounding of the score instead.
+      s = ((part[0] + part[1]) + (part[2] + part[3])) * c2;
+    } else {
+#pragma unroll
+      for (int j = 0; j < QK; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j][e], qf[j][e], s, 0, 0, 0);
+    }
     __builtin_amdgcn_sched_barrier(0);
     if (k + 1 < nk) load_k(next);
     __builtin_amdgcn_sched_barrier(0);
