@@ -73,6 +73,8 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kWaves = 4;  // waves per KV head, unless a launch picks another count
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLog2eLo =  // log2(e) is kLog2e + kLog2eLo to 48 bits
+    static_cast<float>(1.4426950408889634 - static_cast<double>(kLog2e));
 
 template <int D> struct VRow;
 template <> struct VRow<64> { using type = uint2; };   // 4 bf16 per lane
@@ -404,13 +406,14 @@ __device__ __forceinline__ void read_tile_from_lds(Tile<T, 64> &t, const unsigne
 // probabilities.
 template <int D>
 __device__ __forceinline__ void softmax_update(DecodeState<D> &st, const float (&x)[4],
-                                               float (&pr)[4]) {
+                                               float (&pr)[4], const float *fine = nullptr) {
   float mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
   mx = max_xor32(max_xor16(mx));
   const float m_new = fmaxf(st.m, mx);  // finite: every tile has a live token
   const float alpha = __builtin_amdgcn_exp2f(st.m - m_new);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) pr[i] = __builtin_amdgcn_exp2f(x[i] - m_new);
+  for (int i = 0; i < 4; ++i)
+    pr[i] = __builtin_amdgcn_exp2f(fine != nullptr ? (x[i] - m_new) + fine[i] : x[i] - m_new);
   st.l = st.l * alpha + ((pr[0] + pr[1]) + (pr[2] + pr[3]));
   st.m = m_new;
   if (__any(alpha != 1.f)) {
@@ -525,17 +528,36 @@ __device__ __forceinline__ void compute_tile(DecodeState<D> &st, Tile<float, D> 
     }
   }
   f32x4_t s = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t part[4] = {s, s, s, s};
 #pragma unroll
   for (int j = 0; j < QK; ++j) {
     const f32x4_t k = __builtin_bit_cast(f32x4_t, t.k[j]);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(k[e], qf[j][e], s, 0, 0, 0);
+    for (int e = 0; e < 4; ++e) {
+      f32x4_t &to = kPad ? part[e] : s;
+      to = __builtin_amdgcn_mfma_f32_16x16x4f32(k[e], qf[j][e], to, 0, 0, 0);
+    }
   }
-  float x[4];
+  if constexpr (kPad) s = (part[0] + part[1]) + (part[2] + part[3]);
+  float x[4], pr[4];
+  if constexpr (kPad) {
+    // Four chains, and the exponent's rounded-off part kept: one chain and
+    // log2(e) in one float were 7% further from 64 bits than the generic
+    // kernel these head sizes ran on, at contexts up to 300 keys.
+    float fine[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) x[i] = (4 * g + i < lim) ? (s[i] * scale) * kLog2e : -INFINITY;
-  float pr[4];
-  softmax_update(st, x, pr);
+    for (int i = 0; i < 4; ++i) {
+      const float y = s[i] * scale, z = y * kLog2e;
+      const float rest = fmaf(y, kLog2eLo, fmaf(y, kLog2e, -z));
+      fine[i] = fabsf(z) < INFINITY ? rest : 0.f;
+      x[i] = (4 * g + i < lim) ? z : -INFINITY;
+    }
+    softmax_update(st, x, pr, fine);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = (4 * g + i < lim) ? (s[i] * scale) * kLog2e : -INFINITY;
+    softmax_update(st, x, pr);
+  }
   // Tokens past the context may hold anything (even NaN): zero their V.
   if (lim < 16) {
 #pragma unroll

@@ -132,7 +132,15 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
   // Q^T fragments of query q0 + m (zeros past the chunk and past the head).
   const int qi = q0 + m;
   const bool q_ok = qi < qlen;
-  const float c2 = static_cast<float>(p.scale) * kLog2eF32;
+  // The score's factor. With kPad it is kept in two floats and applied to the
+  // score, so the exponent is rounded once and not by c2 and the product too;
+  // its sign goes into q (exact) and a zero factor multiplies q, so a masked
+  // score stays -inf under it.
+  const double c64 = p.scale * 1.4426950408889634;
+  const float c2 = kPad ? (c64 == 0 ? 1.f : static_cast<float>(fabs(c64)))
+                        : static_cast<float>(p.scale) * kLog2eF32;
+  const float c2_lo = kPad && c64 != 0 ? static_cast<float>(fabs(c64) - c2) : 0.f;
+  const float q_factor = kPad ? (c64 == 0 ? 0.f : c64 < 0 ? -1.f : 1.f) : c2;
   f32x4_t qf[QK];
   {
     const float *qrow = static_cast<const float *>(p.q) +
@@ -141,8 +149,7 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
     for (int j = 0; j < QK; ++j) {
       const int e = 8 * j + 4 * half;
       const f32x4_t v = *reinterpret_cast<const f32x4_t *>(qrow + (kPad && e >= d ? 0 : e));
-      qf[j] = q_ok && !(kPad && e >= d) ? (kPad ? v : v * c2)
-                                            : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      qf[j] = q_ok && !(kPad && e >= d) ? v * q_factor : f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
   }
   // Keys the workgroup needs: up to its last query's position.
@@ -272,8 +279,7 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
         for (int e = 0; e < 4; ++e)
           part[j & 3] = __builtin_amdgcn_mfma_f32_32x32x2f32(
               kf[j][e], qf[j][e], j < 4 && e == 0 ? f32x16_t{} : part[j & 3], 0, 0, 0);
-      // q is not pre-scaled here: one FP32 rounding of the score instead.
-      s = ((part[0] + part[1]) + (part[2] + part[3])) * c2;
+      s = (part[0] + part[1]) + (part[2] + part[3]);  // times c2 below
     } else {
 #pragma unroll
       for (int j = 0; j < QK; ++j)
@@ -297,7 +303,7 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
 #pragma unroll
     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
     mx = other_half_max(mx);
-    const float m_new = fmaxf(m_run, mx);
+    const float m_new = fmaxf(m_run, kPad ? mx * c2 : mx);
     const float ref = m_new == -INFINITY ? 0.f : m_new;
     if (__any(m_new > m_run)) {
       const float alpha = __builtin_amdgcn_exp2f(m_run - ref);  // 0 while m_run is -inf
@@ -309,7 +315,10 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
     float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      s[i] = __builtin_amdgcn_exp2f(s[i] - ref);
+      if constexpr (kPad)  // the max keeps a masked score's small term finite
+        s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c2, -ref) + fmaxf(s[i], -1e30f) * c2_lo);
+      else
+        s[i] = __builtin_amdgcn_exp2f(s[i] - ref);
       sum[i & 3] += s[i];
     }
     l_run += (sum[0] + sum[1]) + (sum[2] + sum[3]);
