@@ -418,16 +418,24 @@ int run_decode(const void *q, int64_t q_stride_b, int64_t q_stride_h,
                 "mlr_paged_decode: tokens_per_split must be a multiple of 16");
   }
   const int64_t max_splits = ceil_div(max_context, ts);
-  MLR_REQUIRE(max_splits <= 8192,
+  // A padded head size asks for what the generic kernel's default split needs,
+  // never less than its own: the same calls are refused on either kernel.
+  const int64_t asked_splits =
+      mfma && padded && tokens_per_split <= 0
+          ? ceil_div(max_context, default_tokens_per_split(false, head_dim, max_context, dtype))
+          : max_splits;
+  MLR_REQUIRE(asked_splits <= 8192,
               "mlr_paged_decode: %lld splits exceed the combine limit of 8192; "
-              "raise tokens_per_split", (long long)max_splits);
+              "raise tokens_per_split", (long long)asked_splits);
   const DecodeWorkspace wl =
       decode_workspace_layout(batch, num_q_heads, head_dim, max_splits, dtype);
-  if (!workspace || workspace_bytes < static_cast<size_t>(wl.total)) {
+  const int64_t asked = std::max<int64_t>(
+      wl.total, decode_workspace_layout(batch, num_q_heads, head_dim, asked_splits, dtype).total);
+  if (!workspace || workspace_bytes < static_cast<size_t>(asked)) {
     return set_error(MLR_ERR_WORKSPACE,
                      "mlr_paged_decode: workspace of %zu bytes is smaller than "
                      "the %lld bytes required",
-                     workspace_bytes, (long long)wl.total);
+                     workspace_bytes, (long long)asked);
   }
   MLR_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0,
               "mlr_paged_decode: workspace must be 256-byte aligned");

@@ -109,3 +109,19 @@ def test_out_of_range_block_and_refusals(device):
     for split in (528, 1024):  # the generic kernel's limit stays these sizes' limit
         with pytest.raises(_lib.KernelError):
             kpa.paged_decode_launch(*args, tokens_per_split=split)
+
+
+def test_scratch_limit_stays_the_generic_kernels(device, monkeypatch):
+    """8,192-token tables: the generic default asks for 32 splits, the padded
+    kernel uses 16; a workspace that was too small stays refused."""
+    q, kc, vc, bt, _ = _case(torch.float16, 80, 4, 2, 16, [100, 33], seed=2)
+    bt = torch.nn.functional.pad(bt, (0, 512 - bt.shape[1]), value=-1)
+    args = (q.to(device), kc.to(device), vc.to(device), bt.to(device),
+            torch.tensor([100, 33]).to(device))
+    need = kpa.decode_workspace_bytes(2, 4, 80, 8192, torch.float16, 0)
+    want = kpa.paged_decode_launch(*args)
+    ws = torch.zeros(need, dtype=torch.uint8, device=device)
+    assert torch.equal(kpa.paged_decode_launch(*args, workspace=ws), want)
+    monkeypatch.setattr(_lib.load(), "mlr_paged_decode_workspace_size", lambda *a: 0)
+    with pytest.raises(_lib.KernelError, match="smaller than"):  # the C entry's own check
+        kpa.paged_decode_launch(*args, workspace=ws[:need - 256])
