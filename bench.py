@@ -1488,7 +1488,7 @@ def main():
             "frac_of_fp16_peak": round(pre16["tflops"] / BF16_PEAK_TFLOPS, 5)}
         pre32 = bench_prefill(device, dtype=torch.float32)
         line["prefill"]["fp32"] = {
-            "what": ("the same call in FP32 (v_mfma_f32_16x16x4_f32), against the 157.3 "
+            "what": ("the same call in FP32 (v_mfma_f32_32x32x2_f32), against the 157.3 "
                      "TFLOP/s FP32 matrix-core peak"),
             "us_per_call": pre32["us_per_call"],
             "tflops": round(pre32["tflops"], 3),

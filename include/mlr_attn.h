@@ -93,12 +93,12 @@ int mlr_kv_write(const void *k, const void *v, int src_dtype,
  * Bytes of workspace mlr_paged_decode needs for these sizes. `max_context`
  * bounds every context length (the host passes block_table width * block_size).
  * tokens_per_split <= 0 sizes for the library's default splits, whichever
- * kernel the call takes. The defaults: bf16 and FP32 with head_dim 64/128, at
- * most 16 query heads per KV head and block_size a multiple of 16
- * (matrix-core kernel): 320 tokens for bf16 head_dim 64 when max_context <=
- * 5120, else max(256, ceil(max_context / 16)) rounded up to a multiple of
- * 256; other dtypes and shapes an eighth of max_context as a power of two in
- * [32, 256].
+ * kernel the call takes. The defaults: bf16, fp16 and FP32 with head_dim a
+ * multiple of 8 up to 128, at most 16 query heads per KV head and block_size a
+ * multiple of 16 (matrix-core kernel): 320 tokens for 16-bit head_dim 64 when
+ * max_context <= 5120, else max(256, ceil(max_context / 16)) rounded up to a
+ * multiple of 256; other dtypes and shapes an eighth of max_context as a power
+ * of two in [32, 256].
  */
 size_t mlr_paged_decode_workspace_size(int64_t batch, int64_t num_q_heads,
                                        int64_t head_dim, int64_t max_context,
@@ -272,7 +272,8 @@ int mlr_paged_decode_static_check(void *stream);
  * P@V, output rounded once to the input type. kv_tile is the reference's
  * tile_size (the key tile of its online-softmax loop, :398-431), which orders
  * the FP32 accumulation and nothing else; the kernels step by their own key
- * tile (64 keys on the bf16 matrix-core kernel) whatever kv_tile is, so
+ * tile (64 keys on the 16-bit matrix-core kernel, 32 on the FP32 one)
+ * whatever kv_tile is, so
  * results differ from the reference's only by rounding, as they do between
  * the reference's own tile sizes.
  *   q               : [total_q, num_q_heads, head_dim], strides (q_stride_t, q_stride_h)

@@ -7,7 +7,8 @@
 //     MFMAs. Lane l holds K row l%32 and Q row l%32, floats 8j + 4(l/32) ..
 //     +4 of 8-float block j (one 16-byte load each): MFMA e of block j takes
 //     element e of both, so the k pairs of an MFMA lie 4 floats apart in K and
-//     Q alike. Q is loaded once, pre-multiplied by scale*log2(e).
+//     Q alike. Q is loaded once, at head sizes 32, 64 and 128 pre-multiplied
+//     by scale*log2(e) (see below for the others).
 //   Lane l then holds the scores of query l%32 and keys 8(i/4) + 4(l/32) + i%4,
 //     i < 16: the row max is 15 maxima and one swap with lane l^32; row sums
 //     stay per lane until the end. Online softmax in FP32, base 2.
@@ -31,14 +32,15 @@
 //
 // K rows past the last key the workgroup needs are read as that key's row and
 // masked, V rows past it as zeros; so are the rows of an out-of-range block.
-// Unwritten pool rows never reach a product. Head sizes other than 32, 64 and 128 (multiples of 4 up to 128) run
-// in the next larger kernel with the dims past the head as zeros, each score in
-// four chains, and q unscaled (the score is scaled instead): as close to 64
-// bits as the generic kernel they ran on at short contexts, closer at long ones.
+// Unwritten pool rows never reach a product. Head sizes other than 32, 64 and
+// 128 (multiples of 4 up to 128) run in the next larger kernel with the dims
+// past the head as zeros, each score in four chains, and q unscaled (the score
+// is scaled instead): as close to 64 bits as the generic kernel they ran on at
+// short contexts, closer at long ones.
 //
 // Numerics: FP32 products and sums throughout (the reference's FP32 path,
 // kernels/reference/paged_attention.py:346-434); the scale is folded into q
-// (one FP32 rounding). The reference's tile_size only orders its FP32
+// (one FP32 rounding) at the unpadded head sizes. The reference's tile_size only orders its FP32
 // accumulation, as the tiles and waves here do.
 //
 // Work: items are (sequence, 32-query tile) pairs, each run once per query

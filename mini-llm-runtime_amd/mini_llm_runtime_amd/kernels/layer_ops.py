@@ -1,12 +1,17 @@
-"""RMSNorm (with the residual add before it) and the MLP's silu(gate) * up on
-the HIP library: one launch each where PyTorch issues several.
+"""RMSNorm (with the residual add before it), the MLP's silu(gate) * up and
+linear layers over a decode step's few rows on the HIP library: one launch each
+where PyTorch issues several.
 
 ``rms_norm`` computes what ``Qwen2RMSNorm.forward`` computes (reference
 model/qwen2.py:88-123) and ``silu_mul`` what ``F.silu(gate) * up`` in
 ``Qwen2MLP.forward`` (:768-792) computes, with the same roundings (see
 csrc/layer_ops.hip); the decoder layer's residual add before its
 post-attention norm rides on ``rms_norm(..., residual=...)``. bf16, fp16 and
-FP32 on a HIP device; there is no PyTorch fallback.
+FP32 on a HIP device; there is no PyTorch fallback. ``apply_linear``,
+``linear_silu_mul``, ``norm_silu_mul`` and ``rms_norm_sums`` stream the weights
+of a 16-bit linear layer once for a few rows (csrc/rows_linear.hip), with the
+norm before it or the activation after it in the same launch; more rows go to
+the library's GEMM.
 """
 
 from __future__ import annotations
