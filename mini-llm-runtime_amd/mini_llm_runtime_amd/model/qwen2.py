@@ -199,9 +199,15 @@ class Qwen2DecoderLayer(nn.Module):
         with the bits of the separate modules, or None where those run (other
         sizes and dtypes, hooks, gradients)."""
         norm, mlp = self.post_attention_layernorm, self.mlp
-        if (attended.shape[-1] > 1024 or attended.numel() > 32 * attended.shape[-1]
+        # The stacked weight is asked for last: making it reads and copies gate
+        # and up, which a call that is not taken (on the CPU, under a
+        # transform, with a replaced projection) must not do.
+        if (not attended.is_cuda or attended.dtype not in (torch.bfloat16, torch.float16)
+                or attended.shape[-1] > 1024 or attended.numel() > 32 * attended.shape[-1]
+                or kops._transformed()
                 or not kops.plain(norm, Qwen2RMSNorm) or not kops.plain(mlp, Qwen2MLP)
                 or "forward_with_residual" in norm.__dict__
+                or type(mlp.gate_proj) is not nn.Linear or type(mlp.up_proj) is not nn.Linear
                 or not kops.plain(mlp.down_proj, nn.Linear)):
             return None
         got = kops.norm_silu_mul(attended, residual, norm.weight, norm.variance_epsilon,
