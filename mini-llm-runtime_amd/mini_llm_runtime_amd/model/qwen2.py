@@ -216,7 +216,8 @@ class Qwen2DecoderLayer(nn.Module):
             return None
         gated, residual = got
         down = mlp.down_proj
-        delta = kops._rows_linear(gated, down.weight, down.bias, False, sums=True)
+        # A bias is added after the sums: such a product is summed here.
+        delta = kops._rows_linear(gated, down.weight, down.bias, False, sums=down.bias is None)
         return residual, (mlp.down_proj(gated) if delta is None else delta)
 
     def _block(self, hidden_states: torch.Tensor, attend) -> torch.Tensor:

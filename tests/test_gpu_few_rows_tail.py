@@ -104,6 +104,27 @@ def test_tail_leaves_hooks_and_gradients_alone(device):
         assert layer._few_rows_tail(x, x) is None
 
 
+def test_biased_down_projection(device):
+    """A down projection with a bias whose k is split over workgroups: the tail
+    sums it, with the bits of the module's own product."""
+    config = TinyQwen2Config(hidden_size=896, intermediate_size=4864, num_attention_heads=14,
+                             num_key_value_heads=2)
+    torch.manual_seed(0)
+    with device, torch.no_grad():
+        layer = Qwen2DecoderLayer(config)
+        layer.mlp.down_proj = nn.Linear(4864, 896)
+        layer = layer.to(torch.bfloat16).eval()
+        x = torch.randn(4, 1, 896, dtype=torch.bfloat16)
+        residual, delta = layer._few_rows_tail(x, x)
+        gated, same = kops.norm_silu_mul(x, x, layer.post_attention_layernorm.weight, 1e-6,
+                                         layer.mlp._gate_up_weight())
+        want = torch.nn.functional.linear(gated.double(), layer.mlp.down_proj.weight.double(),
+                                          layer.mlp.down_proj.bias.double())
+    assert torch.equal(residual, same)
+    # One rounding to bf16, and FP32 sums of 4,864 products.
+    assert ((delta.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
+
+
 def test_entry_points_refuse(device):
     lib = _lib.load()
     b = torch.zeros(64, 1024, device=device, dtype=torch.bfloat16)
