@@ -175,27 +175,30 @@ class Qwen2DecoderLayer(nn.Module):
         self.post_attention_layernorm = Qwen2RMSNorm(config.hidden_size,
                                                      eps=config.rms_norm_eps)
 
-    def _block_parts(self, residual: torch.Tensor, delta: torch.Tensor | None, attend):
+    def _block_parts(self, residual: torch.Tensor, delta: torch.Tensor | None, attend,
+                     sums: bool = False):
         """The layer on the input residual + delta (delta None: the input is
         residual), returned as (residual', delta') whose sum is the layer's
         output. Each residual add rides in the launch of the norm after it
         (Qwen2RMSNorm.forward_with_residual), with the bits of a separate add
-        followed by the norm."""
+        followed by the norm. sums: delta' may be the parts of an unsummed
+        product (kops.RowSums), as its consumer is a Qwen2RMSNorm's
+        forward_with_residual."""
         if delta is None:
             normed = self.input_layernorm(residual)
         else:
             normed, residual = self.input_layernorm.forward_with_residual(delta, residual)
         attended = attend(normed)
-        tail = self._few_rows_tail(attended, residual)
+        tail = self._few_rows_tail(attended, residual, sums)
         if tail is not None:
             return tail
         normed, residual = self.post_attention_layernorm.forward_with_residual(attended, residual)
         return residual, self.mlp(normed)
 
-    def _few_rows_tail(self, attended: torch.Tensor, residual: torch.Tensor):
+    def _few_rows_tail(self, attended: torch.Tensor, residual: torch.Tensor, sums: bool = False):
         """The layer after its attention for a decode step's few rows: add, norm,
         gate/up and activation in one launch, then the down projection, whose
-        parts stay unsummed for the next norm (RowSums). (residual', delta')
+        parts stay unsummed for the next norm with `sums`. (residual', delta')
         with the bits of the separate modules, or None where those run (other
         sizes and dtypes, hooks, gradients)."""
         norm, mlp = self.post_attention_layernorm, self.mlp
@@ -217,12 +220,13 @@ class Qwen2DecoderLayer(nn.Module):
         gated, residual = got
         down = mlp.down_proj
         # A bias is added after the sums: such a product is summed here.
-        delta = kops._rows_linear(gated, down.weight, down.bias, False, sums=down.bias is None)
+        delta = kops._rows_linear(gated, down.weight, down.bias, False,
+                                  sums=sums and down.bias is None)
         return residual, (mlp.down_proj(gated) if delta is None else delta)
 
     def _block(self, hidden_states: torch.Tensor, attend) -> torch.Tensor:
         residual, delta = self._block_parts(hidden_states, None, attend)
-        return residual + (delta.tensor() if isinstance(delta, kops.RowSums) else delta)
+        return residual + delta
 
     def forward(self, hidden_states: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
         return self._block(hidden_states, lambda h: self.self_attn(h, position_ids))
@@ -321,11 +325,27 @@ class TinyQwen2Model(nn.Module):
         layer's MLP output rides in the next norm's launch, with the bits of a
         separate add (Qwen2DecoderLayer._block_parts)."""
         residual, delta = self.embed_tokens(input_ids), None
-        for layer_idx, layer in enumerate(self.layers):
-            residual, delta = layer._block_parts(residual, delta, attend_of(layer, layer_idx))
+        layers = list(self.layers)
+        for layer_idx, (layer, after) in enumerate(zip(layers, layers[1:] + [None])):
+            args = (residual, delta, attend_of(layer, layer_idx))
+            residual, delta = (layer._block_parts(*args, sums=True)
+                               if self._takes_sums(layer, after) else layer._block_parts(*args))
         if delta is None:
             return self.norm(residual)
         return self.norm.forward_with_residual(delta, residual)[0]
+
+    def _takes_sums(self, layer, after) -> bool:
+        """Whether `layer` may leave its down projection unsummed
+        (kops.RowSums): it and what takes its output, the layer `after` it or
+        (None) the final norm, are this file's own. A subclass or a method
+        replaced on an instance gets tensors."""
+        norm = self.norm
+        if after is not None:
+            if type(after) is not Qwen2DecoderLayer or "_block_parts" in after.__dict__:
+                return False
+            norm = after.input_layernorm
+        return (type(layer) is Qwen2DecoderLayer and "_block_parts" not in layer.__dict__
+                and type(norm) is Qwen2RMSNorm and "forward_with_residual" not in norm.__dict__)
 
     # Entry points -----------------------------------------------------------
     def forward(self, input_ids: torch.Tensor,

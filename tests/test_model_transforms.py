@@ -9,7 +9,9 @@ import torch
 import torch.nn as nn
 from torch.func import functional_call, grad, jvp, vmap
 
-from mini_llm_runtime_amd.model.qwen2 import TinyQwen2Config, TinyQwen2ForCausalLM
+from mini_llm_runtime_amd.kernels import layer_ops as kops
+from mini_llm_runtime_amd.model.qwen2 import (
+    Qwen2DecoderLayer, Qwen2RMSNorm, TinyQwen2Config, TinyQwen2ForCausalLM)
 
 IDS = torch.tensor([[1, 7, 3, 9, 2]])  # few enough rows for the fused layer tail
 
@@ -77,3 +79,74 @@ def test_replaced_projections_are_called(model, name):
         for layer in model.model.layers:
             setattr(layer.mlp, name, _Wrapped(getattr(layer.mlp, name)))
         assert torch.equal(model(IDS), want)
+
+
+class _AddingNorm(Qwen2RMSNorm):
+    def forward_with_residual(self, hidden_states, residual):
+        total = residual + hidden_states
+        return self(total), total
+
+
+class _ScalingLayer(Qwen2DecoderLayer):
+    def _block_parts(self, residual, delta, attend):
+        residual, delta = super()._block_parts(residual, delta, attend)
+        return residual, delta * 1.0
+
+
+def _replace(model, what):
+    """Replace one part of a four-layer model; the layers whose unsummed output
+    would have reached it."""
+    layers = model.model.layers
+    if what == "layer":
+        layer = _ScalingLayer(model.model.config)
+        layer.load_state_dict(layers[2].state_dict())
+        layers[2] = layer.to(layers[1].mlp.down_proj.weight)
+        return {1, 2}
+    if what == "method":
+        parts = layers[2]._block_parts
+        layers[2]._block_parts = lambda residual, delta, attend: parts(residual, delta, attend)
+        return {1, 2}
+    owner, name, producer = ((layers[2], "input_layernorm", 1) if what == "norm"
+                             else (model.model, "norm", 3))
+    norm = _AddingNorm(model.model.config.hidden_size)
+    norm.load_state_dict(getattr(owner, name).state_dict())
+    setattr(owner, name, norm.to(getattr(owner, name).weight))
+    return {producer}
+
+
+REPLACED = ["layer", "method", "norm", "final norm"]
+
+
+@pytest.mark.parametrize("what", REPLACED)
+def test_replaced_parts_get_tensors(monkeypatch, what):
+    model = TinyQwen2ForCausalLM(TinyQwen2Config(num_hidden_layers=4))
+    plain = _replace(model, what)
+    asked = []
+
+    def tail(layer, attended, residual, sums=True):
+        asked.append(sums)
+
+    monkeypatch.setattr(Qwen2DecoderLayer, "_few_rows_tail", tail)
+    with torch.no_grad():
+        model(IDS)
+    assert {i for i, sums in enumerate(asked) if not sums} == plain
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", REPLACED)
+def test_replaced_parts_run_on_the_gpu(device, what):
+    """A product whose k is split (4,864 columns): its parts reach only what
+    adds them, and the replaced model computes what the plain one does."""
+    torch.manual_seed(0)
+    model = TinyQwen2ForCausalLM(TinyQwen2Config(
+        hidden_size=896, intermediate_size=4864, num_hidden_layers=4, num_attention_heads=14,
+        num_key_value_heads=2)).to(device, torch.bfloat16).eval()
+    ids = IDS.to(device)
+    with torch.no_grad():
+        want = model(ids)
+        layer = model.model.layers[0]
+        x = torch.randn(1, 5, 896, device=device, dtype=torch.bfloat16)
+        assert isinstance(layer._few_rows_tail(x, x, True)[1], kops.RowSums)
+        assert isinstance(layer._few_rows_tail(x, x)[1], torch.Tensor)
+        _replace(model, what)
+        assert torch.equal(model(ids), want)
