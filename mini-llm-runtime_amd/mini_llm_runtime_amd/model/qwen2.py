@@ -386,10 +386,25 @@ class TinyQwen2Model(nn.Module):
             raise ValueError("slot_mapping length must match sequence length "
                              f"({input_ids.shape[1]}), got {slot_mapping.shape[0]}")
         self._check_cache(kv_cache)
-        return self._run(input_ids, lambda layer, i: lambda h:
-                         layer.self_attn.forward_prefill_with_cache(
-                             hidden_states=h, position_ids=position_ids, kv_cache=kv_cache,
-                             layer_idx=i, slot_mapping=slot_mapping, slots_checked=i > 0))
+        # Every layer gets the same slots: the first Qwen2Attention checks their
+        # values and the others do not repeat that. A replaced attention (whose
+        # signature may lack slots_checked) neither skips nor stands for it.
+        checked = False
+
+        def attend(layer, i, h):
+            nonlocal checked
+            attn, known = layer.self_attn, {}
+            own = (type(attn) is Qwen2Attention
+                   and "forward_prefill_with_cache" not in attn.__dict__)
+            if own and checked:
+                known = {"slots_checked": True}
+            out = attn.forward_prefill_with_cache(
+                hidden_states=h, position_ids=position_ids, kv_cache=kv_cache, layer_idx=i,
+                slot_mapping=slot_mapping, **known)
+            checked = checked or own
+            return out
+
+        return self._run(input_ids, lambda layer, i: lambda h: attend(layer, i, h))
 
     def forward_decode_with_cache(self, input_ids, position_ids, kv_cache, slot_mapping,
                                   block_table, context_len) -> torch.Tensor:

@@ -12,6 +12,8 @@ from torch.func import functional_call, grad, jvp, vmap
 from mini_llm_runtime_amd.kernels import layer_ops as kops
 from mini_llm_runtime_amd.model.qwen2 import (
     Qwen2DecoderLayer, Qwen2RMSNorm, TinyQwen2Config, TinyQwen2ForCausalLM)
+from mini_llm_runtime_amd.model.qwen2_attention import Qwen2Attention
+from mini_llm_runtime_amd.runtime.paged_kv_cache import PagedKVCache
 
 IDS = torch.tensor([[1, 7, 3, 9, 2]])  # few enough rows for the fused layer tail
 
@@ -130,6 +132,37 @@ def test_replaced_parts_get_tensors(monkeypatch, what):
     with torch.no_grad():
         model(IDS)
     assert {i for i, sums in enumerate(asked) if not sums} == plain
+
+
+class _PlainAttention(nn.Module):
+    """An attention with the reference's signature, and no slot check."""
+
+    def forward_prefill_with_cache(self, hidden_states, position_ids, kv_cache, layer_idx,
+                                   slot_mapping):
+        return hidden_states
+
+
+@pytest.mark.parametrize("replaced,want", [
+    ([], [False, True, True]), ([1], [False, True]), ([0], [False, True]), ([0, 1, 2], [])])
+def test_replaced_attention_keeps_its_signature(monkeypatch, replaced, want):
+    """The first Qwen2Attention of a whole-prompt prefill checks the slots,
+    wherever it is; a replacement is not told that they were checked."""
+    model = TinyQwen2ForCausalLM(TinyQwen2Config(num_hidden_layers=3))
+    seen = []
+
+    def attention(self, hidden_states, position_ids, kv_cache, layer_idx, slot_mapping, *,
+                  slots_checked=False):
+        seen.append(slots_checked)
+        return hidden_states
+
+    monkeypatch.setattr(Qwen2Attention, "forward_prefill_with_cache", attention)
+    for i in replaced:
+        model.model.layers[i].self_attn = _PlainAttention()
+    cache = PagedKVCache(3, 2, 16, model.model.config.num_key_value_heads,
+                         model.model.config.head_dim, device="cpu")
+    with torch.no_grad():
+        model.forward_prefill_with_cache(IDS, torch.arange(5)[None], cache, torch.arange(5))
+    assert seen == want
 
 
 @pytest.mark.gpu
