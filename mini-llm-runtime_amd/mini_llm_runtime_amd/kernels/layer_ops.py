@@ -68,7 +68,7 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     device = x.device
     with _lib.on(device):
         status = _lib.load().mlr_rms_norm(
-            xr.data_ptr(), xs, rp, rs or hidden, ro, hidden, weight.data_ptr(), out.data_ptr(),
+            xr.data_ptr(), xs, rp, hidden if rs is None else rs, ro, hidden, weight.data_ptr(), out.data_ptr(),
             hidden, rows, hidden, eps, _lib.DTYPE_CODES[x.dtype], _lib.stream_handle(device))
     _lib.check(status, "mlr_rms_norm")
     return out if residual is None else (out, res_out)

@@ -1,0 +1,59 @@
+"""What the Python entry points hand to the HIP library, on the CPU: a stand-in
+library records the calls, so a form that the kernels must refuse or never see
+is shown without a GPU."""
+
+from __future__ import annotations
+
+import contextlib
+
+import pytest
+import torch
+
+from mini_llm_runtime_amd import _lib
+from mini_llm_runtime_amd.kernels import layer_ops as kops
+from mini_llm_runtime_amd.kernels import paged_attention as kpa
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    """[(entry point, arguments)] of the library calls a test makes."""
+    seen = []
+
+    class Library:
+        def __getattr__(self, name):
+            def entry(*args):
+                seen.append((name, args))
+                return 0
+
+            return entry
+
+    monkeypatch.setattr(_lib, "load", Library)
+    monkeypatch.setattr(_lib, "on", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(_lib, "stream_handle", lambda device: 0)
+    monkeypatch.setattr(_lib, "require_hip", lambda *tensors, what: tensors[0].device)
+    monkeypatch.setattr(kops, "supported", lambda x: x.dtype in kops.DTYPES)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    return seen
+
+
+@pytest.mark.parametrize("strided", ["x", "residual", "neither"])
+def test_rms_norm_passes_a_zero_row_stride_on(calls, strided):
+    """One row expanded over many has row stride 0, which the entry point
+    refuses; read as whole rows it would run past the buffer."""
+    row = torch.ones(1, 64)
+    x, residual = (row.expand(4, 64) if strided == name else torch.ones(4, 64)
+                   for name in ("x", "residual"))
+    kops.rms_norm(x, torch.ones(64), 1e-6, residual=residual)
+    (name, args), = calls
+    assert name == "mlr_rms_norm"
+    assert (args[1], args[3]) == (0 if strided == "x" else 64, 0 if strided == "residual" else 64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("strided", ["x", "residual"])
+def test_rms_norm_refuses_a_zero_row_stride(device, strided):
+    row = torch.ones(1, 64, device=device)
+    x, residual = (row.expand(4, 64) if strided == name else torch.ones(4, 64, device=device)
+                   for name in ("x", "residual"))
+    with pytest.raises(_lib.KernelError, match="row stride"):
+        kops.rms_norm(x, torch.ones(64, device=device), 1e-6, residual=residual)
