@@ -44,13 +44,15 @@ _STAGE_MAX = 3840
 
 def _host_blocks(entries, required: int, num_blocks: int) -> array | None:
     """The first `required` block ids of a host table as an int64 array, or
-    None when one of them is out of range."""
+    None when one of them is out of range; entries past them may hold any
+    number."""
     try:
         used = array("q", entries)
-    except TypeError:  # numpy or tensor elements
-        used = array("q", [int(b) for b in entries])
-    except OverflowError:
-        return None
+    except (TypeError, OverflowError):  # other number types; beyond 64 bits
+        ids = [int(b) for b in entries][:required]
+        if any(b < 0 or b >= num_blocks for b in ids):
+            return None
+        return array("q", ids)
     del used[required:]
     if used and (min(used) < 0 or max(used) >= num_blocks):
         return None

@@ -57,3 +57,25 @@ def test_rms_norm_refuses_a_zero_row_stride(device, strided):
                    for name in ("x", "residual"))
     with pytest.raises(_lib.KernelError, match="row stride"):
         kops.rms_norm(x, torch.ones(64, device=device), 1e-6, residual=residual)
+
+
+@pytest.mark.parametrize("entries,want", [
+    ([3, 1, 2 ** 70], [3, 1]),  # past the blocks in use: any number
+    ([3, 1, -2 ** 70], [3, 1]), ([3, 1, 99], [3, 1]), ([3, 1.0, -1.5], [3, 1]),
+    ([3, 2 ** 70, 1], None), ([1e300, 3, 1], None), ([3, -1, 1], None), ([3, 8, 1], None),
+    ([torch.tensor(3), torch.tensor(1), torch.tensor(-4)], [3, 1]),
+    ([torch.tensor(3.0), torch.tensor(1.0), torch.tensor(-4.0)], [3, 1])])
+def test_host_tables_beyond_the_blocks_in_use(calls, entries, want):
+    """Only the blocks that the context uses are looked at for range."""
+    def chunk():
+        kv = torch.zeros(8, 16, 1, 8)
+        return kpa.paged_attention_prefill_chunk_tiled(torch.zeros(4, 1, 8), kv, kv, entries, 20,
+                                                       24, 16, 64)
+
+    if want is None:
+        with pytest.raises(ValueError, match="out-of-range physical block"):
+            chunk()
+        return
+    chunk()
+    assert list(kpa._host_blocks(entries, 2, 8)) == want
+    assert [a for a in calls if a[0] == "mlr_stage_i64"][0][1][1] == 2
