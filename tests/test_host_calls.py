@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import contextlib
 
+import numpy as np
 import pytest
 import torch
 
@@ -57,6 +58,17 @@ def test_rms_norm_refuses_a_zero_row_stride(device, strided):
                    for name in ("x", "residual"))
     with pytest.raises(_lib.KernelError, match="row stride"):
         kops.rms_norm(x, torch.ones(64, device=device), 1e-6, residual=residual)
+
+
+@pytest.mark.parametrize("eps", [1e-6, np.float32(1e-6), torch.tensor(1e-6), 1])
+def test_norms_take_any_number_as_eps(calls, eps):
+    """The library takes a C double, which ctypes makes of int and float only."""
+    kops.rms_norm(torch.ones(4, 64), torch.ones(64), eps)
+    kops.rms_norm_sums(kops.RowSums(torch.zeros(2, 4, 64), (4, 64), torch.float32),
+                       torch.ones(64), eps, torch.ones(4, 64))
+    assert [name for name, _ in calls] == ["mlr_rms_norm", "mlr_rms_norm_sums"]
+    for _, args in calls:
+        assert float(eps) in [a for a in args if type(a) is float]
 
 
 @pytest.mark.parametrize("entries,want", [
