@@ -586,6 +586,8 @@ def paged_attention_prefill_varlen(
     block_tables = _as_index_tensor(block_tables, device)
     query_start_loc = _as_index_tensor(query_start_loc, device)
     context_lens = _as_index_tensor(context_lens, device)
+    if query_start_loc.ndim == 0:
+        raise IndexError("query_start_loc must have at least one dimension")
     if max_query_len is None:
         qlens = query_start_loc[1:] - query_start_loc[:-1]
         max_query_len = int(qlens.max().item()) if qlens.numel() else 0

@@ -91,3 +91,14 @@ def test_host_tables_beyond_the_blocks_in_use(calls, entries, want):
     chunk()
     assert list(kpa._host_blocks(entries, 2, 8)) == want
     assert [a for a in calls if a[0] == "mlr_stage_i64"][0][1][1] == 2
+
+
+@pytest.mark.parametrize("max_query_len", [None, 4])
+def test_varlen_refuses_a_scalar_query_start_loc(calls, max_query_len):
+    """A 0-d query_start_loc holds one number where the kernel reads two."""
+    kv = torch.zeros(8, 16, 1, 8)
+    with pytest.raises(IndexError):
+        kpa.paged_attention_prefill_varlen(
+            torch.zeros(4, 1, 8), kv, kv, torch.zeros(1, 1, dtype=torch.long), torch.tensor(0),
+            torch.tensor([4]), 16, max_query_len=max_query_len)
+    assert not calls
