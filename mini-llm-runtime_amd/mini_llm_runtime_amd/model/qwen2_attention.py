@@ -333,7 +333,8 @@ class Qwen2Attention(nn.Module):
                         slot_mapping) -> bool:
         """Whether the prompt's rotation and cache write go through
         mlr_qkv_rope_write_prompt: a HIP cache of the model's shape and dtype,
-        integer positions and slots on its device, and a plain rotary module.
+        integer positions and slots on its device, and a plain rotary module
+        (what the projections give is looked at where it is used).
         Anything else takes the PyTorch rotation and write_slots, with their
         conversions and errors."""
         rotary, dtype = self.rotary_embedding, hidden_states.dtype
@@ -341,7 +342,6 @@ class Qwen2Attention(nn.Module):
                 and dtype in (torch.float32, torch.float16, torch.bfloat16)
                 and kv_cache.dtype == dtype and kv_cache.device == hidden_states.device
                 and kv_cache.k_cache.device == hidden_states.device
-                and self.qkv_proj.q_proj.weight.dtype == dtype
                 and 0 <= layer_idx < kv_cache.num_layers
                 and kv_cache.num_kv_heads == self.num_key_value_heads
                 and kv_cache.head_dim == self.head_dim

@@ -100,3 +100,22 @@ def test_what_keeps_the_torch_rotation(device):
             layer.forward_prefill_with_cache(x, pos, cache, 0, bad)
     with pytest.raises(IndexError, match="layer_idx"):
         layer.forward_prefill_with_cache(x, pos, cache, 2, slots)
+
+
+def test_replaced_projection_without_weights(device):
+    """A projection module without q_proj is called, as for any other path."""
+    class Wrapped(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, x):
+            return self.inner(x)
+
+    layer = _layer(64, 4, 2, torch.bfloat16, device)
+    x = torch.randn(1, 5, 64, device=device).bfloat16()
+    pos, slots = torch.arange(5, device=device)[None], torch.arange(5, device=device)
+    want = _run(layer, x, pos, slots, torch.bfloat16, device, 2, 16)
+    layer.qkv_proj = Wrapped(layer.qkv_proj)
+    for g, w in zip(_run(layer, x, pos, slots, torch.bfloat16, device, 2, 16), want):
+        assert torch.equal(g, w)
