@@ -110,11 +110,11 @@ def test_biased_down_projection(device):
     config = TinyQwen2Config(hidden_size=896, intermediate_size=4864, num_attention_heads=14,
                              num_key_value_heads=2)
     torch.manual_seed(0)
-    with device, torch.no_grad():
-        layer = Qwen2DecoderLayer(config)
-        layer.mlp.down_proj = nn.Linear(4864, 896)
-        layer = layer.to(torch.bfloat16).eval()
-        x = torch.randn(4, 1, 896, dtype=torch.bfloat16)
+    layer = Qwen2DecoderLayer(config)
+    layer.mlp.down_proj = nn.Linear(4864, 896)
+    layer = layer.to(device, torch.bfloat16).eval()
+    x = torch.randn(4, 1, 896, device=device, dtype=torch.bfloat16)
+    with torch.no_grad():
         residual, delta = layer._few_rows_tail(x, x)
         gated, same = kops.norm_silu_mul(x, x, layer.post_attention_layernorm.weight, 1e-6,
                                          layer.mlp._gate_up_weight())
