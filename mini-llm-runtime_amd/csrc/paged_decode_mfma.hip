@@ -157,6 +157,9 @@ template <> struct Half16<bf16_t> {
   __device__ static void round2(float &a, float &b) { bf16_round2(a, b); }
   __device__ static uint32_t pack2(float lo, float hi) { return bf16_pack2(lo, hi); }
   __device__ static float elem(const uint4 &v, int e) { return bf16_elem(v, e); }
+  __device__ static float widen(uint32_t w, int half) {
+    return __uint_as_float(half ? w & 0xffff0000u : w << 16);
+  }
   __device__ static f32x4_t qk(uint4 k, v8 q, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, k), q, c, 0, 0, 0);
   }
@@ -170,6 +173,9 @@ template <> struct Half16<f16_t> {
   __device__ static void round2(float &a, float &b) { f16_round2(a, b); }
   __device__ static uint32_t pack2(float lo, float hi) { return f16_pack2(lo, hi); }
   __device__ static float elem(const uint4 &v, int e) { return f16_elem(v, e); }
+  __device__ static float widen(uint32_t w, int half) {
+    return f16_bits_to_float(static_cast<uint16_t>(half ? w >> 16 : w));
+  }
   __device__ static f32x4_t qk(uint4 k, v8 q, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8, k), q, c, 0, 0, 0);
   }
@@ -471,19 +477,21 @@ __device__ __forceinline__ void compute_tile(DecodeState<D> &st, Tile<T, D> &t,
     for (int i = 0; i < 4; ++i)
       if (4 * g + i >= lim) t.v[i] = VT{};
   }
+  if constexpr (kPad) {
+    // The generic kernel multiplies FP32 probabilities by V in FP32, and so do
+    // these head sizes: with 16-bit parts of a probability a small one is lost,
+    // and a part that is 0 or negative turns an infinite V into NaN. V is
+    // widened (exactly); step i takes the tokens 4 g + i, as the FP32 tile does.
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int n = 0; n < VC; ++n)
+        st.acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+            H::widen(vword<D>(t.v[i], n >> 1), n & 1), pr[i], st.acc[n], 0, 0, 0);
+    return;
+  }
   const s16x4_t pb = __builtin_bit_cast(
       s16x4_t, make_uint2(H::pack2(pr[0], pr[1]), H::pack2(pr[2], pr[3])));
-  // With kPad the rounded-off part of each probability goes through a second
-  // MFMA: the generic kernel these head sizes ran on keeps them FP32.
-  s16x4_t pl{};
-  if constexpr (kPad) {
-    float lo4[4] = {pr[0], pr[1], pr[2], pr[3]};
-    H::round2(lo4[0], lo4[1]);
-    H::round2(lo4[2], lo4[3]);
-    pl = __builtin_bit_cast(s16x4_t,
-                            make_uint2(H::pack2(pr[0] - lo4[0], pr[1] - lo4[1]),
-                                       H::pack2(pr[2] - lo4[2], pr[3] - lo4[3])));
-  }
 #pragma unroll
   for (int n = 0; n < VC; ++n) {
     const int c = n >> 1, h = n & 1;
@@ -493,7 +501,6 @@ __device__ __forceinline__ void compute_tile(DecodeState<D> &st, Tile<T, D> &t,
     const uint32_t hi = __builtin_amdgcn_perm(vword<D>(t.v[3], c), vword<D>(t.v[2], c), sel);
     const s16x4_t va = __builtin_bit_cast(s16x4_t, make_uint2(lo, hi));
     st.acc[n] = H::pv(va, pb, st.acc[n]);
-    if constexpr (kPad) st.acc[n] = H::pv(va, pl, st.acc[n]);
   }
 }
 
@@ -1371,8 +1378,10 @@ int launch_16bit(const DecodeParams &p, int tiles_per_wave, bool pairs, hipStrea
 // layout with the dims past the head as zeros, double-buffered, one KV head
 // per workgroup. The generic kernel they ran on walks a split's tokens in
 // FP32 on the VALU and combines in a second launch: 13 bf16 requests of up to
-// 2,011 tokens, 10/2 heads of 80, checked call 193 us, here 34; 83 of up to 337,
-// 6/3 heads of 32, 38 and 12 us; 3 fp16 of up to 747, 4/2 heads of 16, 36 and 13.
+// 2,011 tokens, 10/2 heads of 80, 132 us in graphs, here 11.0; 83 of up to 337,
+// 6/3 heads of 32, 25.6 and 10.9; 3 fp16 of up to 747, 4/2 heads of 16, 33.4 and
+// 8.1; 32 fp16 of 4,000, 8/2 heads of 96, 238 and 33. P.V runs on the FP32 matrix
+// cores (16-bit parts of P were faster, 9.7, 9.8, 7.9 and 29 us, but fewer bits).
 template <typename T>
 int launch_padded(const DecodeParams &p, hipStream_t stream) {
   constexpr bool kF32 = std::is_same<T, float>::value;

@@ -125,3 +125,100 @@ def test_scratch_limit_stays_the_generic_kernels(device, monkeypatch):
     monkeypatch.setattr(_lib.load(), "mlr_paged_decode_workspace_size", lambda *a: 0)
     with pytest.raises(_lib.KernelError, match="smaller than"):  # the C entry's own check
         kpa.paged_decode_launch(*args, workspace=ws[:need - 256])
+
+
+def _close_with_nonfinite(got, want, tol):
+    got, want = got.double().cpu(), want.double().cpu()
+    for same in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(same(got), same(want))
+    fine = torch.isfinite(want)
+    assert bool(fine.any()) and (got - want)[fine].abs().max().item() <= tol
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda t: str(t)[6:])
+@pytest.mark.parametrize("d,hq,hkv", [(24, 4, 2), (80, 10, 2), (120, 3, 3)])
+def test_infinite_values_as_in_float64(device, dtype, d, hq, hkv):
+    """An infinite V gives that infinity, infinities of both signs NaN, at one
+    token (p = 1) and among many."""
+    lens = [1, 17, 40, 333, 700]
+    q, kc, vc, bt, tables = _case(dtype, d, hq, hkv, 16, lens, seed=d)
+
+    def put(b, token, dim, value):
+        vc[tables[b][token // 16], token % 16, :, dim] = value
+
+    put(0, 0, 0, math.inf)
+    put(1, 16, 3, -math.inf)
+    put(2, 5, 2, math.inf)
+    put(2, 20, 2, -math.inf)  # both signs: NaN
+    put(2, 7, 1, math.inf)
+    put(2, 33, 1, math.inf)
+    for token in range(0, 333, 9):
+        put(3, token, d - 1, math.inf)
+    put(4, 350, 5, math.nan)
+    args = (q.to(device), kc.to(device), vc.to(device), bt.to(device),
+            torch.tensor(lens).to(device))
+    tol = 1e-5 if dtype is torch.float32 else 2e-2
+    _close_with_nonfinite(kpa.paged_decode_launch(*args), _exact(q, kc, vc, tables, lens), tol)
+    _close_with_nonfinite(kpa.paged_decode_launch(*args, tokens_per_split=24),
+                          _exact(q, kc, vc, tables, lens), tol)
+
+
+def _one_query(dtype, d, scores, values):
+    """One request and head per row of scores [B, T]: q = (1, 0, ..), K rows whose
+    first element gives those scores after the scale, V = values [B, T] in dim 1;
+    (operands, the scores as rounded to dtype twice, in 64 bits)."""
+    batch, tokens = scores.shape
+    blocks = -(-tokens // 16)
+    kc = torch.zeros(batch * blocks, 16, 1, d, dtype=dtype)
+    vc = torch.zeros_like(kc)
+    k0 = (scores * math.sqrt(d)).to(dtype)
+    pad = blocks * 16 - tokens
+    kc[..., 0, 0] = torch.nn.functional.pad(k0, (0, pad)).view(-1, 16)
+    vc[..., 0, 1] = torch.nn.functional.pad(values.to(dtype), (0, pad)).view(-1, 16)
+    q = torch.zeros(batch, 1, d, dtype=dtype)
+    q[..., 0] = 1
+    scale = torch.tensor(1 / math.sqrt(d), dtype=torch.float32)
+    rounded = (k0.float() * scale).to(dtype).double()
+    return q, kc, vc, torch.arange(batch * blocks).view(batch, blocks), rounded
+
+
+@pytest.mark.parametrize("d", [40, 96])
+def test_small_probabilities_count(device, d):
+    """fp16: 999 probabilities of 2^-26 with V = 60,000 beside a larger key with
+    V = 0. Half the smallest fp16 is 2^-25: as 16-bit parts they vanish."""
+    scores = torch.full((1, 1000), -18.0)
+    scores[0, 500] = 0
+    values = torch.full((1, 1000), 60000.0)
+    values[0, 500] = 0
+    q, kc, vc, bt, rounded = _one_query(torch.float16, d, scores, values)
+    p = torch.softmax(rounded, dim=1)
+    want = (p * values.double()).sum().item()
+    got = kpa.paged_decode_launch(q.to(device), kc.to(device), vc.to(device), bt.to(device),
+                                  torch.tensor([1000]).to(device))[0, 0, 1].item()
+    # fp16 rounding 2^-11, and FP32 exponents of 18 * log2(e) = 26 +- 26 * 2^-24.
+    assert 0.4 < want and abs(got - want) <= 1e-3 * want
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda t: str(t)[6:])
+@pytest.mark.parametrize("d", [40, 96])
+def test_probabilities_keep_24_bits(device, dtype, d):
+    """Keys of score s, s and s beside one of score 0 with V chosen to cancel:
+    1 - p v1 - p v2 is about 2^-16 of the sum, where an error of 2^-18 in p shows.
+    FP32 leaves 2^-24 in p (exp2 to one unit, its argument s log2(e) of up to 2 to
+    half of one) and in each sum: 6 of them, 4e-7; 2^-8 is the output."""
+    batch = 64
+    s = torch.linspace(-1.3, -0.05, batch)[:, None]
+    scores = torch.cat([torch.zeros(batch, 1), s.expand(batch, 2)], dim=1)
+    rounded = _one_query(dtype, d, scores, torch.zeros(batch, 3))[4]
+    p = rounded.exp()[:, 1]
+    v1 = (1 / p).to(dtype).double()
+    rest = 1 - p * v1
+    # The last key takes what is left but for about 2^-15.
+    v2 = ((rest - 2.0 ** -15) / p).to(dtype).double()
+    values = torch.stack([torch.ones(batch).double(), -v1, -v2], dim=1)
+    q, kc, vc, bt, rounded = _one_query(dtype, d, scores, values)
+    want = (rounded.exp() * values).sum(1) / rounded.exp().sum(1)
+    got = kpa.paged_decode_launch(q.to(device), kc.to(device), vc.to(device), bt.to(device),
+                                  torch.full((batch,), 3).to(device))[:, 0, 1].double().cpu()
+    assert want.abs().min().item() > 2.0 ** -18
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 4e-7).all()
