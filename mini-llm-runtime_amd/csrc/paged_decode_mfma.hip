@@ -406,20 +406,31 @@ __device__ __forceinline__ void read_tile_from_lds(Tile<T, 64> &t, const unsigne
   }
 }
 
+// What exponents are taken against for a running maximum m. With kPad a maximum
+// of -inf (no key, or none with a score above -inf) counts as 0, so that what it
+// weighs becomes 0 and not exp2(-inf + inf).
+template <bool kPad>
+__device__ __forceinline__ float ref_point(float m) {
+  return kPad && m == -INFINITY ? 0.f : m;
+}
+
 // The online-softmax update of one tile: x[i] are the base-2 scores of the
 // lane's tokens 4g + i for head l%16 (-inf where masked; every tile has a
 // live token). Updates (m, l), rescales acc when m moved, and returns the
-// probabilities.
-template <int D>
+// probabilities. With kPad a head whose live scores are all -inf so far (q.K
+// past the type's range) keeps the reference point 0 and gets zeros, as on the
+// generic kernel; see ref_point.
+template <int D, bool kPad>
 __device__ __forceinline__ void softmax_update(DecodeState<D> &st, const float (&x)[4],
                                                float (&pr)[4], const float *fine = nullptr) {
   float mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
   mx = max_xor32(max_xor16(mx));
-  const float m_new = fmaxf(st.m, mx);  // finite: every tile has a live token
-  const float alpha = __builtin_amdgcn_exp2f(st.m - m_new);
+  const float m_new = fmaxf(st.m, mx);
+  const float ref = ref_point<kPad>(m_new);
+  const float alpha = __builtin_amdgcn_exp2f(st.m - ref);
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    pr[i] = __builtin_amdgcn_exp2f(fine != nullptr ? (x[i] - m_new) + fine[i] : x[i] - m_new);
+    pr[i] = __builtin_amdgcn_exp2f(fine != nullptr ? (x[i] - ref) + fine[i] : x[i] - ref);
   st.l = st.l * alpha + ((pr[0] + pr[1]) + (pr[2] + pr[3]));
   st.m = m_new;
   if (__any(alpha != 1.f)) {
@@ -470,7 +481,7 @@ __device__ __forceinline__ void compute_tile(DecodeState<D> &st, Tile<T, D> &t,
 #pragma unroll
   for (int i = 0; i < 4; ++i) x[i] = (4 * g + i < lim) ? r[i] * kLog2e : -INFINITY;
   float pr[4];
-  softmax_update(st, x, pr);
+  softmax_update<D, kPad>(st, x, pr);
   // Tokens past the context may hold anything (even NaN): zero their V.
   if (lim < 16) {
 #pragma unroll
@@ -559,11 +570,11 @@ __device__ __forceinline__ void compute_tile(DecodeState<D> &st, Tile<float, D> 
       fine[i] = fabsf(z) < INFINITY ? rest : 0.f;
       x[i] = (4 * g + i < lim) ? z : -INFINITY;
     }
-    softmax_update(st, x, pr, fine);
+    softmax_update<D, kPad>(st, x, pr, fine);
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) x[i] = (4 * g + i < lim) ? (s[i] * scale) * kLog2e : -INFINITY;
-    softmax_update(st, x, pr);
+    softmax_update<D, kPad>(st, x, pr);
   }
   // Tokens past the context may hold anything (even NaN): zero their V.
   if (lim < 16) {
@@ -1078,9 +1089,10 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
 #pragma unroll
       for (int ww = 1; ww < kW; ++ww) M = fmaxf(M, m_s[w0 + ww][hg]);
       float num = 0.f, den = 0.f;
+      const float ref = ref_point<kPad>(M);
 #pragma unroll
       for (int ww = 0; ww < kW; ++ww) {
-        const float f = __builtin_amdgcn_exp2f(m_s[w0 + ww][hg] - M);
+        const float f = __builtin_amdgcn_exp2f(m_s[w0 + ww][hg] - ref);
         num += f * o_s[w0 + ww][hg][d];
         den += f * l_s[w0 + ww][hg];
       }
@@ -1256,12 +1268,13 @@ __device__ __forceinline__ void decode_item(const DecodeParams &p, const WorkIte
           const float mc = ms < cnt ? unpublish(mw) : -INFINITY;
           float m_new = row_max16(fmaxf(m_old, mc));
           if (last) m_new = fmaxf(m_new, own_m_s[h]);
-          const float f = ms < cnt ? __builtin_amdgcn_exp2f(mc - m_new) : 0.f;
+          const float ref = ref_point<kPad>(m_new);
+          const float f = ms < cnt ? __builtin_amdgcn_exp2f(mc - ref) : 0.f;
           const float part = row_sum16(f * unpublish(lw));
           f_s[ms][h] = f;
           if (ms == 0) {
-            const float rs = __builtin_amdgcn_exp2f(m_old - m_new);  // 0 on the first chunk
-            const float f_own = last ? __builtin_amdgcn_exp2f(own_m_s[h] - m_new) : 0.f;
+            const float rs = __builtin_amdgcn_exp2f(m_old - ref);  // 0 on the first chunk
+            const float f_own = last ? __builtin_amdgcn_exp2f(own_m_s[h] - ref) : 0.f;
             f_s[kChunk][h] = f_own;
             rescale_s[h] = rs;
             den_s[h] = den_s[h] * rs + part + f_own * own_l_s[h];

@@ -222,3 +222,51 @@ def test_probabilities_keep_24_bits(device, dtype, d):
                                   torch.full((batch,), 3).to(device))[:, 0, 1].double().cpu()
     assert want.abs().min().item() > 2.0 ** -18
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 4e-7).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda t: str(t)[6:])
+@pytest.mark.parametrize("d,hq,hkv", [(24, 4, 2), (80, 10, 2)])
+def test_scores_of_minus_infinity(device, dtype, d, hq, hkv):
+    """Keys whose scores pass the type's range, alone in a 16-token tile or all
+    of a split: -inf takes no weight, +inf makes the output NaN, as on the
+    generic kernel (and in 64 bits with the scores so rounded)."""
+    lens = [1, 17, 18, 333, 700]
+    q, kc, vc, bt, tables = _case(dtype, d, hq, hkv, 16, lens, seed=d + 7)
+
+    def key(b, tokens, value):
+        for t in tokens:
+            kc[tables[b][t // 16], t % 16] = 0
+            kc[tables[b][t // 16], t % 16, :, 1] = value
+
+    q[:, :, 1] = q[:, :, 1].abs() + 2
+    q[2, 0, 1] *= -1  # this head's scores are +inf
+    big = 60000.0 if dtype is torch.float16 else 3e38
+    key(0, [0], -big)
+    key(1, [16], -big)
+    key(2, [17], -big)
+    key(3, range(0, 330), -big)
+    key(4, range(0, 64), -big)
+    key(4, [699], -big)
+    args = (q.to(device), kc.to(device), vc.to(device), bt.to(device),
+            torch.tensor(lens).to(device))
+    got = kpa.paged_decode_launch(*args)
+    tol = 1e-5 if dtype is torch.float32 else 2e-2
+    _close_with_nonfinite(got, kpa.paged_decode_launch(*args, tokens_per_split=24), tol)
+    assert got[0].isnan().all() and got[2, 0].isnan().all()
+    assert torch.isfinite(got[[1, 3, 4]]).all() and torch.isfinite(got[2, 1:]).all()
+    assert not any(w.any() for w in kpa._WORKSPACES.values())
+
+
+def test_whole_splits_of_out_of_range_blocks(device):
+    """Block ids out of range over whole splits, the first and the last ones."""
+    lens = [700, 700, 1500]
+    q, kc, vc, bt, _ = _case(torch.bfloat16, 80, 10, 2, 16, lens, seed=3)
+    bt[0, :30] = -5
+    bt[1, 20:44] = kc.shape[0] + 1
+    bt[2, :80] = 2 ** 40
+    args = (q.to(device), kc.to(device), vc.to(device), bt.to(device),
+            torch.tensor(lens).to(device))
+    for split in (0, 64, 256):
+        got = kpa.paged_decode_launch(*args, tokens_per_split=split)
+        _close_with_nonfinite(got, kpa.paged_decode_launch(*args, tokens_per_split=24), 2e-2)
+        assert torch.isfinite(got).all()
