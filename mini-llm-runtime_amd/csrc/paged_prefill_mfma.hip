@@ -64,13 +64,14 @@
 // the buffer resource, so the LDS rows are padded with zeros, Q likewise.
 // They ran on the generic kernel, whose queries, scores and probabilities
 // are FP32, so this form keeps them: q is not pre-scaled (the scores are
-// scaled and shifted by one FP32 fma each), and each probability goes to the
-// matrix cores as two 16-bit parts, the rounded value and what was rounded
-// off. That is half as many MFMAs again and 40 registers; the generic kernel
-// was bound by one FP32 multiply-add per lane and three shuffles per key.
+// scaled and shifted by one FP32 fma each), and P.V runs on the FP32 matrix
+// cores with V widened. That bounds it: eight times the matrix-core cycles of
+// the 16-bit P.V; the generic kernel was bound by one FP32 multiply-add per lane
+// and three shuffles per key.
 // fp16, 3 sequences of 60..400 queries on prefixes up to 800, 8/2 heads of 96:
-// 1,618 us per call before, 31.7 us now; error against 64 bits 6.7e-4 before,
-// 2.1e-4 now (the generic kernel rounds each score to the 16-bit type).
+// 1,618 us per call there, 78 us here (30 with each probability as two 16-bit
+// parts, which is fewer bits); error against 64 bits 6.7e-4 there, 2.1e-4 here
+// (the generic kernel rounds each score to the 16-bit type).
 #include "paged_prefill.h"
 
 #include <algorithm>
@@ -575,12 +576,10 @@ void prefill_mfma(PrefillParams p) {
     }
     if (bad != nullptr) bad[4 * lane + w] = static_cast<unsigned char>(sp.bad);
   };
-  constexpr int kLowBlocks = kPad ? KB : 1;
   // exp2 of a tile's S^T packed to the 16-bit type (the P@V operand), with the FP32
-  // probabilities added to the row sum (four chains).
-  // With kPad the rounded-off part of each probability is packed as well.
-  auto probs = [&](const f32x16_t (&sc)[KB], uint32_t (&pk)[KB][8],
-                   uint32_t (&pl)[kLowBlocks][8]) __attribute__((always_inline)) {
+  // probabilities added to the row sum (four chains). With kPad they stay FP32,
+  // in place of the scores.
+  auto probs = [&](f32x16_t (&sc)[KB], uint32_t (&pk)[KB][8]) __attribute__((always_inline)) {
     float lsum[4];
 #pragma unroll
     for (int j = 0; j < KB; ++j)
@@ -588,8 +587,12 @@ void prefill_mfma(PrefillParams p) {
       for (int x = 0; x < 8; ++x) {
         const float p0 = __builtin_amdgcn_exp2f(sc[j][2 * x]);
         const float p1 = __builtin_amdgcn_exp2f(sc[j][2 * x + 1]);
-        pk[j][x] = M::pack2(p0, p1);
-        if constexpr (kPad) pl[j][x] = M::pack2(p0 - M::lo(pk[j][x]), p1 - M::hi(pk[j][x]));
+        if constexpr (kPad) {
+          sc[j][2 * x] = p0;
+          sc[j][2 * x + 1] = p1;
+        } else {
+          pk[j][x] = M::pack2(p0, p1);
+        }
         if (j == 0 && x < 2) {
           lsum[2 * x] = p0;
           lsum[2 * x + 1] = p1;
@@ -600,9 +603,37 @@ void prefill_mfma(PrefillParams p) {
       }
     l_run += (lsum[0] + lsum[1]) + (lsum[2] + lsum[3]);
   };
+  // O^T += V^T P^T with kPad, from FP32 P: the V^T fragments of the 16-bit MFMA
+  // are widened, and element e of a lane's fragment meets the lane's own register
+  // 8 h16 + e of S^T, so each of its eight keys is one step of the FP32 MFMA (two
+  // keys, one per half-wave). 64 cycles a step: the VALU work hides behind it.
+  auto pv_f32 = [&](const f32x16_t (&p)[KB], const unsigned char *vst)
+      __attribute__((always_inline)) {
+    int voff[2][NB];
+    voffs(voff);
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      if (n == NB - 1 && 32 * n >= d) break;  // no dims of the head in the last block
+#pragma unroll
+      for (int kb = 0; kb < 2 * KB; ++kb) {
+        const uint2 lo = __builtin_bit_cast(
+            uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                       (lds_s16x4_t *)(vst + 16 * kb * C::kRowB + voff[0][n])));
+        const uint2 hi = __builtin_bit_cast(
+            uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                       (lds_s16x4_t *)(vst + 16 * kb * C::kRowB + voff[1][n])));
+        const uint32_t v4[4] = {lo.x, lo.y, hi.x, hi.y};
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+              e & 1 ? M::hi(v4[e >> 1]) : M::lo(v4[e >> 1]), p[kb >> 1][8 * (kb & 1) + e], acc[n],
+              0, 0, 0);
+      }
+    }
+  };
   // O^T += V^T P^T from packed P.
-  auto pv = [&](const uint32_t (&pk)[KB][8], const uint32_t (&pl)[kLowBlocks][8],
-                const unsigned char *vst) __attribute__((always_inline)) {
+  auto pv = [&](const uint32_t (&pk)[KB][8], const unsigned char *vst)
+      __attribute__((always_inline)) {
     int voff[2][NB];
     voffs(voff);
 #pragma unroll
@@ -622,23 +653,17 @@ void prefill_mfma(PrefillParams p) {
           const uint2 ulo = __builtin_bit_cast(uint2, lo), uhi = __builtin_bit_cast(uint2, hi);
           const v8 a = __builtin_bit_cast(v8, make_uint4(ulo.x, ulo.y, uhi.x, uhi.y));
           acc[n] = M::mfma(a, pb, acc[n]);
-          if constexpr (kPad)
-            acc[n] = M::mfma(a,
-                             __builtin_bit_cast(v8, make_uint4(pl[j][4 * h16], pl[j][4 * h16 + 1],
-                                                               pl[j][4 * h16 + 2],
-                                                               pl[j][4 * h16 + 3])),
-                             acc[n]);
         }
       }
     // Two MFMAs' V^T reads (two each) ahead of the MFMAs.
-    constexpr int kMfma = 2 * KB * NB, kEach = kPad ? 2 : 1;
+    constexpr int kMfma = 2 * KB * NB;
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
     for (int g = 0; g < kMfma - 2; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, kEach, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 2 * kEach, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
   };
 
   // Main loop: a ping-pong schedule of the two key-range splits (waves w and
@@ -694,8 +719,9 @@ void prefill_mfma(PrefillParams p) {
   if (split == 1) __builtin_amdgcn_s_barrier();
   // S^T (M to V) and packed P (V to M) are defined in every phase, idle
   // ones included, so neither is live across the phase that does not use it.
+  // With kPad s holds both in turn.
   f32x16_t s[KB];
-  uint32_t pk[KB][8], pl[kLowBlocks][8];
+  uint32_t pk[KB][8];
   uint32_t badw = 0;
   // M_i: K stage kst holds K(i) and its out-of-range flags kbad (read here:
   // V_i overwrites them), V stage vst holds V(i-1).
@@ -705,7 +731,10 @@ void prefill_mfma(PrefillParams p) {
     // Raised wave priority for the matrix work: the other split's softmax
     // phase on this SIMD takes the issue slots the MFMAs leave.
     __builtin_amdgcn_s_setprio(3);
-    if (i >= 1 && i - 1 < nw) pv(pk, pl, vst);
+    if (i >= 1 && i - 1 < nw) {
+      if constexpr (kPad) pv_f32(s, vst);
+      else pv(pk, vst);
+    }
     // P dies with the last P@V MFMA before S^T is allocated.
     __builtin_amdgcn_sched_barrier(0);
     if (i < nw) {
@@ -736,15 +765,12 @@ void prefill_mfma(PrefillParams p) {
       }
       if (t >= wave_nfull || badw != 0) mask(t, badw, s);
       rescale(tile_max(s), s);
-      probs(s, pk, pl);
+      probs(s, pk);
     } else {
 #pragma unroll
       for (int j = 0; j < KB; ++j)
 #pragma unroll
-        for (int x = 0; x < 8; ++x) {
-          pk[j][x] = 0;
-          if constexpr (kPad) pl[j][x] = 0;
-        }
+        for (int x = 0; x < 8; ++x) pk[j][x] = 0;
     }
     __builtin_amdgcn_s_waitcnt(kWaitBatch);
     __builtin_amdgcn_s_barrier();

@@ -3,10 +3,9 @@ bits.
 
 Bound per output: q.k of 16-bit inputs in FP32 is off by at most
 (d + 2) * 2^-24 * sum |q||k| (under 2^-15 after the scale, for these inputs),
-which moves a probability by that much relative; exp2 and the sums add a few
-2^-22, and the probability operand of the matrix cores carries at least 16
-bits (two 8-bit bf16 parts): 2^-16. The weighted mean of V is then off by
-under 2^-13 max |V|, and the result is rounded once (2^-8 bf16, 2^-11 fp16).
+which moves a probability by that much relative; exp2 and the sums, FP32
+probabilities times V, add a few 2^-22. The weighted mean of V is then off by
+under 2^-14 max |V|, and the result is rounded once (2^-8 bf16, 2^-11 fp16).
 FP32 inputs stay FP32 throughout: errors of independent roundings, about
 sqrt(d) 2^-24 |q||k| in a score, stay under the 1e-5 that the FP32 paths are
 held to.
@@ -27,7 +26,7 @@ HALF_ULP = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32:
 
 
 def _slack(dtype, vmax):
-    return 1e-5 if dtype is torch.float32 else 2.0 ** -13 * vmax
+    return 1e-5 if dtype is torch.float32 else 2.0 ** -14 * vmax
 
 
 def _attend(q, k, v, prefix):
@@ -111,3 +110,58 @@ def test_fp32_workgroup_shapes_match_float64(device, seqs, longest, prefix, hq, 
         want = _attend(q[qsl[i]:qsl[i + 1]].double(), k, v, p[i])
         off = (got[qsl[i]:qsl[i + 1]].double() - want).abs().max().item()
         assert off <= 1e-5, (i, off)
+
+
+def _one_chunk(device, q, k, v, prefix):
+    """One sequence in 16-row blocks, in order: (its chunk prefill, the
+    operands moved)."""
+    n = k.shape[0]
+    pools = []
+    for t in (k, v):
+        pool = torch.full((-(-n // 16) * 16, *t.shape[1:]), float("nan"), dtype=t.dtype)
+        pool[:n] = t
+        pools.append(pool.view(-1, 16, *t.shape[1:]).to(device))
+    return kpa.paged_attention_prefill_chunk_tiled(
+        q.to(device), *pools, list(range(pools[0].shape[0])), prefix, n, 16, 64)
+
+
+@pytest.mark.parametrize("d", [40, 96])
+@pytest.mark.parametrize("prefix", [999, 3999])  # whole, and split over workgroups
+def test_small_probabilities_count(device, d, prefix):
+    """fp16: probabilities of 2^-26 with V = 60,000 beside one larger key with
+    V = 0. Half the smallest fp16 is 2^-25: as 16-bit parts they vanish."""
+    k, v = (torch.zeros(prefix + 1, 1, d, dtype=torch.float16) for _ in range(2))
+    q = torch.zeros(1, 1, d, dtype=torch.float16)
+    q[..., 0] = 1
+    k[:, 0, 0] = -18 * math.sqrt(d)
+    k[500, 0, 0] = 0
+    v[:, 0, 1] = 60000
+    v[500, 0, 1] = 0
+    scores = k[:, 0, 0].double() / math.sqrt(d)
+    want = (torch.softmax(scores, 0) * v[:, 0, 1].double()).sum().item()
+    got = _one_chunk(device, q, k, v, prefix)[0, 0, 1].item()
+    # fp16 rounding 2^-11; FP32 scores of 18 move a probability by 18 * 2^-23.
+    assert 0.4 < want and abs(got - want) <= 1e-3 * want
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=lambda t: str(t)[6:])
+@pytest.mark.parametrize("d", [40, 96])
+def test_probabilities_keep_24_bits(device, dtype, d):
+    """Keys of score s, s and s beside one of score 0 with V chosen to cancel:
+    1 - p v1 - p v2 is about 2^-16 of the sum, where an error of 2^-18 in p shows.
+    FP32 leaves 2^-23 in p (its score and exp2) and 2^-24 in each sum: 4e-7 in
+    all; 2^-8 is the output."""
+    for s in torch.linspace(-1.3, -0.05, 24).tolist():
+        k, v = (torch.zeros(3, 1, d, dtype=dtype) for _ in range(2))
+        q = torch.zeros(1, 1, d, dtype=dtype)
+        q[..., 0] = 1
+        k[1:, 0, 0] = s * math.sqrt(d)
+        p = (k[1, 0, 0].double() / math.sqrt(d)).exp()
+        v[0, 0, 1] = 1
+        v[1, 0, 1] = -1 / p
+        v[2, 0, 1] = -(1 + p * v[1, 0, 1].double() - 2.0 ** -15) / p
+        want = (1 + p * v[1:, 0, 1].double().sum()) / (1 + 2 * p)
+        got = _one_chunk(device, q, k, v, 2)[0, 0, 1].double().cpu()
+        assert 2.0 ** -18 < abs(want)
+        assert abs(got - want) <= 2.0 ** -8 * abs(want) + 4e-7, (s, got, want)
+
