@@ -69,7 +69,7 @@
 // the 16-bit P.V; the generic kernel was bound by one FP32 multiply-add per lane
 // and three shuffles per key.
 // fp16, 3 sequences of 60..400 queries on prefixes up to 800, 8/2 heads of 96:
-// 1,618 us per call there, 78 us here (30 with each probability as two 16-bit
+// 1,618 us per call there, 82 us here (30 with each probability as two 16-bit
 // parts, which is fewer bits); error against 64 bits 6.7e-4 there, 2.1e-4 here
 // (the generic kernel rounds each score to the 16-bit type).
 #include "paged_prefill.h"
@@ -134,6 +134,9 @@ template <> struct Mma<bf16_t> {
   __device__ static float lo(uint32_t w) { return __uint_as_float(w << 16); }
   __device__ static float hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
   __device__ static uint32_t bits(float x) { return float_to_bf16_bits(x); }
+  // Bits 15 and 31: whether each half of w is an infinity or NaN (an exponent of
+  // all ones carries into the sign's place, and no further).
+  __device__ static uint32_t not_finite(uint32_t w) { return (w & 0x7f807f80u) + 0x00800080u; }
 };
 template <> struct Mma<f16_t> {
   using v8 = f16x8_t;
@@ -147,6 +150,7 @@ template <> struct Mma<f16_t> {
   __device__ static float lo(uint32_t w) { return f16_bits_to_float(static_cast<uint16_t>(w)); }
   __device__ static float hi(uint32_t w) { return f16_bits_to_float(static_cast<uint16_t>(w >> 16)); }
   __device__ static uint32_t bits(float x) { return float_to_f16_bits(x); }
+  __device__ static uint32_t not_finite(uint32_t w) { return (w & 0x7c007c00u) + 0x04000400u; }
 };
 
 // max(a, b, c) as one v_maximum3_f32 (NaN-propagating, no canonicalisation).
@@ -607,8 +611,53 @@ void prefill_mfma(PrefillParams p) {
   // are widened, and element e of a lane's fragment meets the lane's own register
   // 8 h16 + e of S^T, so each of its eight keys is one step of the FP32 MFMA (two
   // keys, one per half-wave). 64 cycles a step: the VALU work hides behind it.
-  auto pv_f32 = [&](const f32x16_t (&p)[KB], const unsigned char *vst)
+  //
+  // In tile t a masked key (p = 0) still meets V: a V row that is not finite
+  // would make NaN of the queries before it, which the generic kernel never
+  // showed it to. So the rows of a masked tile are looked through (a lane each,
+  // its chunks in an order of its own against bank conflicts), such rows are
+  // added apart, for the queries that see them, and count as zeros in the MFMAs.
+  // The search and the selects take 5% of a call (78 -> 82 us, see above).
+  auto pv_f32 = [&](int t, const f32x16_t (&p)[KB], const unsigned char *vst)
       __attribute__((always_inline)) {
+    static_assert(BN == 64, "a lane per row");
+    uint64_t rows = 0;
+    if (t >= wave_nfull) {  // uniform
+      uint32_t top = 0;
+#pragma unroll
+      for (int c = 0; c < C::kChunks; ++c) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(
+            vst + lane * C::kRowB + 16 * ((c + lane) & (C::kChunks - 1)));
+        top |= M::not_finite(v.x) | M::not_finite(v.y) | M::not_finite(v.z) | M::not_finite(v.w);
+      }
+      rows = __ballot(top & 0x80008000u);
+    }
+    for (uint64_t left = rows; left != 0; left &= left - 1) {
+      const int r = __builtin_ctzll(left);
+      float mine = 0.f;  // the lane's register for keys r and r ^ 4
+#pragma unroll
+      for (int j = 0; j < KB; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if ((r & ~4) == 32 * j + 8 * (i >> 2) + (i & 3)) mine = p[j][i];
+      const float pr = __shfl(mine, m32 + 8 * (r & 4));
+      if (t * BN + r <= qpos) {
+        const unsigned char *vrow = vst + r * C::kRowB + 8 * hh;
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+          for (int g4 = 0; g4 < 4; ++g4) {
+            const uint2 v = *reinterpret_cast<const uint2 *>(vrow + 16 * ((4 * n + g4) ^ swz<D>(r)));
+            acc[n][4 * g4] += pr * M::lo(v.x);
+            acc[n][4 * g4 + 1] += pr * M::hi(v.x);
+            acc[n][4 * g4 + 2] += pr * M::lo(v.y);
+            acc[n][4 * g4 + 3] += pr * M::hi(v.y);
+          }
+      }
+    }
+    // Bit 8 (e / 4) + e % 4 of each 16: the lane's key of element e is one.
+    const uint32_t skip[2] = {static_cast<uint32_t>(rows) >> (4 * hh),
+                              static_cast<uint32_t>(rows >> 32) >> (4 * hh)};
     int voff[2][NB];
     voffs(voff);
 #pragma unroll
@@ -624,10 +673,13 @@ void prefill_mfma(PrefillParams p) {
                        (lds_s16x4_t *)(vst + 16 * kb * C::kRowB + voff[1][n])));
         const uint32_t v4[4] = {lo.x, lo.y, hi.x, hi.y};
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-              e & 1 ? M::hi(v4[e >> 1]) : M::lo(v4[e >> 1]), p[kb >> 1][8 * (kb & 1) + e], acc[n],
-              0, 0, 0);
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t bit = 1u << (16 * (kb & 1) + 8 * (e >> 2) + (e & 3));
+          const float v = e & 1 ? M::hi(v4[e >> 1]) : M::lo(v4[e >> 1]);
+          acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(skip[kb >> 1] & bit ? 0.f : v,
+                                                        p[kb >> 1][8 * (kb & 1) + e], acc[n], 0, 0,
+                                                        0);
+        }
       }
     }
   };
@@ -732,7 +784,7 @@ void prefill_mfma(PrefillParams p) {
     // phase on this SIMD takes the issue slots the MFMAs leave.
     __builtin_amdgcn_s_setprio(3);
     if (i >= 1 && i - 1 < nw) {
-      if constexpr (kPad) pv_f32(s, vst);
+      if constexpr (kPad) pv_f32(t_lo + i - 1, s, vst);
       else pv(pk, vst);
     }
     // P dies with the last P@V MFMA before S^T is allocated.

@@ -165,3 +165,44 @@ def test_probabilities_keep_24_bits(device, dtype, d):
         assert 2.0 ** -18 < abs(want)
         assert abs(got - want) <= 2.0 ** -8 * abs(want) + 4e-7, (s, got, want)
 
+
+def _nonfinite_case(dtype, hq, hkv, d, prefix, n, seed):
+    """q, k, v with infinities and NaN in V rows a sequence owns: behind the
+    prefix, on the diagonal, next to each other and of both signs."""
+    gen = torch.Generator().manual_seed(seed)
+    q = torch.randn(n, hq, d, generator=gen).to(dtype)
+    k, v = (torch.randn(prefix + n, hkv, d, generator=gen).to(dtype) for _ in range(2))
+    last = prefix + n - 1
+    for t, dim, value in ((last, 0, math.inf), (last - n // 2, 1, -math.inf),
+                          (last - n // 3, 2, math.nan), (last - n // 3, 3, math.inf),
+                          (last - n // 3 + 1, 3, -math.inf), (prefix, d - 1, math.inf),
+                          (prefix // 2, 4, math.inf), (last - n // 5, d - 1, math.inf),
+                          (last - n // 7, d // 2, -math.inf)):
+        t = min(t, last)
+        v[t, t % hkv, dim] = value
+    return q, k, v
+
+
+def _attend_nonfinite(q, k, v, prefix):
+    """_attend where only the keys a query sees meet it."""
+    return torch.cat([_attend(q[i:i + 1], k[:prefix + i + 1], v[:prefix + i + 1], prefix + i)
+                      for i in range(q.shape[0])])
+
+
+NONFINITE = [(t, d, *rest) for t in (torch.bfloat16, torch.float16) for d in (24, 80, 96, 120)
+             for rest in ((0, 75), (300, 1), (70, 160), (2500, 40))]
+
+
+@pytest.mark.parametrize("dtype,d,prefix,n", NONFINITE, ids=lambda v: str(v).split(".")[-1])
+def test_infinite_values_as_in_float64(device, dtype, d, prefix, n):
+    """A value that is not finite reaches the queries that see its key, as that
+    infinity or NaN, and no other query."""
+    hq, hkv = 4, 2
+    q, k, v = _nonfinite_case(dtype, hq, hkv, d, prefix, n, d + n)
+    got = _one_chunk(device, q, k, v, prefix).double().cpu()
+    want = _attend_nonfinite(q.double(), k.double(), v.double(), prefix)
+    for same in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(same(got), same(want))
+    fine = torch.isfinite(want)
+    bound = HALF_ULP[dtype] * 1.01 * want.abs() + _slack(dtype, 5)
+    assert fine.any() and bool(((got - want).abs() <= bound)[fine].all())
