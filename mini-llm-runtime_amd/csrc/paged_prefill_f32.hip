@@ -7,8 +7,8 @@
 //     MFMAs. Lane l holds K row l%32 and Q row l%32, floats 8j + 4(l/32) ..
 //     +4 of 8-float block j (one 16-byte load each): MFMA e of block j takes
 //     element e of both, so the k pairs of an MFMA lie 4 floats apart in K and
-//     Q alike. Q is loaded once, at head sizes 32, 64 and 128 pre-multiplied
-//     by scale*log2(e) (see below for the others).
+//     Q alike. Q is loaded once, at head sizes 64 and 128 pre-multiplied by
+//     scale*log2(e) (see below for the others).
 //   Lane l then holds the scores of query l%32 and keys 8(i/4) + 4(l/32) + i%4,
 //     i < 16: the row max is 15 maxima and one swap with lane l^32; row sums
 //     stay per lane until the end. Online softmax in FP32, base 2.
@@ -31,12 +31,11 @@
 // x 512 queries after 2,000 keys 454 and 334 us (99 TFLOP/s).
 //
 // K rows past the last key the workgroup needs are read as that key's row and
-// masked, V rows past it as zeros; so are the rows of an out-of-range block.
-// Unwritten pool rows never reach a product. Head sizes other than 32, 64 and
-// 128 (multiples of 4 up to 128) run in the next larger kernel with the dims
-// past the head as zeros, each score in four chains, and q unscaled (the score
-// is scaled instead): as close to 64 bits as the generic kernel they ran on at
-// short contexts, closer at long ones.
+// masked, V rows past it as zeros. Of an out-of-range block, V rows are zeros and
+// pool row 0 stands in for K, masked: it may hold anything, no score of it is
+// used. Head sizes other than 64 and 128 (multiples of 4 up to 128) run in the
+// kernel of 32, 64 or 128 dims that holds them, with the dims past the head as
+// zeros, each score in four chains, and q unscaled (the score is scaled instead).
 //
 // Numerics: FP32 products and sums throughout (the reference's FP32 path,
 // kernels/reference/paged_attention.py:346-434); the scale is folded into q
@@ -134,15 +133,12 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
   // Q^T fragments of query q0 + m (zeros past the chunk and past the head).
   const int qi = q0 + m;
   const bool q_ok = qi < qlen;
-  // The score's factor. With kPad it is kept in two floats and applied to the
-  // score, so the exponent is rounded once and not by c2 and the product too;
-  // its sign goes into q (exact) and a zero factor multiplies q, so a masked
-  // score stays -inf under it.
+  // The score's factor, positive. With kPad it is kept in two floats and applied
+  // to the score, so the exponent is rounded once and not by c2 and the product
+  // too.
   const double c64 = p.scale * 1.4426950408889634;
-  const float c2 = kPad ? (c64 == 0 ? 1.f : static_cast<float>(fabs(c64)))
-                        : static_cast<float>(p.scale) * kLog2eF32;
-  const float c2_lo = kPad && c64 != 0 ? static_cast<float>(fabs(c64) - c2) : 0.f;
-  const float q_factor = kPad ? (c64 == 0 ? 0.f : c64 < 0 ? -1.f : 1.f) : c2;
+  const float c2 = kPad ? static_cast<float>(c64) : static_cast<float>(p.scale) * kLog2eF32;
+  const float c2_lo = kPad ? static_cast<float>(c64 - c2) : 0.f;
   f32x4_t qf[QK];
   {
     const float *qrow = static_cast<const float *>(p.q) +
@@ -151,7 +147,7 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
     for (int j = 0; j < QK; ++j) {
       const int e = 8 * j + 4 * half;
       const f32x4_t v = *reinterpret_cast<const f32x4_t *>(qrow + (kPad && e >= d ? 0 : e));
-      qf[j] = q_ok && !(kPad && e >= d) ? v * q_factor : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      qf[j] = q_ok && !(kPad && e >= d) ? (kPad ? v : v * c2) : f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
   }
   // Keys the workgroup needs: up to its last query's position.
@@ -426,11 +422,14 @@ bool prefill_f32_eligible(const PrefillParams &p, int dtype) {
                        (reinterpret_cast<uintptr_t>(p.out) & 15u) == 0 &&
                        p.q_st % 4 == 0 && p.q_sh % 4 == 0 && p.o_st % 4 == 0 &&
                        p.o_sh % 4 == 0;
-  // Positions are 32-bit inside the kernel.
+  // Positions are 32-bit inside the kernel. Where the scale multiplies the score
+  // (the padded form), it must not round to 0 in FP32: 0 times a masked score of
+  // -inf would be NaN. Smaller scales stay on the generic kernel.
   constexpr int64_t k2g = int64_t(1) << 31;
+  const bool padded = p.d != 64 && p.d != 128;
   return dtype == MLR_DTYPE_F32 && p.d % 4 == 0 && p.d <= 128 && aligned && p.bs_log2 >= 4 &&
          p.max_blocks * p.block_size < k2g && 16 * static_cast<int64_t>(p.hkv) * p.d * 4 < k2g &&
-         p.scale > 0.0 && p.scale < 1e30;
+         p.scale > (padded ? 1e-30 : 0.0) && p.scale < 1e30;
 }
 
 int launch_prefill_f32(const PrefillParams &p, int64_t max_query_len, hipStream_t stream) {

@@ -112,6 +112,25 @@ def test_fp32_workgroup_shapes_match_float64(device, seqs, longest, prefix, hq, 
         assert off <= 1e-5, (i, off)
 
 
+@pytest.mark.parametrize("dtype", list(HALF_ULP), ids=lambda t: str(t)[6:])
+@pytest.mark.parametrize("d", [24, 80])
+@pytest.mark.parametrize("scale", [1e-50, 1e-40, 1e-29])
+def test_scales_near_zero(device, dtype, d, scale):
+    """A scale that rounds to 0 or a subnormal FP32 number weighs all keys that a
+    query sees alike: the running mean of V."""
+    gen = torch.Generator().manual_seed(d)
+    n = 50
+    k, v = (torch.randn(4, 16, 2, d, generator=gen).to(dtype) for _ in range(2))
+    q = torch.randn(n, 4, d, generator=gen).to(dtype)
+    got = kpa.paged_prefill_launch(
+        q.to(device), k.to(device), v.to(device), torch.arange(4)[None].to(device),
+        torch.tensor([0, n]).to(device), torch.tensor([n]).to(device), n, scale=scale)
+    rows = v.view(64, 2, d)[:n].double().repeat_interleave(2, dim=1)
+    want = rows.cumsum(0) / torch.arange(1, n + 1)[:, None, None]
+    bound = HALF_ULP[dtype] * 1.01 * want.abs() + _slack(dtype, 5)
+    assert bool(((got.double().cpu() - want).abs() <= bound).all())
+
+
 def _one_chunk(device, q, k, v, prefix):
     """One sequence in 16-row blocks, in order: (its chunk prefill, the
     operands moved)."""
