@@ -37,6 +37,13 @@
 // kernel of 32, 64 or 128 dims that holds them, with the dims past the head as
 // zeros, each score in four chains, and q unscaled (the score is scaled instead).
 //
+// A V row that is not finite reaches the queries that see its key and no other,
+// though a masked key is in the MFMAs with probability 0: see the mask and the
+// loop after the tiles. Looking for one costs a masked tile 16 D / 32 multiply-adds;
+// no measurable time at 64 and 128 (4 x 300 tokens, 28/4 heads of 128, 52.1 and
+// 52.7 us), 8-10% at padded sizes, whose registers are full (3 chunks, 10/2 heads of
+// 80, 131 and 144 us).
+//
 // Numerics: FP32 products and sums throughout (the reference's FP32 path,
 // kernels/reference/paged_attention.py:346-434); the scale is folded into q
 // (one FP32 rounding) at the unpadded head sizes. The reference's tile_size only orders its FP32
@@ -244,6 +251,9 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
     }
   };
 
+  // V rows of the last tile and the one before it (no other is masked) that are
+  // not finite, bit r for row r, where this wave has the tile.
+  uint32_t late[2] = {0, 0};
   const int nk = ntiles > wave ? (ntiles - wave + kWaves - 1) / kWaves : 0;
   TileAt cur{};
   if (nk > 0) {  // uniform per wave
@@ -294,6 +304,46 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
 #pragma unroll
       for (int i = 0; i < 16; ++i)
         if (cur.bad[i >> 3] || key0 + 8 * (i >> 2) + 4 * half + (i & 3) > qpos) s[i] = -INFINITY;
+      // A masked key's probability is 0, but 0 times an infinity or NaN is NaN:
+      // V rows that are not finite count as zeros in the MFMAs of a masked tile
+      // and are added after the last one, for the queries that see them.
+      float none[2] = {0.f, 0.f};  // NaN if the lane's part of some row is not finite
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+#pragma unroll
+        for (int c = 0; c < VC; ++c) {
+          if constexpr (VC == 1) none[i & 1] = fmaf(vf[i], 0.f, none[i & 1]);
+          else none[i & 1] = fmaf(vf[i][c], 0.f, none[i & 1]);
+        }
+      const float any_off = none[0] + none[1];
+      if (__builtin_expect(key0 + kBNF - 1 > first_masked && __any(any_off != any_off), 0)) {
+        uint32_t rows = 0;  // bit r: row r of the tile
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          bool off = false;
+#pragma unroll
+          for (int c = 0; c < VC; ++c) {
+            float v;
+            if constexpr (VC == 1) v = vf[i];
+            else v = vf[i][c];
+            off |= !(fabsf(v) < INFINITY);
+          }
+          const uint64_t lanes = __ballot(off);
+          const int r = 8 * (i >> 2) + (i & 3);
+          if (static_cast<uint32_t>(lanes) != 0) rows |= 1u << r;
+          if (static_cast<uint32_t>(lanes >> 32) != 0) rows |= 16u << r;
+        }
+        // A span past the last key holds that key's row again: zeros as well,
+        // but not a key to look up in the block table.
+        const int keys = kv_end - key0;
+        if (keys <= kBNF) late[0] = rows & (~0u >> (kBNF - keys));
+        else late[1] = rows;
+        uint32_t own = rows >> (4 * half);
+        asm volatile("" : "+v"(own));
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (own & (1u << (8 * (i >> 2) + (i & 3)))) vf[i] = vec_t(0.f);
+      }
     }
     // Online softmax (base 2). The reference point stays 0 until the query
     // has seen a key, so masked scores give exactly zero probabilities.
@@ -334,6 +384,64 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_mfma(PrefillParams p)
     if (k + 1 < nk) load_v(next);
     __builtin_amdgcn_sched_barrier(0);
     cur = next;
+  }
+
+  // Out of line: a branch over it costs an instruction fetch.
+  if (__builtin_expect((late[0] | late[1]) != 0, 0)) {
+#pragma unroll 1
+    for (int t = 0; t < 2; ++t) {
+      const int key0 = (ntiles - 1 - t) * kBNF;
+#pragma unroll 1
+      for (uint32_t left = t == 0 ? late[0] : late[1]; left != 0; left &= left - 1) {  // uniform
+        const int key = key0 + __builtin_ctz(left);
+        // A uniform row under buffer resources, as in the main loop (an address in
+        // vector registers here would move the pools' there too). Dims past the
+        // head read as zeros.
+        const int64_t id = bt_row[key >> bs_log2];
+        const int64_t block = static_cast<int64_t>(
+            static_cast<uint64_t>(static_cast<uint32_t>(
+                __builtin_amdgcn_readfirstlane(static_cast<int>(id)))) |
+            (static_cast<uint64_t>(static_cast<uint32_t>(
+                 __builtin_amdgcn_readfirstlane(static_cast<int>(id >> 32))))
+             << 32));
+        const int64_t at = ((block << bs_log2) + (key & bs_mask)) * row_elems;
+        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float *>(kc + at), 0, 4u * d, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float *>(vc + at), 0, 4u * d, 0x00020000);
+        uint32_t hf = half;  // opaque: nothing of this is kept across the main loop
+        asm volatile("" : "+v"(hf));
+        float x = 0.f;  // the query's score for the key: a half-wave's dims, then both
+#pragma unroll
+        for (int j = 0; j < QK; ++j) {
+          const f32x4_t k = __builtin_bit_cast(
+              f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rk, 32 * j + 16 * hf, 0, 0));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x = fmaf(qf[j][i], k[i], x);
+        }
+        x += __shfl_xor(x, 32);
+        const float ref = m_run == -INFINITY ? 0.f : m_run;
+        const float pr = __builtin_amdgcn_exp2f(kPad ? fmaf(x, c2, -ref) + x * c2_lo : x - ref);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {  // dims VC * (8 (i / 4) + 4 half + i % 4) and on
+          const uint32_t off = 4u * VC * (8 * (i >> 2) + (i & 3)) + 16u * VC * hf;
+          vec_t v;
+          if constexpr (VC == 1)
+            v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, off, 0, 0));
+          else if constexpr (VC == 2)
+            v = __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b64(rv, off, 0, 0));
+          else
+            v = __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b128(rv, off, 0, 0));
+#pragma unroll
+          for (int c = 0; c < VC; ++c) {
+            float y;
+            if constexpr (VC == 1) y = v;
+            else y = v[c];
+            acc[c][i] += key <= qpos ? pr * y : 0.f;
+          }
+        }
+      }
+    }
   }
 
   // The waves' parts: (O^T, m, l) of each, lane-major, then wave w adds and

@@ -208,8 +208,10 @@ def _attend_nonfinite(q, k, v, prefix):
                       for i in range(q.shape[0])])
 
 
-NONFINITE = [(t, d, *rest) for t in (torch.bfloat16, torch.float16) for d in (24, 80, 96, 120)
+NONFINITE = [(t, d, *rest) for t in HALF_ULP for d in (24, 80, 96, 120)
              for rest in ((0, 75), (300, 1), (70, 160), (2500, 40))]
+NONFINITE += [(torch.float32, d, *rest) for d in (16, 32, 64, 128)
+              for rest in ((0, 75), (70, 160), (2500, 40))]
 
 
 @pytest.mark.parametrize("dtype,d,prefix,n", NONFINITE, ids=lambda v: str(v).split(".")[-1])
