@@ -69,8 +69,8 @@
 // the 16-bit P.V; the generic kernel was bound by one FP32 multiply-add per lane
 // and three shuffles per key.
 // fp16, 3 sequences of 60..400 queries on prefixes up to 800, 8/2 heads of 96:
-// 1,618 us per call there, 82 us here (30 with each probability as two 16-bit
-// parts, which is fewer bits); error against 64 bits 6.7e-4 there, 2.1e-4 here
+// 1,618 us per call there, 82 us here, 57 with the key ranges split (30 with each
+// probability as two 16-bit parts, which is fewer bits); error against 64 bits 6.7e-4 there, 2.1e-4 here
 // (the generic kernel rounds each score to the 16-bit type).
 #include "paged_prefill.h"
 
@@ -942,7 +942,7 @@ __global__ __launch_bounds__(256) void prefill_merge(PrefillParams p) {
 
 constexpr int kKeyTile = 64;      // BN of every instantiation
 constexpr int kMaxKeySplits = 8;  // most splits of an item's key range
-constexpr int kMinSplitTiles = 8; // fewest key tiles worth a workgroup
+constexpr int kMinSplitTiles = 8; // fewest key tiles worth a workgroup at 64 and 128
 
 // How a launch of `items` work items x `hq` heads splits key ranges of up to
 // max_tiles tiles: into as many parts as give the GPU one workgroup per CU,
@@ -955,6 +955,12 @@ constexpr int kMinSplitTiles = 8; // fewest key tiles worth a workgroup
 // 16 tiles in two 17.3 / 17.2 and a 1024-token prompt in two 20.6 / 17.6.
 // 28/4 heads of 128: a chunk of 16 after 2000 27.2 / 36.8, of 512 after 4000
 // 57 / 69, after 16000 142 / 213; of 512 after 1000 36.3 / 33.6.
+// The padded head sizes, P.V on the FP32 matrix cores, take 1.4 us a tile up to 64
+// dims and 3.4 past them, so half the tiles are worth a workgroup and two saved pay:
+// 8/2 heads of 96, a chunk of 16 after 1000 34 / 79, of 128 after 200 33 / 40; 3 of
+// 60..400 on up to 800 57 / 82; 6/3 heads of 32, of 16 after 400 19.5 / 20.9; parts
+// of two tiles are a little better at 96 (16 after 600 27 against 33) and worse at
+// 32 (16 after 200 16.7 / 15.3).
 struct KeySplits {
   int max_splits, split_tiles;  // max_splits 1: no split
 };
@@ -962,8 +968,10 @@ KeySplits key_splits(int64_t items, int64_t hq, int64_t max_tiles, int64_t head_
   const int64_t want =
       std::min<int64_t>(kMaxKeySplits, current_device_cus() / (items * hq));
   if (want < 2 || items * want > kRankMax) return {1, 1};
-  const int64_t per = std::max<int64_t>(kMinSplitTiles, ceil_div(max_tiles, want));
-  if (max_tiles - per < (head_dim == 64 ? 20 : 16)) return {1, 1};
+  const bool padded = head_dim != 64 && head_dim != 128;
+  const int64_t per =
+      std::max<int64_t>(padded ? kMinSplitTiles / 2 : kMinSplitTiles, ceil_div(max_tiles, want));
+  if (max_tiles - per < (padded ? 2 : head_dim == 64 ? 20 : 16)) return {1, 1};
   return {static_cast<int>(ceil_div(max_tiles, per)), static_cast<int>(per)};
 }
 

@@ -74,6 +74,18 @@ def test_chunk_split_equals_unsplit(device, monkeypatch, dtype, hq, hkv, d, pref
 
 
 @pytest.mark.parametrize("dtype", list(ULP), ids=lambda t: str(t)[6:])
+@pytest.mark.parametrize("hq,hkv,d,prefix,chunk,splits", [
+    (8, 2, 96, 256, 64, False),  # 5 tiles
+    (8, 2, 96, 257, 64, True),   # 6 tiles, in parts of 3
+    (6, 3, 32, 448, 64, True),   # 8 tiles in parts of 4
+    (4, 2, 16, 1000, 9, True), (5, 1, 80, 640, 129, True),
+    (32, 8, 96, 900, 640, False)])  # a workgroup per CU without a split
+def test_padded_heads_split_equals_unsplit(device, monkeypatch, dtype, hq, hkv, d, prefix, chunk,
+                                           splits):
+    test_chunk_split_equals_unsplit(device, monkeypatch, dtype, hq, hkv, d, prefix, chunk, splits)
+
+
+@pytest.mark.parametrize("dtype", list(ULP), ids=lambda t: str(t)[6:])
 def test_ragged_varlen_split_equals_unsplit(device, monkeypatch, dtype):
     """Items with one split, several, and none (query tiles past a chunk), and
     an out-of-range block inside one split."""
