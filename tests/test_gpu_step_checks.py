@@ -23,14 +23,14 @@ pytestmark = pytest.mark.gpu
 BS, BLOCKS = 16, 700
 
 
-def _metadata(rng, reqs, decode_only, long_one=0):
+def _metadata(rng, reqs, decode_only, long_one=0, longest=90):
     """A well-formed step: {name: CPU tensor} and the requests' phases."""
     free = list(range(BLOCKS))
     rng.shuffle(free)
     tables, ctx, counts, phases = [], [], [], []
     for i in range(reqs):
         decode = decode_only or rng.random() < 0.5
-        n = long_one if i == 0 and long_one else rng.randint(1, 90)
+        n = long_one if i == 0 and long_one else rng.randint(1, longest)
         count = 1 if decode and not (i == 0 and long_one) else rng.randint(1, n)
         if i == 0 and long_one:
             count, decode = n, False
@@ -51,19 +51,26 @@ def _metadata(rng, reqs, decode_only, long_one=0):
     return t, phases
 
 
-def _corrupt(rng, t):
+def _corrupt(rng, t, first=0):
+    """Change one entry, of request `first` or a later one."""
+    start = {"tables": first * t["tables"].shape[1], "ctx": first, "qsl": first}
     name = rng.choice(["tables", "ctx", "qsl", "pos", "slots", "repeat", "none"])
     if name == "none":
         return
     if name == "repeat":
         if len(t["slots"]) > 1:
             i, j = rng.sample(range(len(t["slots"])), 2)
+            i = max(i, _first_token(t, first))
             t["slots"][i] = t["slots"][j]
         return
     flat = t[name].view(-1)
-    i = rng.randrange(len(flat))
+    i = rng.randrange(start.get(name, _first_token(t, first)), len(flat))
     flat[i] = rng.choice([-1, 0, -7, int(flat[i]) + 1, int(flat[i]) - 1, 2 ** 40, BLOCKS,
                           BLOCKS * BS, int(flat[rng.randrange(len(flat))])])
+
+
+def _first_token(t, request):
+    return min(max(int(t["qsl"][request]), 0), len(t["slots"]) - 1)
 
 
 def _outcome(f):
@@ -85,12 +92,16 @@ def test_same_errors_as_the_torch_checks(device, reqs):
     rng = random.Random(reqs)
     cache = SimpleNamespace(block_size=BS, num_blocks=BLOCKS)
     seen = set()
-    for trial in range(150 if reqs < 100 else 12):
+    # 300 requests of one or two blocks are more than the launch's workgroups
+    # (256): rows from 256 on are second rows, and are corrupted on their own.
+    many = reqs > 256
+    for trial in range(60 if many else 150):
         decode_only = trial % 3 == 0
-        t, phases = _metadata(rng, min(reqs, 100) if not decode_only else reqs, decode_only) \
-            if reqs < 100 else _metadata(rng, 100, False, long_one=0)
+        t, phases = _metadata(rng, reqs, decode_only, longest=30 if many else 90)
+        assert len(t["ctx"]) == reqs and kchk._lib.load().mlr_check_step_groups(
+            reqs, len(t["slots"])) == max(min(reqs, 256), -(-len(t["slots"]) // 64))
         for _ in range(rng.randint(0, 2)):
-            _corrupt(rng, t)
+            _corrupt(rng, t, first=257 if many and trial % 2 else 0)
         seen.add(_same(device, t, lambda m: kpa._validate_tables(m["tables"], m["ctx"], BS,
                                                                  BLOCKS)))
         if decode_only and len(t["pos"]) == len(t["ctx"]):
