@@ -319,10 +319,13 @@ int mlr_paged_prefill_chunk(const void *q, int64_t q_stride_t,
  * The two prefill calls with a workspace. Where a call's work items (128-query
  * tiles x query heads) leave most of the GPU idle, a long key range is split
  * over several workgroups, whose FP32 partial results go through the
- * workspace, and a second kernel merges them; results differ from the calls
- * above by the order of FP32 sums. workspace: 16-byte aligned, any content,
- * at least mlr_paged_prefill_workspace_size bytes for the split to be taken
- * (0: no split for these sizes); with less the call runs as the one above.
+ * workspace, and a second kernel merges them. Results differ from the calls
+ * above by the order of FP32 sums and, at head sizes 64 and 128, whose
+ * probabilities are rounded to the 16-bit type, by that rounding against
+ * another reference point: at most 2 u (max |V| + |out|), u = 2^-8 (bf16) or
+ * 2^-11 (fp16). workspace: 16-byte aligned, any content, at least
+ * mlr_paged_prefill_workspace_size bytes for the split to be taken (0: no
+ * split for these sizes); with less the call runs as the one above.
  * max_context: max_blocks_per_seq * block_size, or context_len.
  */
 size_t mlr_paged_prefill_workspace_size(int64_t num_seqs, int64_t max_query_len,
@@ -555,8 +558,11 @@ int mlr_rms_norm_sums(const float *sums, int64_t splits, const void *residual,
                       void *stream);
 /*
  * mlr_rms_norm of x with `residual`, then the gated mlr_rows_linear of the
- * normalised rows, in one launch and bit for bit: out [rows, n] for weight
- * [2 n, k], and residual_out [rows, k] contiguous, a buffer of its own. bf16
+ * normalised rows, in one launch: out [rows, n] for weight [2 n, k], and
+ * residual_out [rows, k] contiguous, a buffer of its own. residual_out and the
+ * normalised rows are mlr_rms_norm's bit for bit; the products' FP32 sums may
+ * run in another order than mlr_rows_linear's (k is dealt to 4 waves, 8 past
+ * 16 rows, where that call takes 1 to 16 by k). bf16
  * and fp16, rows <= 32, k a multiple of 8 up to 1024 (1008 past 16 rows), 16-byte aligned
  * operands and row starts.
  *

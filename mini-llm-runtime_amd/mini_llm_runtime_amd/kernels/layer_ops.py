@@ -9,9 +9,9 @@ csrc/layer_ops.hip); the decoder layer's residual add before its
 post-attention norm rides on ``rms_norm(..., residual=...)``. bf16, fp16 and
 FP32 on a HIP device; there is no PyTorch fallback. ``apply_linear``,
 ``linear_silu_mul``, ``norm_silu_mul`` and ``rms_norm_sums`` stream the weights
-of a 16-bit linear layer once for a few rows (csrc/rows_linear.hip), with the
-norm before it or the activation after it in the same launch; more rows go to
-the library's GEMM.
+of a linear layer once for a few rows (up to 32 in 16 bits, 16 in FP32;
+csrc/rows_linear.hip), with the norm before it (16 bits) or the activation
+after it in the same launch; more rows go to the library's GEMM.
 """
 
 from __future__ import annotations

@@ -198,9 +198,10 @@ class Qwen2DecoderLayer(nn.Module):
     def _few_rows_tail(self, attended: torch.Tensor, residual: torch.Tensor, sums: bool = False):
         """The layer after its attention for a decode step's few rows: add, norm,
         gate/up and activation in one launch, then the down projection, whose
-        parts stay unsummed for the next norm with `sums`. (residual', delta')
-        with the bits of the separate modules, or None where those run (other
-        sizes and dtypes, hooks, gradients)."""
+        parts stay unsummed for the next norm with `sums`. (residual', delta'),
+        residual' with the bits of the separate modules and delta' up to the
+        order of FP32 sums, or None where those run (other sizes and dtypes,
+        hooks, gradients)."""
         norm, mlp = self.post_attention_layernorm, self.mlp
         # The stacked weight is asked for last: making it reads and copies gate
         # and up, which a call that is not taken (on the CPU, under a

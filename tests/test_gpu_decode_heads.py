@@ -7,7 +7,10 @@ FP32 sums run in another order, so a score may round to its neighbour: one
 unit (2^-8 bf16, 2^-11 fp16 relative) of a score of up to about 6 moves its
 probability by that much. Outputs are weighted means of |V| < 5, so 2e-2 holds
 them for 16-bit types, and 1e-5 for FP32, the bounds of the other head sizes.
-Against 64 bits the new kernel may not be further off than the generic one."""
+Against 64 bits the two kernels' errors are sums of independent roundings in
+different orders: over 60 draws of one query their ratio is 0.54 to 1.001 in the
+mean and scatters by up to 0.3 in FP32 at 20 keys, 0.01 in 16 bits. Over a case's
+rows together the padded kernel may be 10% further off in one draw."""
 
 from __future__ import annotations
 

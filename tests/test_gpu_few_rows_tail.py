@@ -1,7 +1,8 @@
 """The fused tail of a decoder layer over a decode step's few rows
 (mlr_norm_rows_linear, mlr_rms_norm_sums) against the separate calls: the
-residual and the norm bit for bit, the products too (the same sums in the
-same order)."""
+residual, the norms and the down projection bit for bit; the gated products
+too where both calls deal their k blocks to the same waves, elsewhere within
+FP32 sums in another order."""
 
 from __future__ import annotations
 
@@ -47,7 +48,7 @@ def test_norm_and_gated_product_match_the_two_calls(device, dtype, rows, k, n):
 
 
 @pytest.mark.parametrize("dtype", HALF + [torch.float32], ids=lambda t: str(t)[6:])
-@pytest.mark.parametrize("rows,n", [(1, 896), (16, 896), (3, 64), (9, 1024)])
+@pytest.mark.parametrize("rows,n", [(1, 896), (16, 896), (3, 64), (9, 1024), (2, 1000)])
 def test_norm_of_a_products_parts(device, dtype, rows, n):
     k = 8448 if dtype is not torch.float32 else 4224
     gen = torch.Generator().manual_seed(n)
