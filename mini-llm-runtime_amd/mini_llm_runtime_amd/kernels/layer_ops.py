@@ -138,6 +138,8 @@ def _rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
     dtype = x.dtype
     if not x.is_cuda or weight.dtype != dtype or dtype not in DTYPES or weight.ndim != 2:
         return None
+    if _transformed():  # before the sizes, which are tensors while tracing
+        return None
     n, k = weight.shape
     if x.ndim < 2 or x.shape[-1] != k or k == 0:
         return None
@@ -161,7 +163,7 @@ def _rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
     if stride < k or stride >= 1 << 22 or stride * size % 16 or xr.stride(1) != 1:
         return None
     xp, wp = xr.data_ptr(), weight.data_ptr()
-    if (xp | wp) & 15 or _transformed():
+    if (xp | wp) & 15:
         return None
     n_out = n // 2 if gated else n
     device = x.device
@@ -230,7 +232,8 @@ def norm_silu_mul(x: torch.Tensor, residual: torch.Tensor, norm_weight: torch.Te
     mlr_norm_rows_linear does not take (16-bit types, at most 32 rows of at most
     1024)."""
     dtype, k = x.dtype, x.shape[-1]
-    if (dtype not in (torch.bfloat16, torch.float16) or not x.is_cuda or k % 8 or k == 0
+    if (dtype not in (torch.bfloat16, torch.float16) or not x.is_cuda or _transformed()
+            or k % 8 or k == 0
             or gate_up_weight.ndim != 2 or gate_up_weight.shape[1] != k
             or gate_up_weight.shape[0] % 2):
         return None
@@ -243,7 +246,7 @@ def norm_silu_mul(x: torch.Tensor, residual: torch.Tensor, norm_weight: torch.Te
         if (t.dtype != dtype or t.device != x.device or t.stride(-1) != 1
                 or type(t) not in (torch.Tensor, nn.Parameter) or t.data_ptr() & 15):
             return None
-    if not gate_up_weight.is_contiguous() or _transformed():
+    if not gate_up_weight.is_contiguous():
         return None
     if torch.is_grad_enabled() and (x.requires_grad or residual.requires_grad
                                     or norm_weight.requires_grad):

@@ -207,8 +207,8 @@ class Qwen2DecoderLayer(nn.Module):
         # and up, which a call that is not taken (on the CPU, under a
         # transform, with a replaced projection) must not do.
         if (not attended.is_cuda or attended.dtype not in (torch.bfloat16, torch.float16)
-                or attended.shape[-1] > 1024 or attended.numel() > 32 * attended.shape[-1]
                 or kops._transformed()
+                or attended.shape[-1] > 1024 or attended.numel() > 32 * attended.shape[-1]
                 or not kops.plain(norm, Qwen2RMSNorm) or not kops.plain(mlp, Qwen2MLP)
                 or "forward_with_residual" in norm.__dict__
                 or type(mlp.gate_proj) is not nn.Linear or type(mlp.up_proj) is not nn.Linear

@@ -183,3 +183,17 @@ def test_replaced_parts_run_on_the_gpu(device, what):
         assert isinstance(layer._few_rows_tail(x, x)[1], torch.Tensor)
         _replace(model, what)
         assert torch.equal(model(ids), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_tracing_on_the_gpu_runs_the_torch_operations(device, dtype):
+    """While tracing, sizes are tensors; a projection is recorded as what it is."""
+    torch.manual_seed(0)
+    linear = nn.Linear(64, 96, bias=False).to(device, dtype).requires_grad_(False)
+    x = torch.randn(3, 64, device=device, dtype=dtype)
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda t: kops.apply_linear(linear, t), (x,), check_trace=False)
+        assert torch.equal(traced(x + 1), linear(x + 1))
+        model = TinyQwen2ForCausalLM(TinyQwen2Config()).to(device, dtype).eval()
+        torch.jit.trace(model, (IDS.to(device),), check_trace=False)
