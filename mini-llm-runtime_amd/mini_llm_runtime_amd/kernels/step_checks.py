@@ -62,7 +62,7 @@ def step_flags(block_size: int, num_blocks: int, *, tables: torch.Tensor | None 
     # the wait that the checks cost anyway: no copy behind the kernel. The
     # buffer is this call's own until the wait has ended.
     out = torch.empty(groups + (3 * reqs + 1 if detail else 0), dtype=torch.long,
-                      pin_memory=True)
+                      device="cpu", pin_memory=True)  # whatever the default device is
 
     def ptr(t):
         return None if t is None else t.data_ptr()

@@ -211,7 +211,7 @@ def _upload(values, device: torch.device, dtype: torch.dtype = torch.long) -> to
     (a copy from pageable memory would)."""
     if device.type != "cuda":
         return torch.tensor(values, dtype=dtype, device=device)
-    staged = torch.tensor(values, dtype=dtype, pin_memory=True)
+    staged = torch.tensor(values, dtype=dtype, device="cpu", pin_memory=True)
     return staged.to(device, non_blocking=True)
 
 

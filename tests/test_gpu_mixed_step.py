@@ -8,9 +8,12 @@ relative, 16-bit logits within the rounding that a layer's output carries on
 
 from __future__ import annotations
 
+import contextlib
+
 import pytest
 import torch
 
+from mini_llm_runtime_amd.kernels import paged_attention as kpa
 from mini_llm_runtime_amd.model.qwen2 import TinyQwen2Config, TinyQwen2ForCausalLM
 from mini_llm_runtime_amd.runtime import model_runner
 from mini_llm_runtime_amd.runtime.paged_kv_cache import PagedKVCache
@@ -97,3 +100,25 @@ def test_steps_that_keep_the_two_forwards(device):
                 layer.self_attn, *a, **k))
         model_runner.execute_model_batch(model, batch, caches[1])
         assert seen[2:] == [1]
+
+
+@pytest.mark.parametrize("mixed", [True, False])
+def test_under_a_default_device(device, monkeypatch, mixed):
+    """A step, a slot write and a checked decode inside a torch.device context,
+    where tensors made without a device land on the GPU."""
+    model, batch, caches = _setup(SMALL, torch.float32, device, [(P, 5, 5), (D, 9, 1)], 16)
+    if not mixed:
+        monkeypatch.setattr(model_runner, "_takes_mixed_steps", lambda *a: False)
+    rows = torch.ones(2, 2, 16, device=device)
+    slots = torch.tensor([3, 40], device=device)
+    q = torch.ones(2, 4, 16, device=device)
+    args = (batch.block_tables, batch.context_lens, 16)
+    results = []
+    for cache, context in zip(caches, (torch.device("cuda"), contextlib.nullcontext())):
+        with torch.no_grad(), context:
+            logits = model_runner.execute_model_batch(model, batch, cache)
+            cache.write_slots(slot_mapping=slots, k=rows, v=rows, layer_idx=0)
+            k, v = cache.get_layer_cache(0)
+            results.append((logits, k, kpa.paged_attention_decode_batch_parallel(q, k, v, *args)))
+    for got, want in zip(*results):
+        assert (got - want).norm() <= 1e-4 * want.norm()
