@@ -269,7 +269,8 @@ class Qwen2DecoderLayer(nn.Module):
 
 # Methods that a caller may have replaced on an instance.
 _STEP_METHODS = {"forward", "_run", "_block_parts", "forward_prefill_packed_with_cache",
-                 "forward_decode_batch_with_cache", "forward_mixed_with_cache"}
+                 "forward_decode_batch_with_cache", "forward_mixed_with_cache",
+                 "forward_with_residual"}
 
 
 def _raise_packed_errors(flags) -> None:
@@ -516,9 +517,12 @@ class TinyQwen2Model(nn.Module):
         if (type(self) is not TinyQwen2Model or _STEP_METHODS & self.__dict__.keys()
                 or not plain(self.embed_tokens, nn.Embedding)
                 or self.embed_tokens.weight.dtype not in kops.DTYPES
+                or not plain(self.norm, Qwen2RMSNorm)
                 or nn.modules.module._has_any_global_hook() or kops._transformed()):
             return False
         return all(plain(layer, Qwen2DecoderLayer) and plain(layer.self_attn, Qwen2Attention)
+                   and plain(layer.input_layernorm, Qwen2RMSNorm)
+                   and plain(layer.post_attention_layernorm, Qwen2RMSNorm)
                    and plain(layer.mlp, Qwen2MLP) and plain(layer.mlp.down_proj, nn.Linear)
                    and plain(layer.self_attn.o_proj, nn.Linear) for layer in self.layers)
 

@@ -122,3 +122,20 @@ def test_under_a_default_device(device, monkeypatch, mixed):
             results.append((logits, k, kpa.paged_attention_decode_batch_parallel(q, k, v, *args)))
     for got, want in zip(*results):
         assert (got - want).norm() <= 1e-4 * want.norm()
+
+
+def test_hooks_on_norms_see_the_two_forwards(device):
+    """The first layer's input norm is called as a module, once per forward."""
+    model, batch, caches = _setup(SMALL, torch.float32, device, [(P, 5, 5), (D, 9, 1)], 16)
+    seen = []
+    norm = model.model.layers[0].input_layernorm
+    handle = norm.register_forward_hook(lambda m, i, o: seen.append(o.numel() // 64))
+    with torch.no_grad():
+        model_runner.execute_model_batch(model, batch, caches[0])
+        handle.remove()
+        assert seen == [5, 1]
+        last = model.model.norm
+        add = last.forward_with_residual
+        last.forward_with_residual = lambda x, r: seen.append(r.numel() // 64) or add(x, r)
+        model_runner.execute_model_batch(model, batch, caches[1])
+    assert seen[2:] == [5, 1]
