@@ -138,7 +138,7 @@ def _rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
     dtype = x.dtype
     if not x.is_cuda or weight.dtype != dtype or dtype not in DTYPES or weight.ndim != 2:
         return None
-    if _transformed():  # before the sizes, which are tensors while tracing
+    if torch._C._get_tracing_state() is not None:  # sizes would be tensors
         return None
     n, k = weight.shape
     if x.ndim < 2 or x.shape[-1] != k or k == 0:
@@ -163,7 +163,7 @@ def _rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
     if stride < k or stride >= 1 << 22 or stride * size % 16 or xr.stride(1) != 1:
         return None
     xp, wp = xr.data_ptr(), weight.data_ptr()
-    if (xp | wp) & 15:
+    if (xp | wp) & 15 or _transformed():
         return None
     n_out = n // 2 if gated else n
     device = x.device

@@ -206,9 +206,9 @@ class Qwen2DecoderLayer(nn.Module):
         # The stacked weight is asked for last: making it reads and copies gate
         # and up, which a call that is not taken (on the CPU, under a
         # transform, with a replaced projection) must not do.
-        if (not attended.is_cuda or attended.dtype not in (torch.bfloat16, torch.float16)
+        if (attended.shape[-1] > 1024 or attended.numel() > 32 * attended.shape[-1]
+                or not attended.is_cuda or attended.dtype not in (torch.bfloat16, torch.float16)
                 or kops._transformed()
-                or attended.shape[-1] > 1024 or attended.numel() > 32 * attended.shape[-1]
                 or not kops.plain(norm, Qwen2RMSNorm) or not kops.plain(mlp, Qwen2MLP)
                 or "forward_with_residual" in norm.__dict__
                 or type(mlp.gate_proj) is not nn.Linear or type(mlp.up_proj) is not nn.Linear
@@ -328,10 +328,13 @@ class TinyQwen2Model(nn.Module):
         separate add (Qwen2DecoderLayer._block_parts)."""
         residual, delta = self.embed_tokens(input_ids), None
         layers = list(self.layers)
+        few = residual.numel() <= 32 * residual.shape[-1]  # rows a product may be left in parts for
         for layer_idx, (layer, after) in enumerate(zip(layers, layers[1:] + [None])):
-            args = (residual, delta, attend_of(layer, layer_idx))
-            residual, delta = (layer._block_parts(*args, sums=True)
-                               if self._takes_sums(layer, after) else layer._block_parts(*args))
+            attend = attend_of(layer, layer_idx)
+            if few and self._takes_sums(layer, after):
+                residual, delta = layer._block_parts(residual, delta, attend, sums=True)
+            else:
+                residual, delta = layer._block_parts(residual, delta, attend)
         if delta is None:
             return self.norm(residual)
         return self.norm.forward_with_residual(delta, residual)[0]
@@ -514,17 +517,32 @@ class TinyQwen2Model(nn.Module):
                     and not module._forward_pre_hooks and not module._backward_hooks
                     and not module._backward_pre_hooks and not _STEP_METHODS & module.__dict__.keys())
 
+        def own_norm(norm):
+            return type(norm) is Qwen2RMSNorm and "forward_with_residual" not in norm.__dict__
+
         if (type(self) is not TinyQwen2Model or _STEP_METHODS & self.__dict__.keys()
                 or not plain(self.embed_tokens, nn.Embedding)
                 or self.embed_tokens.weight.dtype not in kops.DTYPES
-                or not plain(self.norm, Qwen2RMSNorm)
+                or not own_norm(self.norm)
+                # Of the norms only the first is called as a module, with hooks.
+                or not all(plain(layer.input_layernorm, Qwen2RMSNorm)
+                           for layer in self.layers[:1])
                 or nn.modules.module._has_any_global_hook() or kops._transformed()):
             return False
-        return all(plain(layer, Qwen2DecoderLayer) and plain(layer.self_attn, Qwen2Attention)
-                   and plain(layer.input_layernorm, Qwen2RMSNorm)
-                   and plain(layer.post_attention_layernorm, Qwen2RMSNorm)
-                   and plain(layer.mlp, Qwen2MLP) and plain(layer.mlp.down_proj, nn.Linear)
-                   and plain(layer.self_attn.o_proj, nn.Linear) for layer in self.layers)
+        for layer in self.layers:
+            if not plain(layer, Qwen2DecoderLayer):
+                return False
+            # Straight from the modules' table: an attribute of a module takes
+            # 0.6 us, six of 24 layers 90 us of a step.
+            parts = layer._modules
+            attn, mlp = parts.get("self_attn"), parts.get("mlp")
+            if not (plain(attn, Qwen2Attention) and plain(mlp, Qwen2MLP)
+                    and own_norm(parts.get("input_layernorm"))
+                    and own_norm(parts.get("post_attention_layernorm"))
+                    and plain(attn._modules.get("o_proj"), nn.Linear)
+                    and plain(mlp._modules.get("down_proj"), nn.Linear)):
+                return False
+        return True
 
     def forward_mixed_with_cache(self, input_ids: torch.Tensor, position_ids: torch.Tensor,
                                  kv_cache: PagedKVCache, num_prefill: int, prefill: tuple,
