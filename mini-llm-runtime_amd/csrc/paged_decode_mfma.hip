@@ -60,6 +60,10 @@
 // accumulator has the bf16 tiles' layout, so the softmax, the merges, the
 // work items and the fused KV write are shared. Scores, probabilities and
 // P@V stay FP32, as in the reference's FP32 path.
+//
+// Head sizes other than 64 and 128 (kPad) keep what the generic kernel does for
+// them: 16-bit scores rounded as above, but FP32 probabilities times V in FP32,
+// and no weight for a score of -inf.
 #include "paged_decode.h"
 
 namespace mlr {

@@ -70,8 +70,11 @@
 // and three shuffles per key.
 // fp16, 3 sequences of 60..400 queries on prefixes up to 800, 8/2 heads of 96:
 // 1,618 us per call there, 82 us here, 57 with the key ranges split (30 with each
-// probability as two 16-bit parts, which is fewer bits); error against 64 bits 6.7e-4 there, 2.1e-4 here
-// (the generic kernel rounds each score to the 16-bit type).
+// probability as two 16-bit parts, which is fewer bits); error against 64 bits
+// 6.7e-4 there, 2.1e-4 here (the generic kernel rounds each score to the 16-bit
+// type). As there, a V row that is not finite reaches only the queries that see
+// its key; at 64 and 128 it also makes NaN of earlier queries whose wave reads its
+// tile.
 #include "paged_prefill.h"
 
 #include <algorithm>
