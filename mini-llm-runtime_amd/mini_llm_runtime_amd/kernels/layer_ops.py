@@ -68,8 +68,8 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     device = x.device
     with _lib.on(device):
         status = _lib.load().mlr_rms_norm(
-            xr.data_ptr(), xs, rp, hidden if rs is None else rs, ro, hidden, weight.data_ptr(), out.data_ptr(),
-            hidden, rows, hidden, float(eps), _lib.DTYPE_CODES[x.dtype],
+            xr.data_ptr(), xs, rp, hidden if rs is None else rs, ro, hidden, weight.data_ptr(),
+            out.data_ptr(), hidden, rows, hidden, float(eps), _lib.DTYPE_CODES[x.dtype],
             _lib.stream_handle(device))
     _lib.check(status, "mlr_rms_norm")
     return out if residual is None else (out, res_out)
@@ -261,8 +261,8 @@ def norm_silu_mul(x: torch.Tensor, residual: torch.Tensor, norm_weight: torch.Te
     with _lib.on(device):
         status = _lib.load().mlr_norm_rows_linear(
             xr.data_ptr(), xs, rr.data_ptr(), rs, res_out.data_ptr(), norm_weight.data_ptr(),
-            float(eps), gate_up_weight.data_ptr(), out.data_ptr(), n, rows, n, k, _lib.DTYPE_CODES[dtype],
-            _lib.stream_handle(device))
+            float(eps), gate_up_weight.data_ptr(), out.data_ptr(), n, rows, n, k,
+            _lib.DTYPE_CODES[dtype], _lib.stream_handle(device))
     _lib.check(status, "mlr_norm_rows_linear")
     return out, res_out
 
